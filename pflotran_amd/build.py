@@ -5,28 +5,41 @@
 import os
 import subprocess
 import sys
+import tempfile
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 LIB = os.path.join(HERE, "libpfx_chem.so")
-SOURCES = ["pfx_react.hip", "pfx_api.hip", "pfx_mlp.hip", "pfx_gi.hip", "pfx_krylov.hip"]
+# (source, extra defines): the reaction kernels' instantiations are split into
+# parts of their own, so that the objects compile in parallel
+UNITS = [("pfx_react.hip", (f"PFX_REACT_PART={p}",)) for p in (2, 3, 1, 0)] + [
+    (s, ()) for s in ("pfx_api.hip", "pfx_mlp.hip", "pfx_gi.hip", "pfx_krylov.hip")]
 ARCH = os.environ.get("PFX_OFFLOAD_ARCH", "gfx950")
 
 
-def hipcc_cmd(out=LIB, defines=()):
+def hipcc_cmd(out, source, defines=()):
     hipcc = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
-    return [hipcc, f"--offload-arch={ARCH}", "-O3", "-std=c++17", "-fPIC", "-shared"] + [f"-D{d}" for d in defines] + [
+    return [hipcc, f"--offload-arch={ARCH}", "-O3", "-std=c++17", "-fPIC"] + [f"-D{d}" for d in defines] + [
             # no packed-FP32 instructions in device code
             "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
             "-Wall", "-Wno-unused-variable", "-Wno-unused-but-set-variable",
-            "-o", out] + [os.path.join(CSRC, s) for s in SOURCES]
+            "-c", os.path.join(CSRC, source), "-o", out]
 
 
 def build(verbose=True):
-    cmd = hipcc_cmd(LIB + ".tmp")
-    if verbose:
-        print(" ".join(cmd), flush=True)
-    subprocess.run(cmd, check=True)
+    with tempfile.TemporaryDirectory(prefix="pfx_build_") as tmp:
+        objs, running = [], []
+        for k, (source, defines) in enumerate(UNITS):
+            objs.append(os.path.join(tmp, f"{k}.o"))
+            cmd = hipcc_cmd(objs[-1], source, defines)
+            if verbose:
+                print(" ".join(cmd), flush=True)
+            running.append((cmd, subprocess.Popen(cmd)))
+        failed = [cmd for cmd, p in running if p.wait() != 0]
+        if failed:
+            raise subprocess.CalledProcessError(1, failed[0])
+        link = [running[0][0][0], f"--offload-arch={ARCH}", "-shared", "-fPIC", "-o", LIB + ".tmp"] + objs
+        subprocess.run(link, check=True)
     os.replace(LIB + ".tmp", LIB)
     return LIB
 

@@ -116,27 +116,6 @@ __device__ __forceinline__ double gmax(double v, int lane) { return greduce<G>(v
 template <int G>
 __device__ __forceinline__ double gmin(double v, int lane) { return greduce<G>(v, lane, OpMin()); }
 
-// argmax with ties resolved to the larger row index
-__device__ __forceinline__ void amax_step(double &v, int &idx, double w, int j) {
-  const bool take = (w > v) | ((w == v) & (j > idx));  // no short circuit: selects
-  v = take ? w : v;
-  idx = take ? j : idx;
-}
-template <int G>
-__device__ __forceinline__ void gargmax(double &v, int &idx, int lane) {
-  if constexpr (G == 8) {
-    amax_step(v, idx, dpp_d<DPP_HALF_MIRROR>(v), dpp_i<DPP_HALF_MIRROR>(idx));
-    amax_step(v, idx, dpp_d<DPP_XOR2>(v), dpp_i<DPP_XOR2>(idx));
-    amax_step(v, idx, dpp_d<DPP_XOR1>(v), dpp_i<DPP_XOR1>(idx));
-  } else {
-    amax_step(v, idx, dpp_d<DPP_ROR8>(v), dpp_i<DPP_ROR8>(idx));
-    amax_step(v, idx, dpp_d<DPP_ROR4>(v), dpp_i<DPP_ROR4>(idx));
-    amax_step(v, idx, dpp_d<DPP_ROR2>(v), dpp_i<DPP_ROR2>(idx));
-    amax_step(v, idx, dpp_d<DPP_ROR1>(v), dpp_i<DPP_ROR1>(idx));
-    if constexpr (G == 32) amax_step(v, idx, bperm_d(v, lane ^ 16), bperm_i(idx, lane ^ 16));
-  }
-}
-
 struct OpMaxNum {  // a NaN candidate never wins the pivot search
   __device__ __forceinline__ double operator()(double a, double b) const { return fmax(a, b); }
 };
@@ -182,6 +161,206 @@ __device__ __forceinline__ double gbcast(double v, int gbase) {
   } else {
     return bperm_d(v, gbase + J);
   }
+}
+
+// acc += f * (lane J's src, of each 16-lane DPP row), one instruction per
+// register: v_fmac_f64_dpp takes its first factor through a row broadcast, so
+// an elimination step needs no separate moves (a 64-bit DPP move costs as
+// much as the multiply-add it feeds: 3.2 against 2.9 ns a SIMD measured).  RM
+// and BM enable 16-lane rows and 4-lane banks; the other lanes keep acc.  A
+// DPP source may not be read within two wait states of its write, which the
+// compiler cannot see inside the statement: every statement waits them itself.
+template <int J, int RM, int BM>
+__device__ __forceinline__ void fmac_bcast(double &acc, double src, double f) {
+  asm("s_nop 1\n\t"
+      "v_fmac_f64_dpp %0, %1, %2 row_newbcast:%3 row_mask:%4 bank_mask:%5"
+      : "+v"(acc)
+      : "v"(src), "v"(f), "n"(J), "n"(RM), "n"(BM));
+}
+template <int J, int RM, int BM>
+__device__ __forceinline__ void fmac_bcast_self(double f, double &a) {
+  asm("s_nop 1\n\t"
+      "v_fmac_f64_dpp %0, %0, %1 row_newbcast:%2 row_mask:%3 bank_mask:%4"
+      : "+v"(a)
+      : "v"(f), "n"(J), "n"(RM), "n"(BM));
+}
+template <int J, int RM, int BM>
+__device__ __forceinline__ void fmac_bcast_self(double f, double &a, double &b, double &c, double &d) {
+  asm("s_nop 1\n\t"
+      "v_fmac_f64_dpp %0, %0, %4 row_newbcast:%5 row_mask:%6 bank_mask:%7\n\t"
+      "v_fmac_f64_dpp %1, %1, %4 row_newbcast:%5 row_mask:%6 bank_mask:%7\n\t"
+      "v_fmac_f64_dpp %2, %2, %4 row_newbcast:%5 row_mask:%6 bank_mask:%7\n\t"
+      "v_fmac_f64_dpp %3, %3, %4 row_newbcast:%5 row_mask:%6 bank_mask:%7"
+      : "+v"(a), "+v"(b), "+v"(c), "+v"(d)
+      : "v"(f), "n"(J), "n"(RM), "n"(BM));
+}
+template <int J, int RM, int BM>
+__device__ __forceinline__ void fmac_bcast4(double f, double &a, double pa, double &b, double pb, double &c, double pc,
+                                            double &d, double pd) {
+  asm("s_nop 1\n\t"
+      "v_fmac_f64_dpp %0, %4, %8 row_newbcast:%9 row_mask:%10 bank_mask:%11\n\t"
+      "v_fmac_f64_dpp %1, %5, %8 row_newbcast:%9 row_mask:%10 bank_mask:%11\n\t"
+      "v_fmac_f64_dpp %2, %6, %8 row_newbcast:%9 row_mask:%10 bank_mask:%11\n\t"
+      "v_fmac_f64_dpp %3, %7, %8 row_newbcast:%9 row_mask:%10 bank_mask:%11"
+      : "+v"(a), "+v"(b), "+v"(c), "+v"(d)
+      : "v"(pa), "v"(pb), "v"(pc), "v"(pd), "v"(f), "n"(J), "n"(RM), "n"(BM));
+}
+
+// v_k += f * (v_k of lane J), k = B .. E-1
+template <int J, int RM, int BM, int B, int E>
+__device__ __forceinline__ void fmac_cols_self(double f, double *v) {
+  if constexpr (B + 4 <= E) {
+    fmac_bcast_self<J, RM, BM>(f, v[B], v[B + 1], v[B + 2], v[B + 3]);
+    fmac_cols_self<J, RM, BM, B + 4, E>(f, v);
+  } else if constexpr (B < E) {
+    fmac_bcast_self<J, RM, BM>(f, v[B]);
+    fmac_cols_self<J, RM, BM, B + 1, E>(f, v);
+  }
+}
+
+// 1/d to one rounding of the exact quotient or so, without the scaling of
+// the full division (a pivot that needs it fails the step's finiteness test)
+__device__ __forceinline__ double fast_rcp(double d) {
+  double y = __builtin_amdgcn_rcp(d);
+  y = fma(fma(-d, y, 1.0), y, y);
+  return fma(fma(-d, y, 1.0), y, y);
+}
+
+// the value of the even (odd) 16-lane row of each 32-lane pair, in both rows
+template <bool ODD>
+__device__ __forceinline__ double pair_row(double v) {
+  const unsigned lo = __double2loint(v), hi = __double2hiint(v);
+  const auto l = __builtin_amdgcn_permlane16_swap(lo, lo, false, false);
+  const auto h = __builtin_amdgcn_permlane16_swap(hi, hi, false, false);
+  return __hiloint2double(h[ODD ? 1 : 0], l[ODD ? 1 : 0]);
+}
+
+// Unpivoted elimination and back substitution of a group's system, row r in
+// lane r with its right-hand side b; returns lane r's unknown.  A breakdown
+// (zero pivot, overflow) leaves a non-finite value in some lane.
+//
+// Instruction-issue bound: G^2/2 multiply-adds a step, each one instruction
+// (fmac_bcast).  A 16-lane group is one DPP row.  Two 8-lane groups share a
+// row and take their broadcasts under complementary bank masks.  A 32-lane
+// group is two DPP rows, A (rows 0..15 of the system) and B: A is factored
+// first; its 16 finished pivot rows are copied across once, a column at a
+// time (pair_row: 6 instructions a column instead of a cross-row permute for
+// every multiplier pair), B is eliminated with the copies and then factored by
+// itself.  Measured against DPP moves and (32 lanes) LDS permutes feeding plain
+// multiply-adds, MI355X: 400k/200k/120k/80k cells of N = 8/12/20/30 46.8 ->
+// 31.4 ms, 1M cells of N = 15 25.5 -> 24.8 ms.
+template <int G>
+__device__ __forceinline__ double lu_solve(double (&row)[G], double b, int r) {
+  double x = 0.0, inv_diag = 0.0;
+  if constexpr (G == 16) {
+    static_for<0, 16>([&](auto jc) {
+      constexpr int j = decltype(jc)::value;
+      const double ip = fast_rcp(dpp_d<0x150 + j>(row[j]));
+      const double nf = r > j ? -row[j] * ip : 0.0;
+      inv_diag = r == j ? ip : inv_diag;
+      fmac_cols_self<j, 15, 15, j + 1, 16>(nf, row);
+      fmac_bcast_self<j, 15, 15>(nf, b);
+    });
+    static_for<0, 16>([&](auto jc) {
+      constexpr int j = 15 - decltype(jc)::value;
+      const double t = b * inv_diag;
+      x = r == j ? t : x;
+      if constexpr (j > 0) fmac_bcast<j, 15, 15>(b, t, -row[j]);
+    });
+  } else if constexpr (G == 8) {
+    static_for<0, 8>([&](auto jc) {
+      constexpr int j = decltype(jc)::value;
+      const double ip = fast_rcp(gbcast<8, j>(row[j], (int)(threadIdx.x & 8)));
+      const double nf = r > j ? -row[j] * ip : 0.0;
+      inv_diag = r == j ? ip : inv_diag;
+      fmac_cols_self<j, 15, 3, j + 1, 8>(nf, row);
+      fmac_cols_self<8 + j, 15, 12, j + 1, 8>(nf, row);
+      fmac_bcast_self<j, 15, 3>(nf, b);
+      fmac_bcast_self<8 + j, 15, 12>(nf, b);
+    });
+    static_for<0, 8>([&](auto jc) {
+      constexpr int j = 7 - decltype(jc)::value;
+      const double t = b * inv_diag;
+      x = r == j ? t : x;
+      if constexpr (j > 0) {
+        fmac_bcast<j, 15, 3>(b, t, -row[j]);
+        fmac_bcast<8 + j, 15, 12>(b, t, -row[j]);
+      }
+    });
+  } else {
+    static_assert(G == 32, "group size");
+    const int l = r & 15;
+    const bool hi = r >= 16;
+    // rows 0..15 (DPP rows A) by themselves
+    static_for<0, 16>([&](auto jc) {
+      constexpr int j = decltype(jc)::value;
+      const double ip = fast_rcp(dpp_d<0x150 + j>(row[j]));
+      const double nf = l > j ? -row[j] * ip : 0.0;
+      inv_diag = l == j ? ip : inv_diag;
+      fmac_cols_self<j, 5, 15, j + 1, 32>(nf, row);
+      fmac_bcast_self<j, 5, 15>(nf, b);
+    });
+    // rows 16..31 (B): the multipliers from the copied columns 0..15, kept
+    // in place of the eliminated entries
+    const double ia = pair_row<false>(inv_diag);
+    double cp[16];
+    static_for<1, 16>([&](auto kc) {
+      constexpr int k = decltype(kc)::value;
+      cp[k] = pair_row<false>(row[k]);
+    });
+    double nf[16];
+    static_for<0, 16>([&](auto jc) {
+      constexpr int j = decltype(jc)::value;
+      nf[j] = -row[j] * dpp_d<0x150 + j>(ia);
+      static_for<j + 1, 16>([&](auto kc) {
+        constexpr int k = decltype(kc)::value;
+        fmac_bcast<j, 10, 15>(row[k], cp[k], nf[j]);
+      });
+    });
+    static_for<4, 8>([&](auto qc) {
+      constexpr int q = 4 * decltype(qc)::value;
+      const double p0 = pair_row<false>(row[q]), p1 = pair_row<false>(row[q + 1]),
+                   p2 = pair_row<false>(row[q + 2]), p3 = pair_row<false>(row[q + 3]);
+      static_for<0, 16>([&](auto jc) {
+        constexpr int j = decltype(jc)::value;
+        fmac_bcast4<j, 10, 15>(nf[j], row[q], p0, row[q + 1], p1, row[q + 2], p2, row[q + 3], p3);
+      });
+    });
+    {
+      const double pb = pair_row<false>(b);
+      static_for<0, 16>([&](auto jc) {
+        constexpr int j = decltype(jc)::value;
+        fmac_bcast<j, 10, 15>(b, pb, nf[j]);
+      });
+    }
+    static_for<0, 16>([&](auto jc) {
+      constexpr int j = decltype(jc)::value;
+      const double ip = fast_rcp(dpp_d<0x150 + j>(row[16 + j]));
+      const double nfj = l > j ? -row[16 + j] * ip : 0.0;
+      inv_diag = (hi && l == j) ? ip : inv_diag;
+      fmac_cols_self<j, 10, 15, 17 + j, 32>(nfj, row);
+      fmac_bcast_self<j, 10, 15>(nfj, b);
+    });
+    // back substitution: B, its unknowns copied to A, then A
+    static_for<0, 16>([&](auto jc) {
+      constexpr int j = 15 - decltype(jc)::value;
+      const double t = b * inv_diag;
+      x = l == j ? t : x;
+      if constexpr (j > 0) fmac_bcast<j, 10, 15>(b, t, -row[16 + j]);
+    });
+    const double xb = pair_row<true>(x);
+    static_for<0, 16>([&](auto jc) {
+      constexpr int j = decltype(jc)::value;
+      fmac_bcast<j, 5, 15>(b, xb, -row[16 + j]);
+    });
+    static_for<0, 16>([&](auto jc) {
+      constexpr int j = 15 - decltype(jc)::value;
+      const double t = b * inv_diag;
+      x = (!hi && l == j) ? t : x;
+      if constexpr (j > 0) fmac_bcast<j, 5, 15>(b, t, -row[j]);
+    });
+  }
+  return x;
 }
 
 __device__ __forceinline__ void wave_sync() {
@@ -1323,7 +1502,7 @@ __device__ __forceinline__ void react_body(uint64_t praw) {
         if (live && !(mx > 0.0)) status = PFX_CELL_SINGULAR;
       }
       // Elimination with the pivot row of step j in lane j, broadcast across
-      // the group.  The reaction step's Jacobian in ln m is the
+      // the group (lu_solve; the pivoting form here).  The reaction step's Jacobian in ln m is the
       // accumulation's diagonal plus positive semi-definite complexation,
       // exchange and mineral terms (nu^T diag(C) nu, diag(X) - X X^T,
       // nu nu^T dI/dlnQ) with rows scaled by positive factors, so it needs
@@ -1345,12 +1524,15 @@ __device__ __forceinline__ void react_body(uint64_t praw) {
       constexpr bool kCanPivot = MODE != PFX_MODE_REACT || LUP != PFX_LU_DEFER;
       const bool pivoting = MODE != PFX_MODE_REACT || LUP == PFX_LU_PIVOT ||
                             (LUP == PFX_LU_ONDEMAND && __ballot(active && !finish && lu_pivot) != 0ull);
-      {
-        bool lbad = false;
-        double inv_diag = 0.0;  // 1 / U_rr, kept by lane r for the back substitution
+      bool lbad = false;
+      if (!kCanPivot || !pivoting) {
+        const double x = lu_solve<G>(row, b, r);
+        upd = live ? x : 0.0;
+        lbad = !(fabs(upd) <= 1.0e300);
+      } else if constexpr (kCanPivot) {
         static_for<0, G>([&](auto jc) {
           constexpr int j = decltype(jc)::value;
-          if (kCanPivot && pivoting && j < N) {
+          if (j < N) {
             const double cand = (r >= j && live) ? vv * fabs(row[j]) : -1.0;
             const int pr = gargmax_row<G>(cand, lane, gbase);
             const int src = gbase + ((r == j) ? pr : ((r == pr) ? j : r));
@@ -1363,14 +1545,9 @@ __device__ __forceinline__ void react_body(uint64_t praw) {
             vv = bperm_d(vv, src);
           }
           double piv = gbcast<G, j>(row[j], gbase);
-          if (pivoting) piv = piv == 0.0 ? 1.0e-20 : piv;  // ludcmp's TINY (utility.F90:462)
-          const double ip = 1.0 / piv;
+          piv = piv == 0.0 ? 1.0e-20 : piv;  // ludcmp's TINY (utility.F90:462)
           const bool elim = r > j;
-          // pivoting divides, as the reference's elimination does; the
-          // unpivoted path multiplies by the reciprocal
-          const double f = elim ? (pivoting ? row[j] / piv : row[j] * ip) : 0.0;
-          lbad = lbad || (r == j && !(fabs(piv) > 0.0)) || !(fabs(f) <= 1.0e300);
-          inv_diag = (r == j) ? ip : inv_diag;
+          const double f = elim ? row[j] / piv : 0.0;
           row[j] = (r == j) ? piv : (elim ? f : row[j]);
 #pragma unroll
           for (int k = j + 1; k < G; k++) {
@@ -1383,21 +1560,21 @@ __device__ __forceinline__ void react_body(uint64_t praw) {
         });
         static_for<0, G>([&](auto jc) {
           constexpr int j = G - 1 - decltype(jc)::value;
-          const double xj = gbcast<G, j>(pivoting ? b / row[j] : b * inv_diag, gbase);
+          const double xj = gbcast<G, j>(b / row[j], gbase);
           upd = (r == j && live) ? xj : upd;
           b -= row[j] * xj;
         });
-        if (!pivoting) {
-          redo = gmax<G>(lbad ? 1.0 : 0.0, lane) > 0.0;
-          if (LUP == PFX_LU_ONDEMAND) lu_pivot = lu_pivot || redo;
-          if (kCanDefer && redo) {
-            // a warm attempt is given up as one that fails (the plain
-            // attempt follows in this launch); otherwise the cell is left as
-            // it came in, for the pivoting launch to redo
-            finish = true;
-            if (P.guess_mode == PFX_GUESS_ARRAY_FALLBACK && !fell_back) status = PFX_CELL_SINGULAR;
-            else deferred = true;
-          }
+      }
+      if (!pivoting) {
+        redo = gmax<G>(lbad ? 1.0 : 0.0, lane) > 0.0;
+        if (LUP == PFX_LU_ONDEMAND) lu_pivot = lu_pivot || redo;
+        if (kCanDefer && redo) {
+          // a warm attempt is given up as one that fails (the plain
+          // attempt follows in this launch); otherwise the cell is left as
+          // it came in, for the pivoting launch to redo
+          finish = true;
+          if (P.guess_mode == PFX_GUESS_ARRAY_FALLBACK && !fell_back) status = PFX_CELL_SINGULAR;
+          else deferred = true;
         }
       }
       const double bad = gmax<G>(status == PFX_CELL_SINGULAR ? 1.0 : 0.0, lane);
@@ -1612,6 +1789,7 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(W))) void
     const pfx_kernel_params *zone_params, const pfx_zone_launch Z, uint64_t *finish) {
   zones_body<XM>(zone_params, Z, finish);
 }
+#if !defined(PFX_REACT_PART) || PFX_REACT_PART == 3
 template __global__ void pfx_react_zones_kernel<1, false>(const pfx_kernel_params *, const pfx_zone_launch,
                                                           uint64_t *);
 template __global__ void pfx_react_zones_kernel<2, false>(const pfx_kernel_params *, const pfx_zone_launch,
@@ -1620,6 +1798,7 @@ template __global__ void pfx_react_zones_kernel<3, false>(const pfx_kernel_param
                                                           uint64_t *);
 template __global__ void pfx_react_zones_kernel<1, true>(const pfx_kernel_params *, const pfx_zone_launch,
                                                          uint64_t *);
+#endif
 
 #define PFX_INST_LU(G, MODE, W, LUP, XM) \
   template __global__ void pfx_react_kernel<G, MODE, W, LUP, XM>(const pfx_kernel_params);
@@ -1640,11 +1819,18 @@ template __global__ void pfx_react_zones_kernel<1, true>(const pfx_kernel_params
   PFX_INST_LU(G, PFX_MODE_REACT, 1, PFX_LU_ONDEMAND, true)  \
   PFX_INST_LU(G, PFX_MODE_REACT, 1, PFX_LU_PIVOT, true)     \
   PFX_INST_LU(G, PFX_MODE_EVAL, 1, PFX_LU_PIVOT, true)
+// The instantiations are compiled in parts (PFX_REACT_PART 0..3), each its
+// own object, so that they build in parallel; without it one object has all.
+#if !defined(PFX_REACT_PART) || PFX_REACT_PART == 0
 PFX_INST(8)
-PFX_INST(16)
-PFX_INST(32)
-
 extern "C" int pfx_scr_doubles(int M, int G, int K, int xm) { return scr_doubles(M, G, K, xm != 0); }
+#endif
+#if !defined(PFX_REACT_PART) || PFX_REACT_PART == 1
+PFX_INST(16)
+#endif
+#if !defined(PFX_REACT_PART) || PFX_REACT_PART == 2
+PFX_INST(32)
+#endif
 
 #ifdef PFX_SECTION_TIMERS
 // Profiling build only (no counterpart in the reference): read and clear the
