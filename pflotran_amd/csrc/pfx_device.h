@@ -150,9 +150,9 @@ const int32_t *bsr_row_ptr(const ::pfx_bsr *h);
 int64_t bsr_rows(const ::pfx_bsr *h);
 int32_t bsr_block(const ::pfx_bsr *h);
 int64_t bsr_nnzb(const ::pfx_bsr *h);
-// right-hand-side and solution vectors [nrows][C] of a handle's
-// several-right-hand-side solve (allocated on first use)
-int bsr_multi_io(::pfx_bsr *h, int C, double **B, double **X);
+// right-hand-side vectors [nrows][C] of a handle's several-right-hand-side
+// solve (allocated on first use)
+int bsr_multi_rhs(::pfx_bsr *h, int C, double **B);
 // allocate what a reaction step of these cells needs (before a graph capture)
 int tables_reserve(pfx_tables *t, const pfx_cells *cells);
 // arm pfx_tables_stats for a replayed stream-ordered reaction step of n cells

@@ -271,9 +271,8 @@ struct os_params {
   const double *porosity, *saturation, *volume;
   double def_porosity, def_saturation, def_volume, dt;
   double *vals;        // [nnzb] matrix
-  double *rhs, *x;     // [ncells] one component
-  double *total;       // [ncells][N] in: old totals; out: transported
-  int32_t comp;
+  double *rhs;         // [ncells][N] right-hand sides
+  const double *total; // [ncells][N] old totals
 };
 
 __device__ __forceinline__ double os_accum(const os_params &P, int64_t c) {
@@ -341,33 +340,6 @@ __global__ void k_os_matrix(const os_params P) {
   }
 }
 
-// right-hand side of one component: accum * T_old plus T_up * T_bc on faces
-// with a boundary total; the old totals start the solve's bookkeeping only
-__global__ void k_os_rhs(const os_params P) {
-  const int64_t nx = P.nx, ny = P.ny, n = nx * ny * (int64_t)P.nz;
-  const int64_t c = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (c >= n) return;
-  const int64_t i = c % nx, j = (c / nx) % ny, k = c / (nx * ny);
-  double r = os_accum(P, c) * P.total[c * P.N + P.comp];
-#pragma unroll
-  for (int side = 0; side < 2; side++) {
-    if (P.bc_q[side] && P.bc_total[side] && i == (side == 0 ? 0 : nx - 1)) {
-      const int64_t f = j + ny * k;
-      double Tup, Tdn;
-      flux_coef(P.area[0], P.bc_q[side][f], P.bc_dd[side][f], Tup, Tdn);
-      r += Tup * P.bc_total[side][P.comp];
-    }
-  }
-  P.rhs[c] = r;
-}
-
-__global__ void k_os_scatter(const os_params P) {
-  const int64_t n = (int64_t)P.nx * P.ny * P.nz;
-  const int64_t c = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (c >= n) return;
-  P.total[c * P.N + P.comp] = P.x[c];
-}
-
 // every component's right-hand side at once, cell-major [n][N] (the
 // layout of the totals and of the several-right-hand-side solve)
 __global__ void k_os_rhs_all(const os_params P) {
@@ -388,12 +360,6 @@ __global__ void k_os_rhs_all(const os_params P) {
     }
   }
   P.rhs[e] = r;
-}
-
-__global__ void k_os_scatter_all(const os_params P) {
-  const int64_t n = (int64_t)P.nx * P.ny * P.nz;
-  const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (e < n * P.N) P.total[e] = P.x[e];
 }
 
 extern "C" int pfx_gi_structure(const pfx_grid *g, int32_t *row_ptr, int32_t *col_idx, int64_t *nnzb) {
@@ -539,8 +505,6 @@ extern "C" int pfx_os_transport_step(pfx_bsr *h, const pfx_grid *g, pfx_cells *c
   P.def_volume = o->volume;
   P.dt = o->dt;
   P.vals = work;
-  P.rhs = work + nnzb;
-  P.x = work + nnzb + n;
   P.total = cells->total;
   P.row_ptr = pfx_internal::bsr_row_ptr(h);
   // the handle must hold this grid's pattern at block size 1: the matrix
@@ -553,22 +517,19 @@ extern "C" int pfx_os_transport_step(pfx_bsr *h, const pfx_grid *g, pfx_cells *c
   // every component in one several-right-hand-side solve, cell-major as
   // the totals are (one pfx_bsr_solve per component has the same scalars
   // and tests per component, in ncomp times the launches)
-  double *B = nullptr, *X = nullptr;
-  if ((rc = pfx_internal::bsr_multi_io(h, ncomp, &B, &X))) return rc;
+  // and writes its solution over the totals, which it does not read
+  double *B = nullptr;
+  if ((rc = pfx_internal::bsr_multi_rhs(h, ncomp, &B))) return rc;
   P.rhs = B;
-  P.x = X;
   const unsigned ge = (unsigned)((n * ncomp + 255) / 256);
   hipLaunchKernelGGL(k_os_matrix, dim3(gb), dim3(256), 0, s, P);
   hipLaunchKernelGGL(k_os_rhs_all, dim3(ge), dim3(256), 0, s, P);
   GCHK(hipGetLastError());
   pfx_krylov_stats acc;
   memset(&acc, 0, sizeof(acc));
-  rc = pfx_bsr_solve_multi(h, P.vals, B, X, ncomp, kopts, o->stream, o->stream_ordered, &acc);
+  rc = pfx_bsr_solve_multi(h, P.vals, B, cells->total, ncomp, kopts, o->stream, o->stream_ordered, &acc);
   if (rc) return rc;
-  hipLaunchKernelGGL(k_os_scatter_all, dim3(ge), dim3(256), 0, s, P);
-  GCHK(hipGetLastError());
   if (o->stream_ordered) return 0;   // the outcome: pfx_bsr_multi_stats
-  GCHK(hipStreamSynchronize(s));
   if (stats) *stats = acc;
   return acc.reason < 0 ? 1 : 0;
 }
@@ -610,8 +571,8 @@ extern "C" int pfx_os_graph_create(pfx_bsr *h, const pfx_grid *grid, pfx_tables 
   to.stream_ordered = 1;
   ro.stream_ordered = 1;
   // every buffer the three calls use is allocated before the capture
-  double *B = nullptr, *X = nullptr;
-  int rc0 = pfx_internal::bsr_multi_io(h, ncomp, &B, &X);
+  double *B = nullptr;
+  int rc0 = pfx_internal::bsr_multi_rhs(h, ncomp, &B);
   if (rc0 == 0) rc0 = pfx_internal::tables_reserve(tables, cells);
   if (rc0) {
     delete g;

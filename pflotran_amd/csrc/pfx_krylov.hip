@@ -36,6 +36,7 @@ namespace {
 
 constexpr int BLOCK = 256;
 constexpr int MAX_GRID = 4096;  // workgroups of the grid-stride kernels
+constexpr int MRHS_GRID = 2048; // of the several-right-hand-side kernels: 8 a compute unit
 
 // sum of (a, b) and (c, d) over the workgroup into partial[2 * blockIdx.x]
 __device__ __forceinline__ void block_reduce2(double a, double b, double *partial) {
@@ -467,10 +468,18 @@ __global__ __launch_bounds__(BLOCK) void k_newton_update(int64_t n, double *__re
 // components per cell); a workgroup holds RB = BLOCK / C whole rows, thread t
 // owns component t % C of row t / C, so each thread always sees the same
 // component and the per-component partial sums of a workgroup are fixed-order
-// sums.  One-workgroup kernels turn the partial sums into each component's
-// scalars and convergence status; the element kernels skip components whose
-// status is set.  No value goes to the host between iterations: a solve is
-// stream-ordered and can be captured in a graph.
+// sums.  The last workgroup of a reducing launch turns the partial sums into
+// each component's scalars and convergence status; the element kernels skip
+// components whose status is set.  No value goes to the host between
+// iterations: a solve is stream-ordered and can be captured in a graph.
+//
+// HBM-bound: 19 passes over an [n][C] vector per iteration (4 p, 3 v, 3 s, 2 t,
+// 7 xr).  The preconditioned vectors are not stored (1/diagonal times p or s
+// where they are used), and the first iteration reads the right-hand side in
+// the place of r, rhat and p, so nothing is initialised.  128^3 x 15
+// components, 3 iterations each: 28.3 ms with one thread a component adding
+// all workgroups' partial sums, 4.9 ms with the whole workgroup adding them
+// (mrhs_sums) and these passes.
 struct mrhs_sc {
   double rho, rho_new, alpha, omega, beta;
   double tol, rnorm0, rnorm, dtol;
@@ -482,48 +491,70 @@ struct mrhs_sc {
 
 __device__ __forceinline__ int mrhs_comps(int C) { return (BLOCK / C) * C; }
 
-// per-component sums over this workgroup's threads: thread c < C of the
-// workgroup writes partial[(blockIdx.x * C + c) * 2 + {0,1}]
-__device__ __forceinline__ void mrhs_block_sum(double a, double b, int C, double *partial) {
-  __shared__ double sh[2][BLOCK];
-  sh[0][threadIdx.x] = a;
-  sh[1][threadIdx.x] = b;
+// per-component sums of NS values over this workgroup's threads: thread c < C
+// of the workgroup writes partial[(blockIdx.x * C + c) * NS + {0..NS-1}]
+template <int NS>
+__device__ __forceinline__ void mrhs_block_sum(const double (&v)[NS], int C, double *partial) {
+  __shared__ double sh[NS][BLOCK];
+#pragma unroll
+  for (int q = 0; q < NS; q++) sh[q][threadIdx.x] = v[q];
   __syncthreads();
   const int used = mrhs_comps(C);
   if ((int)threadIdx.x < C) {
-    double s0 = 0.0, s1 = 0.0;
-    for (int t = threadIdx.x; t < used; t += C) {
-      s0 += sh[0][t];
-      s1 += sh[1][t];
+#pragma unroll
+    for (int q = 0; q < NS; q++) {
+      double s = 0.0;
+      for (int t = threadIdx.x; t < used; t += C) s += sh[q][t];
+      __hip_atomic_store(&partial[((int64_t)blockIdx.x * C + threadIdx.x) * NS + q], s, __ATOMIC_RELAXED,
+                         __HIP_MEMORY_SCOPE_AGENT);
     }
-    partial[((int64_t)blockIdx.x * C + threadIdx.x) * 2] = s0;
-    partial[((int64_t)blockIdx.x * C + threadIdx.x) * 2 + 1] = s1;
   }
 }
 
-// true in the workgroup that finishes last (its partial sums, and every
-// other workgroup's, are then visible to it); that workgroup turns the
-// partial sums into the scalars and re-arms the counter
+// True in the workgroup that finishes last; that workgroup turns the partial
+// sums into the scalars and re-arms the counter.  The partial sums are stored
+// and loaded as device-scope atomics, which pass through the caches that the
+// XCDs do not share, and every wavefront waits for its stores before the
+// workgroup counts itself done: no fence is needed.  (A device-scope fence in
+// each workgroup writes the XCD's whole L2 back: it made a 3-pass kernel over
+// 250 MB take 416 us instead of 145.)
 __device__ __forceinline__ bool mrhs_last_block(int *counter) {
   __shared__ int last;
-  __threadfence();
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   __syncthreads();
   if (threadIdx.x == 0) last = atomicAdd(counter, 1) == (int)gridDim.x - 1;
   __syncthreads();
-  if (last) {
-    __threadfence();
-    if (threadIdx.x == 0) *counter = 0;
-  }
+  if (last && threadIdx.x == 0) *counter = 0;
   return last;
 }
 
-// the two sums of component c over the nb workgroups, in workgroup order
-__device__ __forceinline__ void mrhs_sums(int nb, int C, int c, const double *partial, double &a, double &b) {
-  a = 0.0;
-  b = 0.0;
-  for (int k = 0; k < nb; k++) {
-    a += partial[((int64_t)k * C + c) * 2];
-    b += partial[((int64_t)k * C + c) * 2 + 1];
+// the sums of component threadIdx.x (< C) over the nb workgroups, in a fixed
+// order: thread t adds component t % C of every (BLOCK / C)-th workgroup,
+// then thread c adds those.  (One thread a component took a millisecond over
+// 4096 workgroups: each load waited for the one before.)
+template <int NS>
+__device__ __forceinline__ void mrhs_sums(int nb, int C, const double *partial, double (&out)[NS]) {
+  __shared__ double sh[NS][BLOCK];
+  const int used = mrhs_comps(C), c = threadIdx.x % C, step = BLOCK / C;
+  double v[NS];
+#pragma unroll
+  for (int q = 0; q < NS; q++) v[q] = 0.0;
+  if ((int)threadIdx.x < used) {
+#pragma unroll 8
+    for (int k = threadIdx.x / C; k < nb; k += step)
+#pragma unroll
+      for (int q = 0; q < NS; q++)
+        v[q] += __hip_atomic_load(&partial[((int64_t)k * C + c) * NS + q], __ATOMIC_RELAXED,
+                                  __HIP_MEMORY_SCOPE_AGENT);
+  }
+#pragma unroll
+  for (int q = 0; q < NS; q++) sh[q][threadIdx.x] = v[q];
+  __syncthreads();
+#pragma unroll
+  for (int q = 0; q < NS; q++) {
+    out[q] = 0.0;
+    if ((int)threadIdx.x < C)
+      for (int t = threadIdx.x; t < used; t += C) out[q] += sh[q][t];
   }
 }
 
@@ -536,26 +567,36 @@ __device__ __forceinline__ void mrhs_set_done(int C, const mrhs_sc *sc, int *don
   }
 }
 
-// grid-stride loop over the rows of a workgroup's threads
+// The rows of a workgroup's threads: one contiguous range a workgroup, and the
+// workgroups of an XCD (round-robin by index) take neighbouring ranges, so
+// that the rows a product gathers from the planes above and below are being
+// read by the same XCD at about the same time.
+#define MRHS_RANGE(n)                                                         \
+  const int64_t len_ = ((n) + gridDim.x - 1) / gridDim.x;                     \
+  const int64_t r0_ = len_ * ((gridDim.x & 7) ? blockIdx.x                    \
+                                              : (blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3)); \
+  const int64_t r1_ = r0_ + len_ < (n) ? r0_ + len_ : (n);
+
 #define MRHS_ROWS(n, C)                                                       \
   const int c_ = threadIdx.x % (C);                                           \
   const int rl_ = threadIdx.x / (C);                                          \
   const bool on_ = (int)threadIdx.x < mrhs_comps(C);                          \
-  const int64_t rstep_ = (int64_t)gridDim.x * (BLOCK / (C));                  \
-  for (int64_t row = (int64_t)blockIdx.x * (BLOCK / (C)) + rl_; on_ && row < (n); row += rstep_)
+  MRHS_RANGE(n)                                                               \
+  for (int64_t row = r0_ + rl_; on_ && row < r1_; row += BLOCK / (C))
 
 struct mrhs_args {
   int64_t n;
-  int C, nb, maxit, reserved;
+  int C, nb, maxit, first;   // first: this iteration's r, rhat and p are b, and x is zero
   const int32_t *rp, *ci;
   const double *vals, *dinv, *b;
-  double *x, *r, *rh, *p, *v, *s, *t, *ph, *sh;
+  double *x, *r, *p, *v, *s, *t;
   double *partial;
   mrhs_sc *sc;
   int *counter, *done, *fail;
   double rtol, atol, dtol;
 };
 
+// dinv = 1 / diagonal
 __global__ __launch_bounds__(BLOCK) void k_m_diag(int64_t n, const int32_t *__restrict__ rp,
                                                   const int32_t *__restrict__ ci, const double *__restrict__ vals,
                                                   double *__restrict__ dinv, int *__restrict__ fail) {
@@ -568,196 +609,422 @@ __global__ __launch_bounds__(BLOCK) void k_m_diag(int64_t n, const int32_t *__re
   dinv[row] = d != 0.0 ? 1.0 / d : 0.0;
 }
 
-// x = 0, r = rhat = b, p = v = 0; then the first scalars and the start
-// tests of every component
+// A D^-1, the matrix that both products of an iteration use
+__global__ __launch_bounds__(BLOCK) void k_m_scale(int64_t nnz, const int32_t *__restrict__ ci,
+                                                   const double *__restrict__ vals, const double *__restrict__ dinv,
+                                                   double *__restrict__ out) {
+  for (int64_t k = (int64_t)blockIdx.x * BLOCK + threadIdx.x; k < nnz; k += (int64_t)gridDim.x * BLOCK)
+    out[k] = vals[k] * dinv[ci[k]];
+}
+
+// one component's scalars before the first iteration, (b, b) = sum
+__device__ __forceinline__ mrhs_sc mrhs_start(double sum, double rtol, double atol, double dtol, int fail) {
+  mrhs_sc S;
+  S.rnorm0 = sqrt(sum);
+  S.rnorm = S.rnorm0;
+  S.tol = fmax(rtol * S.rnorm0, atol);
+  S.dtol = dtol * S.rnorm0;
+  S.conv = rtol * S.rnorm0 >= atol ? PFX_KSP_CONVERGED_RTOL : PFX_KSP_CONVERGED_ATOL;
+  S.rho = 1.0;
+  S.alpha = 1.0;
+  S.omega = 1.0;
+  S.rho_new = sum;
+  S.beta = 0.0;
+  S.it = 0;
+  S.pending = 0;
+  S.status = 0;
+  if (fail > 0) S.status = PFX_KSP_DIVERGED_PC_FAILED;
+  else if (!isfinite(S.rnorm0)) S.status = PFX_KSP_DIVERGED_NANORINF;
+  else if (S.rnorm0 <= S.tol) S.status = S.conv;
+  return S;
+}
+
+// alpha = rho_new / (rhat, v)
+__device__ __forceinline__ void mrhs_alpha(mrhs_sc &S, double rv) {
+  if (rv == 0.0 || !isfinite(rv)) {
+    S.status = isfinite(rv) ? PFX_KSP_DIVERGED_BREAKDOWN : PFX_KSP_DIVERGED_NANORINF;
+    S.it += 1;
+  } else {
+    S.alpha = S.rho_new / rv;
+  }
+}
+
+// BiCGStab's early exit: |s| <= tol converges with x += alpha phat owed
+__device__ __forceinline__ void mrhs_snorm(mrhs_sc &S, double ss) {
+  const double sn = sqrt(ss);
+  if (!isfinite(sn)) {
+    S.status = PFX_KSP_DIVERGED_NANORINF;
+    S.it += 1;
+  } else if (sn <= S.tol) {
+    S.rnorm = sn;
+    S.status = S.conv;
+    S.pending = 1;
+    S.it += 1;
+  }
+}
+
+// omega = (t, s) / (t, t)
+__device__ __forceinline__ void mrhs_omega(mrhs_sc &S, double ts, double tt) {
+  if (tt == 0.0 || !isfinite(tt)) {
+    S.status = isfinite(tt) ? PFX_KSP_DIVERGED_BREAKDOWN : PFX_KSP_DIVERGED_NANORINF;
+    S.it += 1;
+  } else {
+    S.omega = ts / tt;
+  }
+}
+
+// the residual tests, and the next iteration's start tests (iteration limit,
+// breakdown) and beta
+__device__ __forceinline__ void mrhs_end(mrhs_sc &S, double rr, double hr, int maxit) {
+  S.it += 1;
+  S.rho = S.rho_new;
+  S.rho_new = hr;
+  S.rnorm = sqrt(rr);
+  if (!isfinite(S.rnorm)) S.status = PFX_KSP_DIVERGED_NANORINF;
+  else if (S.rnorm <= S.tol) S.status = S.conv;
+  else if (S.rnorm >= S.dtol) S.status = PFX_KSP_DIVERGED_DTOL;
+  else if (S.it >= maxit) S.status = PFX_KSP_DIVERGED_ITS;
+  else if (S.rho_new == 0.0 || S.omega == 0.0) S.status = PFX_KSP_DIVERGED_BREAKDOWN;
+  else S.beta = (S.rho_new / S.rho) * (S.alpha / S.omega);
+}
+
+// (b, b), the first scalars and the start tests of every component; x is
+// cleared where a component's solve ends before it starts
 __global__ __launch_bounds__(BLOCK) void k_m_init(const mrhs_args A) {
   const int C = A.C;
-  double bb = 0.0;
+  double bb[1] = {0.0};
   MRHS_ROWS(A.n, C) {
-    const int64_t i = row * C + c_;
-    const double bi = A.b[i];
-    A.x[i] = 0.0;
-    A.r[i] = bi;
-    A.rh[i] = bi;
-    A.p[i] = 0.0;
-    A.v[i] = 0.0;
-    bb += bi * bi;
+    const double bi = A.b[row * C + c_];
+    bb[0] += bi * bi;
   }
-  mrhs_block_sum(bb, 0.0, C, A.partial);
+  mrhs_block_sum(bb, C, A.partial);
   if (!mrhs_last_block(A.counter)) return;
-  const int c = threadIdx.x;
-  if (c < C) {
-    double sum, unused;
-    mrhs_sums(A.nb, C, c, A.partial, sum, unused);
-    mrhs_sc S;
-    S.rnorm0 = sqrt(sum);
-    S.rnorm = S.rnorm0;
-    S.tol = fmax(A.rtol * S.rnorm0, A.atol);
-    S.dtol = A.dtol * S.rnorm0;
-    S.conv = A.rtol * S.rnorm0 >= A.atol ? PFX_KSP_CONVERGED_RTOL : PFX_KSP_CONVERGED_ATOL;
-    S.rho = 1.0;
-    S.alpha = 1.0;
-    S.omega = 1.0;
-    S.rho_new = sum;
-    S.beta = 0.0;
-    S.it = 0;
-    S.pending = 0;
-    S.status = 0;
-    if (*A.fail > 0) S.status = PFX_KSP_DIVERGED_PC_FAILED;
-    else if (!isfinite(S.rnorm0)) S.status = PFX_KSP_DIVERGED_NANORINF;
-    else if (S.rnorm0 <= S.tol) S.status = S.conv;
-    A.sc[c] = S;
-  }
+  double sum[1];
+  mrhs_sums(A.nb, C, A.partial, sum);
+  if ((int)threadIdx.x < C) A.sc[threadIdx.x] = mrhs_start(sum[0], A.rtol, A.atol, A.dtol, *A.fail);
   mrhs_set_done(C, A.sc, A.done);
 }
 
-// p = r + beta (p - omega v);  phat = D^-1 p
-__global__ __launch_bounds__(BLOCK) void k_m_p(const mrhs_args A) {
-  if (*A.done) return;
+// x = 0 of the components already decided at the start
+__global__ __launch_bounds__(BLOCK) void k_m_zero(const mrhs_args A) {
   const int C = A.C;
   MRHS_ROWS(A.n, C) {
-    if (A.sc[c_].status != 0) continue;
-    const int64_t i = row * C + c_;
-    const double pv = A.r[i] + A.sc[c_].beta * (A.p[i] - A.sc[c_].omega * A.v[i]);
-    A.p[i] = pv;
-    A.ph[i] = A.dinv[row] * pv;
+    if (A.sc[c_].status == 0) break;
+    A.x[row * C + c_] = 0.0;
   }
 }
 
-// v = A phat, partial (rhat, v); then alpha = rho_new / (rhat, v)
+// p = r + beta (p - omega v); in the second iteration the first one's p is b
+__global__ __launch_bounds__(BLOCK) void k_m_p(const mrhs_args A, const double *__restrict__ pold) {
+  if (*A.done) return;
+  const int C = A.C;
+  MRHS_ROWS(A.n, C) {
+    if (A.sc[c_].status != 0) break;
+    const int64_t i = row * C + c_;
+    A.p[i] = A.r[i] + A.sc[c_].beta * (pold[i] - A.sc[c_].omega * A.v[i]);
+  }
+}
+
+// A D^-1 y over the workgroup's rows: f(i, value) for every element i = row C
+// + c of a running component.  The C threads of a row need the same matrix
+// entries: a tile of MRHS_TILE rows a thread has its entries staged in LDS by
+// one coalesced read, and the threads then have only the gathers of y to wait
+// for, MRHS_TILE rows' worth in flight (128^3 x 15: 298 -> 235 us for the product
+// with s against each thread reading the row's entries itself).  A tile with
+// more entries than the stage holds reads them from memory.
+constexpr int MRHS_TILE = 4, MRHS_STAGE = 1792;   // 256 rows of 7 entries
+
+template <class F>
+__device__ __forceinline__ void mrhs_product(const mrhs_args &A, const double *y, F &&f) {
+  __shared__ int32_t s_rp[MRHS_STAGE / 7 + 1];
+  __shared__ int32_t s_ci[MRHS_STAGE];
+  __shared__ double s_a[MRHS_STAGE];
+  const int C = A.C, rb = BLOCK / C, c = threadIdx.x % C, rl = threadIdx.x / C;
+  const bool on = (int)threadIdx.x < rb * C && A.sc[c].status == 0;
+  const int per = min(MRHS_TILE, max(1, MRHS_STAGE / (7 * rb))), tile = per * rb;
+  MRHS_RANGE(A.n)
+  for (int64_t t0 = r0_; t0 < r1_; t0 += tile) {
+    const int nr = (int)(r1_ - t0 < tile ? r1_ - t0 : tile);
+    __syncthreads();   // the last tile's entries have been read
+    for (int i = threadIdx.x; i <= nr; i += BLOCK) s_rp[i] = A.rp[t0 + i];
+    __syncthreads();
+    const int32_t e0 = s_rp[0], ne = s_rp[nr] - e0;
+    const bool staged = ne <= MRHS_STAGE;
+    if (staged)
+      for (int i = threadIdx.x; i < ne; i += BLOCK) {
+        s_ci[i] = A.ci[e0 + i];
+        s_a[i] = A.vals[e0 + i];
+      }
+    __syncthreads();
+    if (!on) continue;
+    if (staged) {
+      double acc[MRHS_TILE];
+      int k0[MRHS_TILE], k1[MRHS_TILE];
+#pragma unroll
+      for (int u = 0; u < MRHS_TILE; u++) {
+        const int i = u * rb + rl;
+        acc[u] = 0.0;
+        k0[u] = i < nr ? s_rp[i] - e0 : 0;
+        k1[u] = i < nr ? s_rp[i + 1] - e0 : 0;
+      }
+      // seven entries of every row at a time (a grid's interior rows whole)
+      for (int k = 0;; k += 7) {
+        bool more = false;
+#pragma unroll
+        for (int u = 0; u < MRHS_TILE; u++) {
+          double z[7], a[7];
+#pragma unroll
+          for (int q = 0; q < 7; q++) {
+            const int kk = k0[u] + k + q;
+            const bool in = kk < k1[u];
+            a[q] = in ? s_a[kk] : 0.0;
+            z[q] = in ? y[(int64_t)s_ci[kk] * C + c] : 0.0;
+          }
+#pragma unroll
+          for (int q = 0; q < 7; q++) acc[u] += a[q] * z[q];
+          more = more || k0[u] + k + 7 < k1[u];
+        }
+        if (!more) break;
+      }
+#pragma unroll
+      for (int u = 0; u < MRHS_TILE; u++)
+        if (u * rb + rl < nr) f((t0 + u * rb + rl) * C + c, acc[u]);
+    } else {
+      for (int i = rl; i < nr; i += rb) {
+        double acc = 0.0;
+        for (int32_t k = s_rp[i]; k < s_rp[i + 1]; k++) acc += A.vals[k] * y[(int64_t)A.ci[k] * C + c];
+        f((t0 + i) * C + c, acc);
+      }
+    }
+  }
+}
+
+// v = A D^-1 p, partial (rhat, v), rhat = b; then alpha
 __global__ __launch_bounds__(BLOCK) void k_m_v(const mrhs_args A) {
   if (*A.done) return;
   const int C = A.C;
-  double a = 0.0;
-  MRHS_ROWS(A.n, C) {
-    if (A.sc[c_].status != 0) continue;
-    double acc = 0.0;
-    for (int32_t k = A.rp[row]; k < A.rp[row + 1]; k++) acc += A.vals[k] * A.ph[(int64_t)A.ci[k] * C + c_];
-    const int64_t i = row * C + c_;
+  double a[1] = {0.0};
+  mrhs_product(A, A.first ? A.b : A.p, [&](int64_t i, double acc) {
     A.v[i] = acc;
-    a += A.rh[i] * acc;
-  }
-  mrhs_block_sum(a, 0.0, C, A.partial);
+    a[0] += A.b[i] * acc;
+  });
+  mrhs_block_sum(a, C, A.partial);
   if (!mrhs_last_block(A.counter)) return;
+  double sum[1];
+  mrhs_sums(A.nb, C, A.partial, sum);
   const int c = threadIdx.x;
-  if (c < C && A.sc[c].status == 0) {
-    double rv, unused;
-    mrhs_sums(A.nb, C, c, A.partial, rv, unused);
-    if (rv == 0.0 || !isfinite(rv)) {
-      A.sc[c].status = isfinite(rv) ? PFX_KSP_DIVERGED_BREAKDOWN : PFX_KSP_DIVERGED_NANORINF;
-      A.sc[c].it += 1;
-    } else {
-      A.sc[c].alpha = A.sc[c].rho_new / rv;
-    }
-  }
+  if (c < C && A.sc[c].status == 0) mrhs_alpha(A.sc[c], sum[0]);
 }
 
-// s = r - alpha v;  shat = D^-1 s;  partial (s, s); then BiCGStab's early
-// exit: |s| <= tol converges with x += alpha phat owed
+// s = r - alpha v, partial (s, s)
 __global__ __launch_bounds__(BLOCK) void k_m_s(const mrhs_args A) {
   if (*A.done) return;
   const int C = A.C;
-  double ss = 0.0;
+  const double *r = A.first ? A.b : A.r;
+  double ss[1] = {0.0};
   MRHS_ROWS(A.n, C) {
-    if (A.sc[c_].status != 0) continue;
+    if (A.sc[c_].status != 0) break;
     const int64_t i = row * C + c_;
-    const double si = A.r[i] - A.sc[c_].alpha * A.v[i];
+    const double si = r[i] - A.sc[c_].alpha * A.v[i];
     A.s[i] = si;
-    A.sh[i] = A.dinv[row] * si;
-    ss += si * si;
+    ss[0] += si * si;
   }
-  mrhs_block_sum(ss, 0.0, C, A.partial);
+  mrhs_block_sum(ss, C, A.partial);
   if (!mrhs_last_block(A.counter)) return;
+  double sum[1];
+  mrhs_sums(A.nb, C, A.partial, sum);
   const int c = threadIdx.x;
-  if (c < C && A.sc[c].status == 0) {
-    double sum, unused;
-    mrhs_sums(A.nb, C, c, A.partial, sum, unused);
-    const double sn = sqrt(sum);
-    if (!isfinite(sn)) {
-      A.sc[c].status = PFX_KSP_DIVERGED_NANORINF;
-      A.sc[c].it += 1;
-    } else if (sn <= A.sc[c].tol) {
-      A.sc[c].rnorm = sn;
-      A.sc[c].status = A.sc[c].conv;
-      A.sc[c].pending = 1;
-      A.sc[c].it += 1;
-    }
-  }
+  if (c < C && A.sc[c].status == 0) mrhs_snorm(A.sc[c], sum[0]);
 }
 
-// t = A shat, partial (t, s), (t, t); then omega = (t, s) / (t, t)
+// t = A D^-1 s, partial (t, s), (t, t); then omega
 __global__ __launch_bounds__(BLOCK) void k_m_t(const mrhs_args A) {
   if (*A.done) return;
   const int C = A.C;
-  double ts = 0.0, tt = 0.0;
-  MRHS_ROWS(A.n, C) {
-    if (A.sc[c_].status != 0) continue;
-    double acc = 0.0;
-    for (int32_t k = A.rp[row]; k < A.rp[row + 1]; k++) acc += A.vals[k] * A.sh[(int64_t)A.ci[k] * C + c_];
-    const int64_t i = row * C + c_;
+  double a[2] = {0.0, 0.0};
+  mrhs_product(A, A.s, [&](int64_t i, double acc) {
     A.t[i] = acc;
-    ts += A.s[i] * acc;
-    tt += acc * acc;
-  }
-  mrhs_block_sum(ts, tt, C, A.partial);
+    a[0] += A.s[i] * acc;
+    a[1] += acc * acc;
+  });
+  mrhs_block_sum(a, C, A.partial);
   if (!mrhs_last_block(A.counter)) return;
+  double sum[2];
+  mrhs_sums(A.nb, C, A.partial, sum);
   const int c = threadIdx.x;
-  if (c < C && A.sc[c].status == 0) {
-    double sts, stt;
-    mrhs_sums(A.nb, C, c, A.partial, sts, stt);
-    if (stt == 0.0 || !isfinite(stt)) {
-      A.sc[c].status = isfinite(stt) ? PFX_KSP_DIVERGED_BREAKDOWN : PFX_KSP_DIVERGED_NANORINF;
-      A.sc[c].it += 1;
-    } else {
-      A.sc[c].omega = sts / stt;
-    }
-  }
+  if (c < C && A.sc[c].status == 0) mrhs_omega(A.sc[c], sum[0], sum[1]);
 }
 
-// x += alpha phat + omega shat;  r = s - omega t;  partial (r, r),
-// (rhat, r) (a component converged on |s| takes x += alpha phat only); then
-// the residual tests, and the next iteration's start tests (iteration
-// limit, breakdown) and beta
+// x += D^-1 (alpha p + omega s);  r = s - omega t;  partial (r, r), (rhat, r)
+// (a component converged on |s| takes x += alpha D^-1 p only)
 __global__ __launch_bounds__(BLOCK) void k_m_xr(const mrhs_args A) {
   if (*A.done) return;
   const int C = A.C;
-  double rr = 0.0, hr = 0.0;
+  const double *p = A.first ? A.b : A.p;
+  double a[2] = {0.0, 0.0};
   MRHS_ROWS(A.n, C) {
+    const mrhs_sc &S = A.sc[c_];
+    if (S.status != 0 && !S.pending) {
+      // a first iteration that broke down leaves x at its start, zero
+      if (A.first && S.it > 0) A.x[row * C + c_] = 0.0;
+      continue;
+    }
     const int64_t i = row * C + c_;
-    if (A.sc[c_].pending) {
-      A.x[i] += A.sc[c_].alpha * A.ph[i];
-    } else if (A.sc[c_].status == 0) {
-      A.x[i] += A.sc[c_].alpha * A.ph[i] + A.sc[c_].omega * A.sh[i];
-      const double rv = A.s[i] - A.sc[c_].omega * A.t[i];
+    const double d = A.dinv[row], x0 = A.first ? 0.0 : A.x[i];
+    if (S.pending) {
+      A.x[i] = x0 + S.alpha * (d * p[i]);
+    } else {
+      const double si = A.s[i];
+      A.x[i] = x0 + (S.alpha * (d * p[i]) + S.omega * (d * si));
+      const double rv = si - S.omega * A.t[i];
       A.r[i] = rv;
-      rr += rv * rv;
-      hr += A.rh[i] * rv;
+      a[0] += rv * rv;
+      a[1] += A.b[i] * rv;
     }
   }
-  mrhs_block_sum(rr, hr, C, A.partial);
+  mrhs_block_sum(a, C, A.partial);
   if (!mrhs_last_block(A.counter)) return;
+  double sum[2];
+  mrhs_sums(A.nb, C, A.partial, sum);
   const int c = threadIdx.x;
   if (c < C) {
     mrhs_sc S = A.sc[c];
-    if (S.pending) {
-      S.pending = 0;
-    } else if (S.status == 0) {
-      double srr, shr;
-      mrhs_sums(A.nb, C, c, A.partial, srr, shr);
-      S.it += 1;
-      S.rho = S.rho_new;
-      S.rho_new = shr;
-      S.rnorm = sqrt(srr);
-      if (!isfinite(S.rnorm)) S.status = PFX_KSP_DIVERGED_NANORINF;
-      else if (S.rnorm <= S.tol) S.status = S.conv;
-      else if (S.rnorm >= S.dtol) S.status = PFX_KSP_DIVERGED_DTOL;
-      else if (S.it >= A.maxit) S.status = PFX_KSP_DIVERGED_ITS;
-      else if (S.rho_new == 0.0 || S.omega == 0.0) S.status = PFX_KSP_DIVERGED_BREAKDOWN;
-      else S.beta = (S.rho_new / S.rho) * (S.alpha / S.omega);
-    }
+    if (S.pending) S.pending = 0;
+    else if (S.status == 0) mrhs_end(S, sum[0], sum[1], A.maxit);
     A.sc[c] = S;
   }
   mrhs_set_done(C, A.sc, A.done);
+}
+
+// The whole solve of a small system in one launch, one workgroup a component
+// (they share only the matrix): the vectors live in registers (R rows a
+// thread), the one being multiplied in LDS, and the scalars in every thread.
+// Latency-bound: a launch of its own for every step of an iteration costs
+// 2-3 us each whatever the size, five an iteration; here an iteration is two
+// products and four workgroup sums.  100 cells x 5 components, 12 enqueued
+// iterations: the captured operator-split step 227 -> 80 us.  Used up to
+// MRHS_SMALL rows, where one compute unit's share of the products still costs
+// less than the launches: 16x16x15 cells x 5 components 121 us a step, 16x16x17 by
+// launches 247.
+constexpr int MRHS_SMALL = 4096;
+
+template <int NS>
+__device__ __forceinline__ void wg_sum(double (&v)[NS], double (*sh)[16]) {
+  const int w = threadIdx.x >> 6, nw = blockDim.x >> 6;
+#pragma unroll
+  for (int q = 0; q < NS; q++)
+    for (int o = 32; o > 0; o >>= 1) v[q] += __shfl_xor(v[q], o, 64);
+  __syncthreads();   // the sums of the last call have been read
+  if ((threadIdx.x & 63) == 0)
+#pragma unroll
+    for (int q = 0; q < NS; q++) sh[q][w] = v[q];
+  __syncthreads();
+#pragma unroll
+  for (int q = 0; q < NS; q++) {
+    v[q] = 0.0;
+    for (int i = 0; i < nw; i++) v[q] += sh[q][i];
+  }
+}
+
+template <int R>
+__global__ __launch_bounds__(1024) void k_m_small(const mrhs_args A) {
+  extern __shared__ double y[];
+  __shared__ double sh[2][16];
+  const int n = (int)A.n, C = A.C, c = blockIdx.x, T = blockDim.x;
+  double b[R], d[R], x[R], r[R], p[R], v[R];
+  double bad[1] = {0.0}, one[1] = {0.0};
+#pragma unroll
+  for (int q = 0; q < R; q++) {
+    const int row = threadIdx.x + q * T;
+    b[q] = d[q] = x[q] = p[q] = v[q] = 0.0;
+    if (row < n) {
+      double dg = 0.0;
+      for (int32_t k = A.rp[row]; k < A.rp[row + 1]; k++)
+        if (A.ci[k] == row) dg = A.vals[k];
+      if (dg == 0.0 || !(dg == dg)) bad[0] += 1.0;
+      d[q] = dg != 0.0 ? 1.0 / dg : 0.0;
+      b[q] = A.b[(int64_t)row * C + c];
+    }
+    r[q] = b[q];
+    one[0] += b[q] * b[q];
+  }
+  wg_sum(bad, sh);
+  wg_sum(one, sh);
+  mrhs_sc S = mrhs_start(one[0], A.rtol, A.atol, A.dtol, bad[0] > 0.0 ? 1 : 0);
+  // row `threadIdx.x + q T` of A times the vector in y
+  auto product = [&](const double (&z)[R], double (&out)[R]) {
+    __syncthreads();   // y has been read
+#pragma unroll
+    for (int q = 0; q < R; q++)
+      if (threadIdx.x + q * T < n) y[threadIdx.x + q * T] = d[q] * z[q];
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < R; q++) {
+      const int row = threadIdx.x + q * T;
+      double acc = 0.0;
+      if (row < n)
+        for (int32_t k = A.rp[row]; k < A.rp[row + 1]; k++) acc += A.vals[k] * y[A.ci[k]];
+      out[q] = acc;
+    }
+  };
+  while (S.status == 0) {
+    if (S.it > 0) {
+#pragma unroll
+      for (int q = 0; q < R; q++) p[q] = r[q] + S.beta * (p[q] - S.omega * v[q]);
+    } else {
+#pragma unroll
+      for (int q = 0; q < R; q++) p[q] = b[q];
+    }
+    product(p, v);
+    one[0] = 0.0;
+#pragma unroll
+    for (int q = 0; q < R; q++) one[0] += b[q] * v[q];
+    wg_sum(one, sh);
+    mrhs_alpha(S, one[0]);
+    if (S.status != 0) break;
+    one[0] = 0.0;
+#pragma unroll
+    for (int q = 0; q < R; q++) {
+      r[q] -= S.alpha * v[q];   // s
+      one[0] += r[q] * r[q];
+    }
+    wg_sum(one, sh);
+    mrhs_snorm(S, one[0]);
+    if (S.pending) {
+#pragma unroll
+      for (int q = 0; q < R; q++) x[q] += S.alpha * (d[q] * p[q]);
+      S.pending = 0;
+    }
+    if (S.status != 0) break;
+    double t[R], two[2] = {0.0, 0.0};
+    product(r, t);
+#pragma unroll
+    for (int q = 0; q < R; q++) {
+      two[0] += r[q] * t[q];
+      two[1] += t[q] * t[q];
+    }
+    wg_sum(two, sh);
+    mrhs_omega(S, two[0], two[1]);
+    if (S.status != 0) break;
+    two[0] = two[1] = 0.0;
+#pragma unroll
+    for (int q = 0; q < R; q++) {
+      x[q] += S.alpha * (d[q] * p[q]) + S.omega * (d[q] * r[q]);
+      r[q] -= S.omega * t[q];
+      two[0] += r[q] * r[q];
+      two[1] += b[q] * r[q];
+    }
+    wg_sum(two, sh);
+    mrhs_end(S, two[0], two[1], A.maxit);
+  }
+#pragma unroll
+  for (int q = 0; q < R; q++)
+    if (threadIdx.x + q * T < n) A.x[(int64_t)(threadIdx.x + q * T) * C + c] = x[q];
+  if (threadIdx.x == 0) A.sc[c] = S;
+}
+
+__global__ __launch_bounds__(BLOCK) void k_copy(int64_t n, const double *__restrict__ a, double *__restrict__ b) {
+  for (int64_t i = (int64_t)blockIdx.x * BLOCK + threadIdx.x; i < n; i += (int64_t)gridDim.x * BLOCK) b[i] = a[i];
 }
 
 int grid_for(int64_t work_items) {
@@ -786,7 +1053,7 @@ struct pfx_bsr {
   // components, vectors [nrows][C], the per-component scalars, the
   // all-decided flag and its pinned host copy
   int mC = 0;
-  double *mvec = nullptr, *mdinv = nullptr, *mpartial = nullptr;
+  double *mvec = nullptr, *mdinv = nullptr, *mvals = nullptr, *mpartial = nullptr;
   mrhs_sc *msc = nullptr, *mhost_sc = nullptr;
   int *mdone = nullptr, *mhost_done = nullptr;
   int *mcounter = nullptr;   // workgroups done in the current reduction (0 between launches)
@@ -925,6 +1192,7 @@ extern "C" int pfx_bsr_destroy(pfx_bsr *h) {
   if (h->e1) (void)hipEventDestroy(h->e1);
   if (h->mvec) (void)hipFree(h->mvec);
   if (h->mdinv) (void)hipFree(h->mdinv);
+  if (h->mvals) (void)hipFree(h->mvals);
   if (h->mpartial) (void)hipFree(h->mpartial);
   if (h->msc) (void)hipFree(h->msc);
   if (h->mdone) (void)hipFree(h->mdone);
@@ -1054,15 +1322,16 @@ int ensure_multi(pfx_bsr *h, int C) {
   if (h->mC == C && h->mvec) return 0;
   if (h->mvec) KCHK(hipFree(h->mvec));
   if (h->mdinv) KCHK(hipFree(h->mdinv));
+  if (h->mvals) KCHK(hipFree(h->mvals));
   if (h->mpartial) KCHK(hipFree(h->mpartial));
-  h->mvec = h->mdinv = h->mpartial = nullptr;
+  h->mvec = h->mdinv = h->mvals = h->mpartial = nullptr;
   h->mC = 0;
   const size_t nv = (size_t)h->nrows * C;
-  // r, rhat, p, v, s, t, phat, shat, and a right-hand side and solution
-  // (pfx_os_transport_step's)
-  if (hipMalloc((void **)&h->mvec, 10 * nv * sizeof(double)) != hipSuccess ||
+  // r, p, v, s, t, and a right-hand side (pfx_os_transport_step's)
+  if (hipMalloc((void **)&h->mvec, 6 * nv * sizeof(double)) != hipSuccess ||
       hipMalloc((void **)&h->mdinv, (size_t)h->nrows * sizeof(double)) != hipSuccess ||
-      hipMalloc((void **)&h->mpartial, (size_t)MAX_GRID * C * 2 * sizeof(double)) != hipSuccess) {
+      hipMalloc((void **)&h->mvals, (size_t)h->nnzb * sizeof(double)) != hipSuccess ||
+      hipMalloc((void **)&h->mpartial, (size_t)MRHS_GRID * C * 2 * sizeof(double)) != hipSuccess) {
     (void)hipGetLastError();
     return PFX_E_NOMEM;
   }
@@ -1099,6 +1368,21 @@ void multi_stats(const mrhs_sc *sc, int C, pfx_krylov_stats *st) {
   *st = S;
 }
 
+// the end of a solve that the host waits for
+int multi_finish(pfx_bsr *h, int C, hipStream_t s, pfx_krylov_stats *st) {
+  KCHK(hipMemcpyAsync(h->mhost_sc, h->msc, C * sizeof(mrhs_sc), hipMemcpyDeviceToHost, s));
+  KCHK(hipEventRecord(h->e1, s));
+  KCHK(hipEventSynchronize(h->e1));
+  h->mpending = false;
+  if (st) {
+    multi_stats(h->mhost_sc, C, st);
+    float ms = 0.f;
+    KCHK(hipEventElapsedTime(&ms, h->e0, h->e1));
+    st->ms = ms;
+  }
+  return 0;
+}
+
 }  // namespace
 
 extern "C" int pfx_bsr_solve_multi(pfx_bsr *h, const double *values, const double *B, double *X, int32_t ncomp,
@@ -1117,10 +1401,8 @@ extern "C" int pfx_bsr_solve_multi(pfx_bsr *h, const double *values, const doubl
   const int C = ncomp;
   const int64_t n = h->nrows;
   const size_t nv = (size_t)n * C;
-  double *r = h->mvec, *rh = r + nv, *p = rh + nv, *v = p + nv, *sv = v + nv, *t = sv + nv, *ph = t + nv,
-         *sh = ph + nv;
   const int64_t rb = BLOCK / C;
-  int nb = (int)std::min<int64_t>((n + rb - 1) / rb, MAX_GRID);
+  int nb = (int)std::min<int64_t>((n + rb - 1) / rb, MRHS_GRID);
   if (nb < 1) nb = 1;
   const int gd = (int)std::min<int64_t>((n + BLOCK - 1) / BLOCK, 1 << 20);
   if (!stream_ordered) KCHK(hipEventRecord(h->e0, s));
@@ -1136,14 +1418,11 @@ extern "C" int pfx_bsr_solve_multi(pfx_bsr *h, const double *values, const doubl
   A.dinv = h->mdinv;
   A.b = B;
   A.x = X;
-  A.r = r;
-  A.rh = rh;
-  A.p = p;
-  A.v = v;
-  A.s = sv;
-  A.t = t;
-  A.ph = ph;
-  A.sh = sh;
+  A.r = h->mvec;
+  A.p = A.r + nv;
+  A.v = A.p + nv;
+  A.s = A.v + nv;
+  A.t = A.s + nv;
   A.partial = h->mpartial;
   A.sc = h->msc;
   A.counter = h->mcounter;
@@ -1152,14 +1431,37 @@ extern "C" int pfx_bsr_solve_multi(pfx_bsr *h, const double *values, const doubl
   A.rtol = rtol;
   A.atol = atol;
   A.dtol = dtol;
+  if (X == B) {
+    // in place: the right-hand side is read to the end, the handle keeps a copy
+    double *own = h->mvec + 5 * nv;
+    hipLaunchKernelGGL(k_copy, dim3(grid_for((int64_t)nv)), dim3(BLOCK), 0, s, (int64_t)nv, B, own);
+    A.b = own;
+  }
+  if (n <= MRHS_SMALL) {
+    const int T = n <= 256 ? 256 : 1024;
+    const size_t lds = (size_t)n * sizeof(double);
+    if (n <= 1024) hipLaunchKernelGGL(k_m_small<1>, dim3(C), dim3(T), lds, s, A);
+    else hipLaunchKernelGGL(k_m_small<4>, dim3(C), dim3(T), lds, s, A);
+    KCHK(hipGetLastError());
+    if (stream_ordered) {
+      h->mpending = true;
+      h->mstream = s;
+      return 0;
+    }
+    return multi_finish(h, C, s, st);
+  }
   hipLaunchKernelGGL(k_zero_int, dim3(1), dim3(1), 0, s, h->fail);
   hipLaunchKernelGGL(k_m_diag, dim3(gd), dim3(BLOCK), 0, s, n, h->rp, h->ci, values, h->mdinv, h->fail);
+  hipLaunchKernelGGL(k_m_scale, dim3(gd), dim3(BLOCK), 0, s, h->nnzb, h->ci, values, h->mdinv, h->mvals);
+  A.vals = h->mvals;
   hipLaunchKernelGGL(k_m_init, dim3(nb), dim3(BLOCK), 0, s, A);
   KCHK(hipGetLastError());
-  // five launches per iteration; each reduction's last workgroup turns the
-  // partial sums into the scalars
-  auto iteration = [&]() {
-    hipLaunchKernelGGL(k_m_p, dim3(nb), dim3(BLOCK), 0, s, A);
+  hipLaunchKernelGGL(k_m_zero, dim3(nb), dim3(BLOCK), 0, s, A);
+  // five launches per iteration (four in the first, whose p is b); each
+  // reduction's last workgroup turns the partial sums into the scalars
+  auto iteration = [&](int it) {
+    A.first = it == 0;
+    if (it > 0) hipLaunchKernelGGL(k_m_p, dim3(nb), dim3(BLOCK), 0, s, A, it == 1 ? A.b : A.p);
     hipLaunchKernelGGL(k_m_v, dim3(nb), dim3(BLOCK), 0, s, A);
     hipLaunchKernelGGL(k_m_s, dim3(nb), dim3(BLOCK), 0, s, A);
     hipLaunchKernelGGL(k_m_t, dim3(nb), dim3(BLOCK), 0, s, A);
@@ -1167,7 +1469,7 @@ extern "C" int pfx_bsr_solve_multi(pfx_bsr *h, const double *values, const doubl
   };
   if (stream_ordered) {
     // exactly maxit iterations enqueued; decided components skip their work
-    for (int it = 0; it < maxit; it++) iteration();
+    for (int it = 0; it < maxit; it++) iteration(it);
     KCHK(hipGetLastError());
     h->mpending = true;
     h->mstream = s;
@@ -1180,23 +1482,13 @@ extern "C" int pfx_bsr_solve_multi(pfx_bsr *h, const double *values, const doubl
   int it = 0;
   while (!*h->mhost_done && it < maxit) {
     const int round = std::min(4, maxit - it);
-    for (int k = 0; k < round; k++) iteration();
+    for (int k = 0; k < round; k++) iteration(it + k);
     it += round;
     KCHK(hipGetLastError());
     KCHK(hipMemcpyAsync(h->mhost_done, h->mdone, sizeof(int), hipMemcpyDeviceToHost, s));
     KCHK(hipStreamSynchronize(s));
   }
-  KCHK(hipMemcpyAsync(h->mhost_sc, h->msc, C * sizeof(mrhs_sc), hipMemcpyDeviceToHost, s));
-  KCHK(hipEventRecord(h->e1, s));
-  KCHK(hipEventSynchronize(h->e1));
-  h->mpending = false;
-  if (st) {
-    multi_stats(h->mhost_sc, C, st);
-    float ms = 0.f;
-    KCHK(hipEventElapsedTime(&ms, h->e0, h->e1));
-    st->ms = ms;
-  }
-  return 0;
+  return multi_finish(h, C, s, st);
 }
 
 extern "C" int pfx_bsr_multi_stats(pfx_bsr *h, void *stream, pfx_krylov_stats *st) {
@@ -1211,12 +1503,10 @@ extern "C" int pfx_bsr_multi_stats(pfx_bsr *h, void *stream, pfx_krylov_stats *s
 }
 
 namespace pfx_internal {
-int bsr_multi_io(pfx_bsr *h, int C, double **B, double **X) {
+int bsr_multi_rhs(pfx_bsr *h, int C, double **B) {
   int rc = ensure_multi(h, C);
   if (rc) return rc;
-  const size_t nv = (size_t)h->nrows * C;
-  *B = h->mvec + 8 * nv;
-  *X = h->mvec + 9 * nv;
+  *B = h->mvec + 5 * (size_t)h->nrows * C;
   return 0;
 }
 }  // namespace pfx_internal
