@@ -256,6 +256,39 @@ const void *zones_kernel_ptr(int v, bool xm) {
        : v == 1 ? (const void *)pfx_react_zones_kernel<2, false> : (const void *)pfx_react_zones_kernel<1, false>;
 }
 
+// Workgroups of `lds` bytes that a compute unit holds, at most `occ` (the
+// runtime's answer, which rounds LDS finer than the hardware: it counted 3
+// workgroups of 53,792 bytes where a third starts only when one ends).  LDS is
+// handed out in 128 pieces of 1,280 bytes.  The N = 15 network's workgroups,
+// 424 bytes of unused tables smaller, fit three times: 1M cells 24.8 -> 18.7 ms
+// in the variant that allows three wavefronts per SIMD.
+int resident(int occ, int64_t lds) {
+  const int64_t pieces = std::max<int64_t>(1, (lds + 1279) / 1280);
+  return (int)std::max<int64_t>(1, std::min<int64_t>(occ, 128 / pieces));
+}
+
+// Work distribution of a launch of `blocks` workgroups: the cells that each
+// wavefront owns from the start, and the most it takes per fetch of the rest.
+// Every fetch is an atomic on one address, ~39 ns each one after the other
+// whichever XCD they come from: 63k cells fetched by fours were 0.62 of the
+// 0.84 ms of an evaluation that takes 0.2.  One evaluation per cell is even
+// work, owned whole; Newton cells differ, so half of them stays in the queue to
+// level the wavefronts, in guided sizes (a quarter left four zones of unequal
+// networks 3 % slower, three quarters are no faster).  Owned shares need every
+// workgroup resident from the start: the grid is never larger (resident()).
+// Measured: 50k cells of N = 15 2.46 -> 2.09 ms, 63k-cell evaluation 0.84 ->
+// 0.24 ms, speciation of 200k cells 2.40 -> 2.06 ms.
+void distribute(pfx_kernel_params &P, int G, int mode, int64_t blocks) {
+  const int64_t waves = blocks * (BLOCK / 64), lo = 64 / G;
+  const int64_t fair = (P.ncells + waves - 1) / waves;
+  const bool even = mode == PFX_MODE_EVAL || mode == PFX_MODE_AUX;
+  int64_t share = even ? fair : fair / 2;
+  share = even ? (share + lo - 1) / lo * lo : share / lo * lo;
+  P.share = (int32_t)std::max<int64_t>(share, lo);
+  P.chunk = (int32_t)std::max<int64_t>(lo, std::min<int64_t>(64, fair / 8 + 1));
+  P.waves = (int32_t)waves;
+}
+
 // queue: the work-queue cursors and fallback counter of this launch (the
 // tables' own, or the fixed scratch array of pfx_react_batch_noalloc).
 // A reaction step with a deferred list (P.defer) is two launches: the
@@ -279,15 +312,11 @@ int launch(pfx_tables *t, pfx_kernel_params &P, int mode, hipStream_t stream, do
     if (fn_piv) HIPCHK(hipFuncSetAttribute(fn_piv, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
   }
   HIPCHK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, fn, BLOCK, (size_t)lds));
-  if (occ < 1) occ = 1;
+  occ = resident(occ, lds);
   int64_t need_blocks = (P.ncells + groups - 1) / groups;
   int64_t blocks = std::min<int64_t>(need_blocks, (int64_t)t->num_cu * occ);
   if (blocks < 1) blocks = 1;
-  // chunk: enough cells per fetch to keep queue atomics rare, small enough
-  // to balance the tail
-  int64_t per_wave = std::max<int64_t>(1, P.ncells / (blocks * (BLOCK / 64)));
-  P.chunk = (int32_t)std::max<int64_t>(64 / G, std::min<int64_t>(64, per_wave / 8 + 1));
-  P.waves = (int32_t)(blocks * (BLOCK / 64));
+  distribute(P, G, mode, blocks);
   P.queue = queue;
   P.fallback_count = queue + 1;
   // the pivoting launch: its own cursor, one cell per fetch, one workgroup
@@ -296,6 +325,7 @@ int launch(pfx_tables *t, pfx_kernel_params &P, int mode, hipStream_t stream, do
   P2.queue = queue + 2;
   P2.chunk = 1;
   P2.waves = 0;
+  P2.share = 0;
   const int64_t blocks2 = std::max<int64_t>(1, std::min<int64_t>(need_blocks, (int64_t)t->num_cu));
   hipLaunchKernelGGL(k_zero_launch, dim3(1), dim3(64), 0, stream, queue, P.defer);
   HIPCHK(hipGetLastError());
@@ -501,7 +531,7 @@ int zones_prepare(int32_t nzones, pfx_tables *const *tables, pfx_cells *cells, c
   if (zs.lds > 64 * 1024) HIPCHK(hipFuncSetAttribute(zs.fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)zs.lds));
   int occ = 0;
   HIPCHK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, zs.fn, BLOCK, (size_t)zs.lds));
-  if (occ < 1) occ = 1;
+  occ = resident(occ, zs.lds);
   const int full = tables[0]->num_cu * occ;
   int blocks[PFX_MAX_ZONES];
   bool given = plan && plan->nzones == nzones;
@@ -518,10 +548,8 @@ int zones_prepare(int32_t nzones, pfx_tables *const *tables, pfx_cells *cells, c
   for (int z = 0; z < nzones; z++) {
     zs.Z.block_start[z] = acc;
     acc += blocks[z];
-    // chunk: as in the single-batch launch, from the zone's own share
-    const int64_t per_wave = std::max<int64_t>(1, zs.n[z] / ((int64_t)blocks[z] * (BLOCK / 64)));
-    zs.P[z].chunk = (int32_t)std::max<int64_t>(64 / zs.Z.G[z], std::min<int64_t>(64, per_wave / 8 + 1));
-    zs.P[z].waves = blocks[z] * (BLOCK / 64);
+    distribute(zs.P[z], zs.Z.G[z], PFX_MODE_REACT, blocks[z]);
+    zs.P[z].block0 = zs.Z.block_start[z];
   }
   zs.Z.block_start[nzones] = acc;
   zs.total_blocks = total;
@@ -549,6 +577,8 @@ int zones_enqueue(pfx_tables *const *tables, zone_setup &zs, const pfx_kernel_pa
     P2.queue = t->d_queue + 2;
     P2.chunk = 1;
     P2.waves = 0;
+    P2.share = 0;
+    P2.block0 = 0;
     const int64_t lds = zone_lds(t);
     const void *fn_piv = kernel_ptr(t->L.G, PFX_MODE_REACT, 0, PFX_LU_PIVOT, tables_xm(t));
     if (lds > 64 * 1024) HIPCHK(hipFuncSetAttribute(fn_piv, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
@@ -961,8 +991,6 @@ extern "C" int pfx_tables_create(const pfx_reaction_desc *d, pfx_tables **out) {
   L.o_clogKcoef = B.add(ccoef);
   L.o_mlogKcoef = B.add(mcoef);
   L.o_mmolvol = B.add(mmv);
-  L.o_ch2o = B.add(std::vector<double>(std::max(M, 1), 0.0));
-  L.o_mh2o = B.add(std::vector<double>(std::max(K, 1), 0.0));
   // the coefficient tables are read per cell at load time, from the LDS copy
   // when they fit: stage the whole blob
   B.bytes.resize((B.bytes.size() + 15) & ~size_t(15));

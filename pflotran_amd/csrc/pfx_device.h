@@ -46,7 +46,6 @@ struct pfx_dev_layout {
   int64_t o_cZ, o_ca0;               // [M]
   int64_t o_clogK;                   // [M] log10 K at the reference temperature
   int64_t o_clogKcoef;               // [M][5]
-  int64_t o_ch2o;                    // [M]
   int64_t o_adj_c;                   // int32 [maxdeg][G], -> M = zero slot
   int64_t o_adj_nu;                  // [maxdeg][G]
   int64_t o_offq_c;                  // uint16 [rows][G][4] complex (M = zero slot)
@@ -54,7 +53,7 @@ struct pfx_dev_layout {
   int64_t o_mspec;                   // int32 [K][S]
   int64_t o_mnu;                     // [K][S]
   int64_t o_mnuG;                    // [K][G] dense stoichiometry per lane
-  int64_t o_mlogK, o_mlogKcoef, o_mh2o;
+  int64_t o_mlogK, o_mlogKcoef;
   int64_t o_mk, o_mmolvol, o_mEa, o_mthr, o_mlim, o_mpow, o_mtemkin;  // [K]
   int64_t o_mmsf;                    // [K] min scale factor (1 where unset)
   int64_t o_mpn;                     // int32 [K] rate prefactors of the mineral
@@ -116,8 +115,13 @@ struct pfx_kernel_params {
   unsigned int *queue;          // global cell cursor
   int32_t chunk;                // cells taken per fetch (at most)
   int32_t waves;                // wavefronts draining the queue: a fetch takes
-                                // a quarter of their fair share of what is
-                                // left, at most chunk (0 = always chunk)
+                                // a fifth of their fair share of what was
+                                // left at the last one, at most chunk (0 =
+                                // always chunk)
+  int32_t share;                // cells that each wavefront owns from the start
+                                // (the queue holds the rest)
+  int32_t block0;               // first workgroup of the launch that serves
+                                // this batch
   // cells whose unpivoted factorisation broke down: defer[0] their count,
   // defer[1..] their indices (written by the unpivoted reaction kernel,
   // worked through by the pivoting one); null where the kernel pivots

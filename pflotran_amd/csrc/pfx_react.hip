@@ -654,6 +654,7 @@ __device__ __forceinline__ void react_body(uint64_t praw) {
   constexpr bool kCanDefer = MODE == PFX_MODE_REACT && LUP == PFX_LU_DEFER;
   const bool from_list = MODE == PFX_MODE_REACT && LUP == PFX_LU_PIVOT && P0->defer != nullptr;
   const long long ncl = from_list ? (long long)P0->defer[0] : P0->ncells;
+  if (ncl == 0) return;  // nothing was deferred: the tables need not be staged
   const int lds_tab = (int)P0->L.lds_table_bytes;
 
   // stage the reaction tables into LDS (16-byte words)
@@ -678,8 +679,16 @@ __device__ __forceinline__ void react_body(uint64_t praw) {
   int r_opq = r;
   if (r == 0) SD(make_scr<XM>(sbase, M, G, K).C, M) = 0.0;
 
-  // wave-level work queue state (identical in all lanes of the wave)
-  long long q_next = 0, q_end = 0;
+  // wave-level work queue state (identical in all lanes of the wave): each
+  // wavefront owns a first share of the cells and fetches the rest.  q_seen
+  // is where the queue stood after its last fetch.
+  const long long q_own = from_list ? 0 : P0->share, q_base = q_own * P0->waves;
+  long long q_next = 0, q_end = 0, q_seen = q_base;
+  if (q_own > 0) {
+    const long long wave = (long long)((int)blockIdx.x - P0->block0) * (BLOCK / 64) + (threadIdx.x >> 6);
+    q_next = wave * q_own;
+    q_end = q_next + q_own < ncl ? q_next + q_own : ncl;
+  }
   bool exhausted = false;
 
 #ifdef PFX_SECTION_TIMERS
@@ -733,23 +742,23 @@ __device__ __forceinline__ void react_body(uint64_t praw) {
       while (nneed > 0) {
         long long avail = q_end - q_next;
         if (avail <= 0) {
+          if (q_base >= ncl) {  // the shares cover the batch
+            exhausted = true;
+            break;
+          }
           // guided sizes: near the end of the queue a fetch takes less, so
           // the last wavefronts do not hold long private runs of cells
           unsigned int base = 0, take_n = (unsigned int)P.chunk;
-          if (lane == 0) {
-            if (P.waves > 0) {
-              const long long left =
-                  ncl - (long long)__hip_atomic_load(P.queue, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-              const long long share = left / (4LL * P.waves);
-              const long long lo = 64 / G;
-              take_n = (unsigned int)(share < lo ? lo : (share < (long long)take_n ? share : (long long)take_n));
-            }
-            base = atomicAdd(P.queue, take_n);
+          if (P.waves > 0) {
+            const long long part = (ncl - q_seen) / (5LL * P.waves);
+            const long long lo = 64 / G;
+            take_n = (unsigned int)(part < lo ? lo : (part < (long long)take_n ? part : (long long)take_n));
           }
-          base = __shfl(base, 0);
-          take_n = __shfl(take_n, 0);
+          if (lane == 0) base = atomicAdd(P.queue, take_n);
+          base = __shfl(base, 0) + (unsigned int)q_base;
           q_next = base;
           q_end = (long long)base + take_n;
+          q_seen = q_end;
           if (q_end > ncl) q_end = ncl;
           if (q_next >= ncl) {
             exhausted = true;
