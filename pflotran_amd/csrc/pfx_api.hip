@@ -19,7 +19,7 @@ __global__ void pfx_react_kernel(const pfx_kernel_params P);
 template <int W, bool XM>
 __global__ void pfx_react_zones_kernel(const pfx_kernel_params *zone_params, const pfx_zone_launch Z,
                                        uint64_t *finish);
-extern "C" int pfx_scr_doubles(int M, int G, int K, int xm);
+extern "C" int pfx_scr_bytes(int threads, int N, int M, int G, int K, int xm, int mode);
 
 struct pfx_tables {
   pfx_dev_layout L;
@@ -231,6 +231,8 @@ const void *kernel_ptr(int G, int mode, int v, int lup = PFX_LU_DEFER, bool xm =
          : lup == PFX_LU_ONDEMAND ? kernel_for<PFX_MODE_REACT, 1, PFX_LU_ONDEMAND, true>(G)
                                   : kernel_for<PFX_MODE_REACT, 1, PFX_LU_DEFER, true>(G);
   if (xm && mode == PFX_MODE_EVAL) return kernel_for<PFX_MODE_EVAL, 1, PFX_LU_PIVOT, true>(G);
+  if (mode == PFX_MODE_GI)
+    return xm ? kernel_for<PFX_MODE_GI, 1, PFX_LU_PIVOT, true>(G) : kernel_for<PFX_MODE_GI, 1, PFX_LU_PIVOT>(G);
   switch (mode) {
     case PFX_MODE_REACT:
       if (lup == PFX_LU_PIVOT) return kernel_for<PFX_MODE_REACT, 1, PFX_LU_PIVOT>(G);
@@ -267,7 +269,7 @@ int resident(int occ, int64_t lds) {
   return (int)std::max<int64_t>(1, std::min<int64_t>(occ, 128 / pieces));
 }
 
-// Work distribution of a launch of `blocks` workgroups: the cells that each
+// Work distribution of a launch of `waves` wavefronts: the cells that each
 // wavefront owns from the start, and the most it takes per fetch of the rest.
 // Every fetch is an atomic on one address, ~39 ns each one after the other
 // whichever XCD they come from: 63k cells fetched by fours were 0.62 of the
@@ -278,10 +280,10 @@ int resident(int occ, int64_t lds) {
 // workgroup resident from the start: the grid is never larger (resident()).
 // Measured: 50k cells of N = 15 2.46 -> 2.09 ms, 63k-cell evaluation 0.84 ->
 // 0.24 ms, speciation of 200k cells 2.40 -> 2.06 ms.
-void distribute(pfx_kernel_params &P, int G, int mode, int64_t blocks) {
-  const int64_t waves = blocks * (BLOCK / 64), lo = 64 / G;
+void distribute(pfx_kernel_params &P, int G, int mode, int64_t waves) {
+  const int64_t lo = 64 / G;
   const int64_t fair = (P.ncells + waves - 1) / waves;
-  const bool even = mode == PFX_MODE_EVAL || mode == PFX_MODE_AUX;
+  const bool even = mode == PFX_MODE_EVAL || mode == PFX_MODE_GI || mode == PFX_MODE_AUX;
   int64_t share = even ? fair : fair / 2;
   share = even ? (share + lo - 1) / lo * lo : share / lo * lo;
   P.share = (int32_t)std::max<int64_t>(share, lo);
@@ -299,24 +301,34 @@ int launch(pfx_tables *t, pfx_kernel_params &P, int mode, hipStream_t stream, do
            unsigned int *queue = nullptr) {
   if (!queue) queue = t->d_queue;
   const int G = t->L.G;
-  const int groups = BLOCK / G;
-  const int64_t lds = t->L.lds_table_bytes + (int64_t)groups * pfx_scr_doubles(t->L.M, G, t->L.K, tables_xm(t)) * 8;
+  int threads = BLOCK;
+  const bool xm = tables_xm(t);
+  auto lds_of = [&](int th) { return t->L.lds_table_bytes + pfx_scr_bytes(th, t->L.N, t->L.M, G, t->L.K, xm, mode); };
+  // an evaluation on a grid stages its blocks in LDS too: where that is more
+  // than a compute unit has, the workgroup is halved (every network accepted
+  // by pfx_tables_create then fits).  Larger workgroups, which would share a
+  // copy of the tables between 12 wavefronts, need the registers capped for a
+  // third wavefront per SIMD and lose more by the spills (11.2 against 10.5 ms
+  // at 128^3 x 15).
+  if (mode == PFX_MODE_GI && lds_of(threads) > kMaxLds) threads = BLOCK / 2;
+  const int64_t lds = lds_of(threads);
+  const int groups = threads / G;
   if (lds > kMaxLds) return PFX_E_UNSUP;
   int occ = 0;
   const bool deferring = mode == PFX_MODE_REACT && P.defer != nullptr;
   const int lup = mode != PFX_MODE_REACT ? PFX_LU_PIVOT : (deferring ? PFX_LU_DEFER : PFX_LU_ONDEMAND);
-  const void *fn = kernel_ptr(G, mode, t->variant[mode & 3], lup, tables_xm(t));
+  const void *fn = kernel_ptr(G, mode, mode < 4 ? t->variant[mode] : 0, lup, tables_xm(t));
   const void *fn_piv = deferring ? kernel_ptr(G, mode, 0, PFX_LU_PIVOT, tables_xm(t)) : nullptr;
   if (lds > 64 * 1024) {
     HIPCHK(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
     if (fn_piv) HIPCHK(hipFuncSetAttribute(fn_piv, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
   }
-  HIPCHK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, fn, BLOCK, (size_t)lds));
+  HIPCHK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, fn, threads, (size_t)lds));
   occ = resident(occ, lds);
   int64_t need_blocks = (P.ncells + groups - 1) / groups;
   int64_t blocks = std::min<int64_t>(need_blocks, (int64_t)t->num_cu * occ);
   if (blocks < 1) blocks = 1;
-  distribute(P, G, mode, blocks);
+  distribute(P, G, mode, blocks * (threads / 64));
   P.queue = queue;
   P.fallback_count = queue + 1;
   // the pivoting launch: its own cursor, one cell per fetch, one workgroup
@@ -333,12 +345,12 @@ int launch(pfx_tables *t, pfx_kernel_params &P, int mode, hipStream_t stream, do
   void *args2[] = {(void *)&P2};
   if (!ms) {
     // stream-ordered: no events, no wait (the launches may be graph-captured)
-    HIPCHK(hipLaunchKernel(fn, dim3((unsigned)blocks), dim3(BLOCK), args, (size_t)lds, stream));
+    HIPCHK(hipLaunchKernel(fn, dim3((unsigned)blocks), dim3((unsigned)threads), args, (size_t)lds, stream));
     if (fn_piv) HIPCHK(hipLaunchKernel(fn_piv, dim3((unsigned)blocks2), dim3(BLOCK), args2, (size_t)lds, stream));
     return 0;
   }
   HIPCHK(hipEventRecord(t->ev0, stream));
-  HIPCHK(hipLaunchKernel(fn, dim3((unsigned)blocks), dim3(BLOCK), args, (size_t)lds, stream));
+  HIPCHK(hipLaunchKernel(fn, dim3((unsigned)blocks), dim3((unsigned)threads), args, (size_t)lds, stream));
   if (fn_piv) HIPCHK(hipLaunchKernel(fn_piv, dim3((unsigned)blocks2), dim3(BLOCK), args2, (size_t)lds, stream));
   HIPCHK(hipEventRecord(t->ev1, stream));
   HIPCHK(hipEventSynchronize(t->ev1));
@@ -483,7 +495,7 @@ int ensure_side(pfx_tables *t) {
 
 int zone_lds(const pfx_tables *t) {
   const int G = t->L.G;
-  return (int)(t->L.lds_table_bytes + (int64_t)(BLOCK / G) * pfx_scr_doubles(t->L.M, G, t->L.K, tables_xm(t)) * 8);
+  return (int)(t->L.lds_table_bytes + pfx_scr_bytes(BLOCK, t->L.N, t->L.M, G, t->L.K, tables_xm(t), PFX_MODE_REACT));
 }
 
 int zones_prepare(int32_t nzones, pfx_tables *const *tables, pfx_cells *cells, const pfx_react_opts *o,
@@ -548,7 +560,7 @@ int zones_prepare(int32_t nzones, pfx_tables *const *tables, pfx_cells *cells, c
   for (int z = 0; z < nzones; z++) {
     zs.Z.block_start[z] = acc;
     acc += blocks[z];
-    distribute(zs.P[z], zs.Z.G[z], PFX_MODE_REACT, blocks[z]);
+    distribute(zs.P[z], zs.Z.G[z], PFX_MODE_REACT, blocks[z] * (BLOCK / 64));
     zs.P[z].block0 = zs.Z.block_start[z];
   }
   zs.Z.block_start[nzones] = acc;
@@ -650,41 +662,30 @@ int use_scratch(pfx_tables *t, pfx_kernel_params &P, int64_t n) {
 
 }  // namespace
 
-// per-cell scratch of the global-implicit assembly: non-flux residual [N],
-// non-flux Jacobian [N*N], totals [N], dT/dm [N*N]
-int pfx_internal::gi_scratch(pfx_tables *t, int64_t ncells, double **rnf, double **jnf, double **tot,
-                             double **dtot) {
-  const int64_t N = t->L.N, per = 2 * N + 2 * N * N;
-  if (ncells > t->gi_cells) {
-    HIPCHK(hipSetDevice(t->device));
-    if (t->d_gi) HIPCHK(hipFree(t->d_gi));
-    t->d_gi = nullptr;
-    t->gi_cells = 0;
-    HIPCHK(hipMalloc(&t->d_gi, (size_t)(ncells * per) * sizeof(double)));
-    t->gi_cells = ncells;
-  }
-  *rnf = t->d_gi;
-  *jnf = *rnf + ncells * N;
-  *tot = *jnf + ncells * N * N;
-  *dtot = *tot + ncells * N;
-  return 0;
-}
-
+// one evaluation of every cell of a grid, straight into the block matrix;
+// *tot: the totals (the tables' scratch, grown on demand)
 int pfx_internal::gi_evaluate_cells(pfx_tables *t, pfx_cells *cells, const pfx_react_opts *o, int col_scale,
-                                    double *rnf, double *jnf, double *tot, double *dtot) {
+                                    const pfx_gi_faces &gi, double *residual, double **tot) {
   int rc = check_cells(t, cells, o);
   if (rc) return rc;
   if (cells->ncells == 0) return 0;
   HIPCHK(hipSetDevice(t->device));
+  if (cells->ncells > t->gi_cells) {
+    if (t->d_gi) HIPCHK(hipFree(t->d_gi));
+    t->d_gi = nullptr;
+    t->gi_cells = 0;
+    HIPCHK(hipMalloc(&t->d_gi, (size_t)(cells->ncells * t->L.N) * sizeof(double)));
+    t->gi_cells = cells->ncells;
+  }
+  *tot = t->d_gi;
   pfx_kernel_params P;
   fill_params(t, cells, o, P);
-  P.res_out = rnf;
-  P.jac_out = jnf;
-  P.tot_eval_out = tot;
-  P.dtot_out = dtot;
+  P.res_out = residual;
+  P.gi = gi;
+  P.tot_eval_out = *tot;
   P.col_scale = col_scale ? 1 : 0;
   double ms = 0.0;
-  return launch(t, P, PFX_MODE_EVAL, (hipStream_t)o->stream, o->stream_ordered ? nullptr : &ms);
+  return launch(t, P, PFX_MODE_GI, (hipStream_t)o->stream, o->stream_ordered ? nullptr : &ms);
 }
 
 int pfx_internal::timed_launch_begin(pfx_tables *t, hipStream_t s) {
@@ -1006,7 +1007,7 @@ extern "C" int pfx_tables_create(const pfx_reaction_desc *d, pfx_tables **out) {
   L.max_dlnC = d->max_dlnC;
   L.max_rel_change_tol = d->max_relative_change_tolerance;
   L.max_residual_tol = d->max_residual_tolerance;
-  const int64_t lds = L.lds_table_bytes + (int64_t)(BLOCK / G) * pfx_scr_doubles(M, G, K, (L.mnrl_flags & 48) != 0) * 8;
+  const int64_t lds = L.lds_table_bytes + pfx_scr_bytes(BLOCK, N, M, G, K, (L.mnrl_flags & 48) != 0, PFX_MODE_REACT);
   if (lds > kMaxLds) return PFX_E_UNSUP;
 
   pfx_tables *t = new pfx_tables();

@@ -69,13 +69,24 @@ struct pfx_dev_layout {
   int64_t lds_table_bytes;           // prefix of the blob staged into LDS
 };
 
-enum { PFX_MODE_REACT = 0, PFX_MODE_EVAL = 1, PFX_MODE_EQUIL = 2, PFX_MODE_AUX = 3 };
+enum { PFX_MODE_REACT = 0, PFX_MODE_EVAL = 1, PFX_MODE_EQUIL = 2, PFX_MODE_AUX = 3, PFX_MODE_GI = 4 };
 
 // block split of a zoned launch (pfx_react_zones)
 struct pfx_zone_launch {
   int32_t nzones;
   int32_t block_start[PFX_MAX_ZONES + 1];
   int32_t G[PFX_MAX_ZONES];
+};
+
+// A structured grid's faces and the block matrix of its 7-point pattern
+// (pfx_gi_structure's rows), column-major N x N blocks.
+struct pfx_gi_faces {
+  int32_t nx, ny, nz, reserved;
+  double area[3];
+  const double *q[3], *dd[3];
+  const double *bc_q[2], *bc_dd[2], *bc_total[2];
+  const int32_t *row_ptr;
+  double *vals;
 };
 
 struct pfx_kernel_params {
@@ -100,9 +111,10 @@ struct pfx_kernel_params {
   int32_t reserved0;
   unsigned int *fallback_count; // cells restarted by the fallback
   double *res_out, *jac_out;    // residual/Jacobian outputs
-  double *dtot_out;             // EVAL: dT/dm blocks [ncells][N][N] column-major (kg/L), may be NULL
-  double *tot_eval_out;         // EVAL: totals at the free ions [ncells][N] (mol/L), may be NULL
-  int32_t col_scale;            // EVAL: scale Jacobian and dT/dm columns by m (log unknowns)
+  // GI: the grid whose block rows the cells' Jacobians go to
+  pfx_gi_faces gi;
+  double *tot_eval_out;         // GI: totals at the free ions [ncells][N] (mol/L)
+  int32_t col_scale;            // GI: scale the blocks' columns by m (log unknowns)
   // constraint speciation
   const double *constraint_conc;   // [ncells*N]
   int32_t ctype[PFX_MAX_PRIMARY];  // PFX_CONSTRAINT_* per component
@@ -140,15 +152,33 @@ struct pfx_kernel_params {
 #define PFX_LU_PIVOT 1
 #define PFX_LU_ONDEMAND 2
 
+#ifdef __HIPCC__
+// TFluxCoef (transport.F90:756-819), upwinding, one liquid phase: L/s
+__device__ __forceinline__ void pfx_flux_coef(double area, double q, double dd, double &Tup, double &Tdn) {
+  double cup, cdn;
+  if (q > 0.0) {
+    cup = dd + q;
+    cdn = -dd;
+  } else {
+    cup = dd;
+    cdn = -dd + q;
+  }
+  Tup = cup * area * 1000.0;
+  Tdn = cdn * area * 1000.0;
+}
+#endif
+
 // Sizes of a network held by an opaque pfx_tables (defined in pfx_api.hip)
 // for the other translation units of the library.
 struct pfx_bsr;  // include/pfx_gi_solver.h
 namespace pfx_internal {
 void table_sizes(const pfx_tables *t, int *N, int *M, int *K, int *R);
 void table_max_dlnC(const pfx_tables *t, double *max_dlnC);
-int gi_scratch(pfx_tables *t, int64_t ncells, double **rnf, double **jnf, double **tot, double **dtot);
-int gi_evaluate_cells(pfx_tables *t, pfx_cells *cells, const pfx_react_opts *o, int col_scale, double *rnf,
-                      double *jnf, double *tot, double *dtot);
+// evaluate every cell at its free ions: residual without fluxes into
+// residual, totals into *tot (the tables' scratch), every block of the matrix
+// into gi.vals
+int gi_evaluate_cells(pfx_tables *t, pfx_cells *cells, const pfx_react_opts *o, int col_scale,
+                      const pfx_gi_faces &gi, double *residual, double **tot);
 // shape of a pfx_bsr handle (defined in pfx_krylov.hip)
 const int32_t *bsr_row_ptr(const ::pfx_bsr *h);
 int64_t bsr_rows(const ::pfx_bsr *h);

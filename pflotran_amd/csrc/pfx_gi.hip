@@ -2,16 +2,16 @@
 // pfx_gi_structure / pfx_gi_residual_jacobian).
 //
 // Two launches per evaluation:
-//  1. the persistent per-cell kernel in EVAL mode writes, per cell, the
-//     non-flux residual (accumulation/dt - old accumulation/dt + reaction),
-//     the non-flux Jacobian block, the aqueous totals and dT/dm (column-
-//     major blocks, columns already scaled by m for log unknowns);
-//  2. k_gi_assemble, one wavefront per block row, adds the upwind flux
-//     terms of the row's faces (TFluxCoef, TFlux, TFluxDerivative) and
-//     writes the row's residual and its 7 (or fewer) BSR blocks.  With a
-//     species-independent dispersion every flux block is a scalar times the
-//     neighbour's dT/dm block, so the row is a handful of scaled block copies:
-//     the kernel is HBM-bound (≈7 * N^2 * 8 B written per cell).
+//  1. the per-cell kernel in GI mode (pfx_react.hip) writes, per cell, the
+//     residual without fluxes and the totals, and every block that the cell's
+//     Jacobian and dT/dm give: its own row's diagonal block and, with a
+//     species-independent dispersion a scalar times dT/dm each, the blocks of
+//     its column in its neighbours' rows.  No block is written to memory only
+//     to be read again: 128^3 x 15 wrote 7.5 GB of them and read 8.4 GB back
+//     in a second kernel over the block rows, 15.1 ms an evaluation, 10.5 now
+//     (26.2 GB of matrix);
+//  2. k_gi_flux_residual adds the upwind fluxes of the totals (TFluxCoef,
+//     TFlux) to the residual.
 #include <hip/hip_runtime.h>
 
 #include <cstdio>
@@ -33,153 +33,45 @@ namespace {
     }                                                                         \
   } while (0)
 
-struct gi_params {
-  int32_t nx, ny, nz, N;
-  double area[3];
-  const double *q[3], *dd[3];
-  const double *bc_q[2], *bc_dd[2], *bc_total[2];
-  const int32_t *row_ptr;
-  const double *rnf, *jnf, *tot, *dtot;
-  double *res, *vals;
-};
-
-// TFluxCoef (transport.F90:756-819), upwinding, one liquid phase: L/s
-__device__ __forceinline__ void flux_coef(double area, double q, double dd, double &Tup, double &Tdn) {
-  double cup, cdn;
-  if (q > 0.0) {
-    cup = dd + q;
-    cdn = -dd;
-  } else {
-    cup = dd;
-    cdn = -dd + q;
-  }
-  Tup = cup * area * 1000.0;
-  Tdn = cdn * area * 1000.0;
-}
-
-__global__ __launch_bounds__(256) void k_gi_assemble(const gi_params P) {
-  const int lane = threadIdx.x & 63;
-  const int64_t nx = P.nx, ny = P.ny, nz = P.nz, n = nx * ny * nz;
-  const int64_t c = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
-  if (c >= n) return;  // whole wavefront
-  const int N = P.N, NN = N * N;
-  const int64_t i = c % nx, j = (c / nx) % ny, k = c / (nx * ny);
-  const bool comp = lane < N;
-  const double tc = comp ? P.tot[c * N + lane] : 0.0;
-  double res = comp ? P.rnf[c * N + lane] : 0.0;
-  double s_diag = 0.0;  // scalar of dT_c in the diagonal block
-
-  // neighbours in column order: z-, y-, x-, (self), x+, y+, z+
-  int64_t nb[6];
-  double tnb[6];
-  bool has[6];
-  const int64_t stride[3] = {1, nx, nx * ny};
-  const int64_t idx[3] = {i, j, k};
-  const int64_t ext[3] = {nx, ny, nz};
+// The faces' part of the residual: res holds the cells' own (mol/s) on entry.
+// One thread per cell and component; HBM-bound, the totals and the residual
+// once each.
+__global__ __launch_bounds__(256) void k_gi_flux_residual(const pfx_gi_faces P, int N, const double *__restrict__ tot,
+                                                          double *__restrict__ res_out) {
+  const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  const int nx = P.nx, ny = P.ny, nz = P.nz;
+  if (e >= (int64_t)nx * ny * nz * N) return;
+  const int c = (int)(e / N), comp = (int)(e % N);
+  const int i = c % nx, jk = c / nx, j = jk % ny, k = jk / ny;
+  const double tc = tot[e];
+  double res = res_out[e];
 #pragma unroll
   for (int d = 0; d < 3; d++) {
+    const int at = d == 0 ? i : (d == 1 ? j : k), ext = d == 0 ? nx : (d == 1 ? ny : nz);
+    const int64_t stride = d == 0 ? 1 : (d == 1 ? nx : (int64_t)nx * ny);
     const int64_t ex = nx - (d == 0), ey = ny - (d == 1);
-    // lower face: (c - stride) is up, c is dn
-    const int lo = 2 - d;  // slot: z- = 0, y- = 1, x- = 2
-    has[lo] = idx[d] > 0;
-    if (has[lo]) {
-      const int64_t up = c - stride[d];
-      const int64_t ui = up % nx, uj = (up / nx) % ny, uk = up / (nx * ny);
-      const int64_t f = ui + ex * (uj + ey * uk);
-      double Tup, Tdn;
-      flux_coef(P.area[d], P.q[d][f], P.dd[d][f], Tup, Tdn);
-      const double tn = comp ? P.tot[up * N + lane] : 0.0;
-      res -= Tup * tn + Tdn * tc;
-      s_diag -= Tdn;
-      nb[lo] = up;
-      tnb[lo] = -Tup;
+    const int64_t f = i + ex * (j + ey * k);                   // the face above, c upstream
+    const int64_t below = f - (d == 0 ? 1 : (d == 1 ? ex : ex * ey));
+    double Tup, Tdn;
+    if (at > 0) {  // lower face: (c - stride) is up, c is dn
+      pfx_flux_coef(P.area[d], P.q[d][below], P.dd[d][below], Tup, Tdn);
+      res -= Tup * tot[e - stride * N] + Tdn * tc;
     }
-    // upper face: c is up, (c + stride) is dn
-    const int hi = 3 + d;  // x+ = 3, y+ = 4, z+ = 5
-    has[hi] = idx[d] < ext[d] - 1;
-    if (has[hi]) {
-      const int64_t dn = c + stride[d];
-      const int64_t f = i + ex * (j + ey * k);
-      double Tup, Tdn;
-      flux_coef(P.area[d], P.q[d][f], P.dd[d][f], Tup, Tdn);
-      const double tn = comp ? P.tot[dn * N + lane] : 0.0;
-      res += Tup * tc + Tdn * tn;
-      s_diag += Tup;
-      nb[hi] = dn;
-      tnb[hi] = Tdn;
+    if (at < ext - 1) {  // upper face: c is up, (c + stride) is dn
+      pfx_flux_coef(P.area[d], P.q[d][f], P.dd[d][f], Tup, Tdn);
+      res += Tup * tc + Tdn * tot[e + stride * N];
     }
   }
   // boundary connections on the x faces (boundary = up, cell = dn)
 #pragma unroll
   for (int side = 0; side < 2; side++) {
     if (P.bc_q[side] && i == (side == 0 ? 0 : nx - 1)) {
-      const int64_t f = j + ny * k;
       double Tup, Tdn;
-      flux_coef(P.area[0], P.bc_q[side][f], P.bc_dd[side][f], Tup, Tdn);
-      const double tb = P.bc_total[side] ? (comp ? P.bc_total[side][lane] : 0.0) : tc;
-      res -= Tup * tb + Tdn * tc;
-      s_diag -= Tdn;
+      pfx_flux_coef(P.area[0], P.bc_q[side][jk], P.bc_dd[side][jk], Tup, Tdn);
+      res -= Tup * (P.bc_total[side] ? P.bc_total[side][comp] : tc) + Tdn * tc;
     }
   }
-  if (comp) P.res[c * N + lane] = res;
-
-  // blocks of the row, in column order.  All source words are loaded
-  // before the first store (up to 8 x CH loads in flight per lane); the
-  // row's blocks are written once and not read back here, so they bypass
-  // the caches that hold the neighbours' dT/dm blocks.
-  int64_t b = P.row_ptr[c];
-  const int order[7] = {0, 1, 2, -1, 3, 4, 5};
-  constexpr int CH = 4;  // 64-wide chunks of an N x N block, N <= 16
-  if (NN <= CH * 64) {
-    double v[7][CH], jn[CH];
-#pragma unroll
-    for (int s = 0; s < 7; s++) {
-      const int o = order[s];
-      const bool on = o < 0 || has[o];
-      const double *src = P.dtot + (o < 0 ? c : (on ? nb[o] : c)) * NN;
-#pragma unroll
-      for (int q = 0; q < CH; q++) {
-        const int e = lane + 64 * q;
-        v[s][q] = (on && e < NN) ? src[e] : 0.0;
-      }
-    }
-#pragma unroll
-    for (int q = 0; q < CH; q++) {
-      const int e = lane + 64 * q;
-      jn[q] = e < NN ? __builtin_nontemporal_load(P.jnf + c * NN + e) : 0.0;
-    }
-#pragma unroll
-    for (int s = 0; s < 7; s++) {
-      const int o = order[s];
-      if (o < 0 || has[o]) {
-        double *out = P.vals + b * NN;
-#pragma unroll
-        for (int q = 0; q < CH; q++) {
-          const int e = lane + 64 * q;
-          if (e < NN) __builtin_nontemporal_store(o < 0 ? jn[q] + s_diag * v[s][q] : tnb[o] * v[s][q], out + e);
-        }
-        b++;
-      }
-    }
-    return;
-  }
-#pragma unroll
-  for (int s = 0; s < 7; s++) {
-    const int o = order[s];
-    if (o < 0) {
-      const double *Jn = P.jnf + c * NN;
-      const double *Dc = P.dtot + c * NN;
-      double *out = P.vals + b * NN;
-      for (int e = lane; e < NN; e += 64) out[e] = Jn[e] + s_diag * Dc[e];
-      b++;
-    } else if (has[o]) {
-      const double *Dn = P.dtot + nb[o] * NN;
-      double *out = P.vals + b * NN;
-      const double t = tnb[o];
-      for (int e = lane; e < NN; e += 64) out[e] = t * Dn[e];
-      b++;
-    }
-  }
+  res_out[e] = res;
 }
 
 struct disp_params {
@@ -303,7 +195,7 @@ __global__ void k_os_matrix(const os_params P) {
       const int64_t up = c - stride;
       const int64_t f = (up % nx) + ex * (((up / nx) % ny) + ey * (up / (nx * ny)));
       double Tup, Tdn;
-      flux_coef(P.area[d], P.q[d][f], P.dd[d][f], Tup, Tdn);
+      pfx_flux_coef(P.area[d], P.q[d][f], P.dd[d][f], Tup, Tdn);
       diag -= Tdn;
       off[lo] = -Tup;
     }
@@ -312,7 +204,7 @@ __global__ void k_os_matrix(const os_params P) {
     if (has[hi]) {  // c is the upstream cell of its upper face
       const int64_t f = i + ex * (j + ey * k);
       double Tup, Tdn;
-      flux_coef(P.area[d], P.q[d][f], P.dd[d][f], Tup, Tdn);
+      pfx_flux_coef(P.area[d], P.q[d][f], P.dd[d][f], Tup, Tdn);
       diag += Tup;
       off[hi] = Tdn;
     }
@@ -325,7 +217,7 @@ __global__ void k_os_matrix(const os_params P) {
     if (P.bc_q[side] && i == (side == 0 ? 0 : nx - 1)) {
       const int64_t f = j + ny * k;
       double Tup, Tdn;
-      flux_coef(P.area[0], P.bc_q[side][f], P.bc_dd[side][f], Tup, Tdn);
+      pfx_flux_coef(P.area[0], P.bc_q[side][f], P.bc_dd[side][f], Tup, Tdn);
       diag -= Tdn;
       if (!P.bc_total[side]) diag -= Tup;
     }
@@ -355,7 +247,7 @@ __global__ void k_os_rhs_all(const os_params P) {
     if (P.bc_q[side] && P.bc_total[side] && i == (side == 0 ? 0 : nx - 1)) {
       const int64_t f = j + ny * k;
       double Tup, Tdn;
-      flux_coef(P.area[0], P.bc_q[side][f], P.bc_dd[side][f], Tup, Tdn);
+      pfx_flux_coef(P.area[0], P.bc_q[side][f], P.bc_dd[side][f], Tup, Tdn);
       r += Tup * P.bc_total[side][comp];
     }
   }
@@ -397,17 +289,11 @@ extern "C" int pfx_gi_residual_jacobian(pfx_tables *t, pfx_cells *cells, const p
   if (cells->ncells != n) return PFX_E_ARG;
   int N, M, K, R;
   pfx_internal::table_sizes(t, &N, &M, &K, &R);
-  double *rnf, *jnf, *tot, *dtot;
-  int rc = pfx_internal::gi_scratch(t, n, &rnf, &jnf, &tot, &dtot);
-  if (rc) return rc;
-  rc = pfx_internal::gi_evaluate_cells(t, cells, o, g->log_formulation, rnf, jnf, tot, dtot);
-  if (rc) return rc;
-  gi_params P;
+  pfx_gi_faces P;
   memset(&P, 0, sizeof(P));
   P.nx = g->nx;
   P.ny = g->ny;
   P.nz = g->nz;
-  P.N = N;
   for (int d = 0; d < 3; d++) {
     P.area[d] = g->area[d];
     P.q[d] = g->q[d];
@@ -419,15 +305,13 @@ extern "C" int pfx_gi_residual_jacobian(pfx_tables *t, pfx_cells *cells, const p
     P.bc_total[s] = g->bc_total[s];
   }
   P.row_ptr = row_ptr;
-  P.rnf = rnf;
-  P.jnf = jnf;
-  P.tot = tot;
-  P.dtot = dtot;
-  P.res = residual;
   P.vals = bsr_values;
+  double *tot = nullptr;
+  int rc = pfx_internal::gi_evaluate_cells(t, cells, o, g->log_formulation, P, residual, &tot);
+  if (rc) return rc;
   hipStream_t s = (hipStream_t)o->stream;
   if ((rc = pfx_internal::timed_launch_begin(t, s))) return rc;
-  hipLaunchKernelGGL(k_gi_assemble, dim3((unsigned)((n + 3) / 4)), dim3(256), 0, s, P);
+  hipLaunchKernelGGL(k_gi_flux_residual, dim3((unsigned)((n * N + 255) / 256)), dim3(256), 0, s, P, N, tot, residual);
   GCHK(hipGetLastError());
   return pfx_internal::timed_launch_end(t, s, 1);
 }

@@ -413,14 +413,20 @@ __device__ __forceinline__ double logk_5term_ptr(const double *cf, double tk, do
 //   ionx[PFX_MAX_IONX_RXN] the exchange state, fx[G] the fixed accumulation
 //   of each row.  The last three hold cell state that lives across Newton
 //   passes: in LDS it does not occupy registers for the whole loop.
+//   On a grid (gi): gc[8] the multiples of the cell's dT/dm in its six
+//   neighbours' rows and ([6]) in its own, gp[8] (int32) those blocks' places.
 struct Scr {
-  int C, gsec, lnK, la, mv, im, xb, mlnK, mkeff, marea, mvf, mrate, cs, ionx, fx;
+  int C, gsec, lnK, la, mv, im, xb, mlnK, mkeff, marea, mvf, mrate, cs, ionx, fx, gc, gp;
 };
 
-__host__ __device__ inline int scr_doubles(int M, int G, int K, bool xm) {
-  int n = (M + 1) + 2 * M + 5 * G + 5 * K + (xm ? 6 : 4) + PFX_MAX_IONX_RXN;
+__host__ __device__ inline int scr_doubles(int M, int G, int K, bool xm, bool gi) {
+  int n = (M + 1) + 2 * M + 5 * G + 5 * K + (xm ? 6 : 4) + PFX_MAX_IONX_RXN + (gi ? 12 : 0);
   return (n + 1) & ~1;
 }
+
+// one column-major block per wavefront, through which the groups of up to 16
+// lanes write their blocks in runs of 64 consecutive numbers
+__host__ __device__ inline int gi_stage_doubles(int N, int G) { return G <= 16 ? (N * N + 1) & ~1 : 0; }
 
 // The fields whose size is fixed by the group size come first, at offsets
 // known at compile time: their LDS accesses take the offset as an
@@ -445,7 +451,9 @@ __device__ __forceinline__ Scr make_scr(int base, int M, int G, int K) {
   s.mkeff = p; p += K * 8;
   s.marea = p; p += K * 8;
   s.mvf = p; p += K * 8;
-  s.mrate = p;
+  s.mrate = p; p += K * 8;
+  s.gc = p; p += 64;
+  s.gp = p;
   return s;
 }
 
@@ -468,6 +476,9 @@ __device__ __forceinline__ double pow_ratio(double x, double z) {
 //   PFX_MODE_EVAL   residual + Jacobian at given free ions (reaction.F90:3419-3441)
 //   PFX_MODE_EQUIL  constraint speciation, ReactionEquilibrateConstraint
 //                   (reaction.F90:1308-2046), TOTAL/FREE/LOG/PH rows
+//   PFX_MODE_GI     the same on a grid: the Jacobian and dT/dm go straight to
+//                   the block matrix (RTJacobian), the totals out for the
+//                   flux residual
 //   PFX_MODE_AUX    aux-var refresh, RTUpdateAuxVars (reactive_transport.F90:3790-3846)
 //
 // Phases of a cell in REACT: 0 = RTotal at the previous state, 1 = activity
@@ -640,6 +651,115 @@ __device__ __forceinline__ void mineral_fd_jacobian(KP Pp, const Scr &S, int r, 
   wave_sync();
 }
 
+// The faces of grid cell c, one lane each (z-, y-, x-, x+, y+, z+ in lanes 0..5
+// of the group, the x boundary faces in lanes 6 and 7): the multiple of the
+// cell's dT/dm that the face puts into the neighbour's row, and the place of that
+// block; their sum on the cell's own row in gc[6], that block's place in gp[6].
+// A face that is not there has place -1.
+template <int G>
+__device__ __forceinline__ void gi_load_faces(KP Pp, const Scr &S, int c, int r, int lane) {
+  const int nx = Pp->gi.nx, ny = Pp->gi.ny, nz = Pp->gi.nz;
+  const int i = c % nx, jk = c / nx, j = jk % ny, k = jk / ny;
+  double own = 0.0, coef = 0.0;
+  int place = -1;
+  if (r < 6) {
+    const bool lower = r < 3;
+    const int d = lower ? 2 - r : r - 3;
+    const int at = d == 0 ? i : (d == 1 ? j : k), ext = d == 0 ? nx : (d == 1 ? ny : nz);
+    if (lower ? at > 0 : at < ext - 1) {
+      const int stride = d == 0 ? 1 : (d == 1 ? nx : nx * ny);
+      // the face's upstream cell, and its number among the faces of its direction
+      const int ui = i - (lower && d == 0), uj = j - (lower && d == 1), uk = k - (lower && d == 2);
+      const long long f = ui + (long long)(nx - (d == 0)) * (uj + (long long)(ny - (d == 1)) * uk);
+      double Tup, Tdn;
+      pfx_flux_coef(Pp->gi.area[d], Pp->gi.q[d][f], Pp->gi.dd[d][f], Tup, Tdn);
+      own = lower ? -Tdn : Tup;    // downstream of a lower face, upstream of an upper one
+      coef = lower ? Tdn : -Tup;   // the same face in the neighbour's row
+      // the neighbour's blocks before this cell's column
+      const int s = lower ? -1 : 1;
+      const int a = i + (d == 0 ? s : 0), b = j + (d == 1 ? s : 0), e = k + (d == 2 ? s : 0);
+      const int opp = 5 - r;       // this cell as seen from there
+      int before = opp > 2 ? 1 : 0;
+      before += (opp > 0 && e > 0) + (opp > 1 && b > 0) + (opp > 2 && a > 0);
+      before += (opp > 3 && a < nx - 1) + (opp > 4 && b < ny - 1);
+      place = Pp->gi.row_ptr[c + s * stride] + before;
+    }
+  } else if (r < 8) {
+    const int side = r - 6;
+    const double *bq = Pp->gi.bc_q[side];
+    if (bq && i == (side == 0 ? 0 : nx - 1)) {
+      double Tup, Tdn;
+      pfx_flux_coef(Pp->gi.area[0], bq[jk], Pp->gi.bc_dd[side][jk], Tup, Tdn);
+      own = -Tdn;
+    }
+  }
+  const double diag = gsum<G>(own, lane);
+  if (r == 6) {
+    coef = diag;
+    place = Pp->gi.row_ptr[c] + (k > 0) + (j > 0) + (i > 0);
+  }
+  if (r < 7) {
+    SD(S.gc, r) = coef;
+    ((int32_t *)(smem + S.gp))[r] = place;
+  }
+}
+
+// Blocks s0 .. s1-1 (gi_load_faces) of every active group's cell: gc[s] times
+// the block whose row r is col[], or the block itself for the cell's own (6).
+// Bound by the writes, N^2 doubles a block.  A group of up to 16 lanes stages
+// its block in LDS and the whole wavefront writes it, 512 consecutive bytes an
+// instruction; 32 lanes write their columns directly (136 bytes or more each).
+template <int G, bool XM>
+__device__ __forceinline__ void gi_store_blocks(KP Pp, const double (&col)[G], int r, bool active, int stage, int s0,
+                                                int s1) {
+  const int N = Pp->L.N, NN = N * N;
+  const int lane = threadIdx.x & 63;
+  const int slice = scr_doubles(Pp->L.M, G, Pp->L.K, XM, true) * 8;
+  const int wave0 = (int)Pp->L.lds_table_bytes + (int)(threadIdx.x >> 6) * (64 / G) * slice;
+  double *vals = Pp->gi.vals;
+  if constexpr (G <= 16) {
+    constexpr int CH = G == 16 ? 4 : 1;  // 64-wide runs of an N x N block
+    const unsigned long long on = __ballot(active && r == 0);
+#pragma unroll 1
+    for (int g = 0; g < 64 / G; g++) {
+      if (!((on >> (g * G)) & 1ull)) continue;
+      wave_sync();
+      if (lane / G == g && r < N) {
+#pragma unroll
+        for (int k = 0; k < G; k++)
+          if (k < N) SD(stage, k * N + r) = col[k];
+      }
+      wave_sync();
+      double v[CH];
+#pragma unroll
+      for (int q = 0; q < CH; q++) v[q] = lane + 64 * q < NN ? SD(stage, lane + 64 * q) : 0.0;
+      const Scr T = make_scr<XM>(wave0 + g * slice, Pp->L.M, G, Pp->L.K);
+      for (int s = s0; s < s1; s++) {
+        const int place = LI(T.gp, s);
+        if (place < 0) continue;
+        const double w = s == 6 ? 1.0 : LD(T.gc, s);
+        double *out = vals + (long long)place * NN + lane;
+#pragma unroll
+        for (int q = 0; q < CH; q++)
+          if (lane + 64 * q < NN) __builtin_nontemporal_store(w * v[q], out + 64 * q);
+      }
+    }
+  } else {
+    const Scr T = make_scr<XM>(wave0 + (lane / G) * slice, Pp->L.M, G, Pp->L.K);
+    if (active && r < N) {
+      for (int s = s0; s < s1; s++) {
+        const int place = LI(T.gp, s);
+        if (place < 0) continue;
+        const double w = s == 6 ? 1.0 : LD(T.gc, s);
+        double *out = vals + (long long)place * NN + r;
+#pragma unroll
+        for (int k = 0; k < G; k++)
+          if (k < N) out[(long long)k * N] = w * col[k];
+      }
+    }
+  }
+}
+
 // A load issued whether or not the array is given: a missing array reads
 // `dummy` (any valid device address) and the caller selects its default.
 __device__ __forceinline__ double ld_or(const double *a, long long i, const unsigned char *dummy) {
@@ -650,6 +770,7 @@ template <int G, int MODE, int LUP, bool XM>
 __device__ __forceinline__ void react_body(uint64_t praw) {
   const KP P0 = (KP)praw;
   const int N = P0->L.N, M = P0->L.M, K = P0->L.K, R = P0->L.R;
+  constexpr bool kEval = MODE == PFX_MODE_EVAL || MODE == PFX_MODE_GI;
   // a pivoting reaction launch given the deferred list works through it
   constexpr bool kCanDefer = MODE == PFX_MODE_REACT && LUP == PFX_LU_DEFER;
   const bool from_list = MODE == PFX_MODE_REACT && LUP == PFX_LU_PIVOT && P0->defer != nullptr;
@@ -670,13 +791,15 @@ __device__ __forceinline__ void react_body(uint64_t praw) {
   const int r = threadIdx.x & (G - 1);
   const int gbase = lane - r;
   const bool live = r < N;  // padding lanes carry an identity row
-  const int sdoubles = scr_doubles(M, G, K, XM);
+  const int sdoubles = scr_doubles(M, G, K, XM, MODE == PFX_MODE_GI);
   // The group's scratch offsets, and the lane's charge and ion size, are
   // rebuilt every pass from opaque copies of their base values: held across
   // the persistent loop they cost ~15 registers that the register-capped
   // variants spilled to scratch and reloaded on every pass.
   int sbase = lds_tab + (int)(threadIdx.x / G) * sdoubles * 8;
   int r_opq = r;
+  // the wavefront's staging block (GI, groups of up to 16 lanes)
+  const int gi_stage = lds_tab + (int)(blockDim.x / G) * sdoubles * 8 + (int)(threadIdx.x >> 6) * gi_stage_doubles(N, G) * 8;
   if (r == 0) SD(make_scr<XM>(sbase, M, G, K).C, M) = 0.0;
 
   // wave-level work queue state (identical in all lanes of the wave): each
@@ -685,7 +808,7 @@ __device__ __forceinline__ void react_body(uint64_t praw) {
   const long long q_own = from_list ? 0 : P0->share, q_base = q_own * P0->waves;
   long long q_next = 0, q_end = 0, q_seen = q_base;
   if (q_own > 0) {
-    const long long wave = (long long)((int)blockIdx.x - P0->block0) * (BLOCK / 64) + (threadIdx.x >> 6);
+    const long long wave = (long long)((int)blockIdx.x - P0->block0) * (blockDim.x >> 6) + (threadIdx.x >> 6);
     q_next = wave * q_own;
     q_end = q_next + q_own < ncl ? q_next + q_own : ncl;
   }
@@ -866,6 +989,7 @@ __device__ __forceinline__ void react_body(uint64_t praw) {
           if constexpr (XM) {
             if (r == 0) SD(S.cs, 4) = tempc;
           }
+          if constexpr (MODE == PFX_MODE_GI) gi_load_faces<G>(Pp, S, (int)c, r, lane);
           const double tk = tempc + 273.15;
           const double ln_tk = log(tk);
           if (MODE == PFX_MODE_EQUIL) {
@@ -1110,6 +1234,7 @@ __device__ __forceinline__ void react_body(uint64_t praw) {
     // (not needed at the previous state, whose complexes only feed the
     // activity update)
     double row[G];
+    double col[MODE == PFX_MODE_GI ? G : 1];
     double Tsum = 0.0, absum = 0.0;
     const double den_kg_per_L = SD(S.cs, 3) * 1.0e-3;
     if (active && !(MODE == PFX_MODE_REACT && phase == 0)) {
@@ -1154,15 +1279,13 @@ __device__ __forceinline__ void react_body(uint64_t praw) {
       tot_out = (m + Tsum) * den_kg_per_L;
     }
     PFX_PT(3);
-    if (MODE == PFX_MODE_EVAL && active && live) {
-      // aqueous totals and dT/dm of the cell for the flux terms of the
-      // global-implicit assembly (RTAuxVarCompute's total and dtotal)
-      if (P.tot_eval_out) P.tot_eval_out[cell * N + r] = tot_out;
-      if (P.dtot_out) {
+    if constexpr (MODE == PFX_MODE_GI) {
+      // aqueous totals for the flux residual, and the blocks of the
+      // neighbours' rows in this cell's column: each a scalar times dT/dm
+      if (active && live) P.tot_eval_out[cell * N + r] = tot_out;
 #pragma unroll
-        for (int k = 0; k < G; k++)
-          if (k < N) P.dtot_out[cell * N * N + (long long)k * N + r] = P.col_scale ? row[k] * SD(S.mv, k) : row[k];
-      }
+      for (int k = 0; k < G; k++) col[k] = P.col_scale ? row[k] * SD(S.mv, k) : row[k];
+      gi_store_blocks<G, XM>(Pp, col, r, active, gi_stage, 0, 6);
     }
     if (MODE == PFX_MODE_REACT && active && phase == 0) {
       phase = 1;  // complexes of the previous state are in LDS: update activity next pass
@@ -1178,7 +1301,7 @@ __device__ __forceinline__ void react_body(uint64_t praw) {
     // ---------------------------------------------------------------
     // equilibrium ion exchange (RTotalSorbEqIonx): sorbed total of row r and
     // d(sorbed)/dm added to row[] with weight ionx_w
-    const bool need_ionx = (MODE == PFX_MODE_REACT || MODE == PFX_MODE_EVAL) ? true : false;
+    const bool need_ionx = (MODE == PFX_MODE_REACT || kEval) ? true : false;
     const bool ionx_final = (MODE == PFX_MODE_AUX || MODE == PFX_MODE_EQUIL);
     double Sr = 0.0;
     // d(sorbed total of row r)/dm for a total-sorbed constraint row
@@ -1189,6 +1312,13 @@ __device__ __forceinline__ void react_body(uint64_t praw) {
     const double dt = P.dt;
     const double vol = SD(S.cs, 2);
     const double psv_t = SD(S.cs, 0) * SD(S.cs, 1) * 1000.0 * vol;
+    // On a grid the rows take the accumulation's weight, with the cell's own
+    // share of its faces' fluxes, before sorption and minerals add to them.
+    if (MODE == PFX_MODE_GI && active) {
+      const double w = psv_t / dt + SD(S.gc, 6);
+#pragma unroll
+      for (int k = 0; k < G; k++) row[k] = live ? row[k] * w : row[k];
+    }
     if (active && R > 0 && (need_ionx || ionx_final)) {
       const double ionx_w = need_ionx ? vol / dt : 0.0;
       for (int q = 0; q < R; q++) {
@@ -1236,7 +1366,8 @@ __device__ __forceinline__ void react_body(uint64_t praw) {
         const double t2 = Zr / sumZX;
         Sr += t1;
         if (need_ionx) {
-          const double wscale = ionx_w / (live ? psv_t / dt : 1.0);
+          // row[] is scaled by psv_t/dt later, but on a grid
+          const double wscale = MODE == PFX_MODE_GI ? ionx_w : ionx_w / (live ? psv_t / dt : 1.0);
           SD(S.xb, r) = X;
           wave_sync();
 #pragma unroll
@@ -1282,7 +1413,8 @@ __device__ __forceinline__ void react_body(uint64_t praw) {
           dres = res / m * inv_n;
         }
         Sr += res;
-        const double jw = need_ionx ? vol / psv_t : 1.0;  // row[] is scaled by psv_t/dt later
+        // row[] is scaled by psv_t/dt later, but on a grid
+        const double jw = !need_ionx ? 1.0 : (MODE == PFX_MODE_GI ? vol / dt : vol / psv_t);
 #pragma unroll
         for (int k = 0; k < G; k++) {
           if (k == r) {
@@ -1304,10 +1436,11 @@ __device__ __forceinline__ void react_body(uint64_t praw) {
     double rr = 0.0;
     int use_log = L.use_log;
     if (MODE == PFX_MODE_AUX && active) finish = true;
-    if ((MODE == PFX_MODE_REACT || MODE == PFX_MODE_EVAL) && active) {
+    if ((MODE == PFX_MODE_REACT || kEval) && active) {
       // accumulation (mol/s) and its derivative: the dt-consistent form
+      if (MODE != PFX_MODE_GI)
 #pragma unroll
-      for (int k = 0; k < G; k++) row[k] = live ? row[k] * (psv_t / dt) : row[k];
+        for (int k = 0; k < G; k++) row[k] = live ? row[k] * (psv_t / dt) : row[k];
       if (live) {
         const double fixed = SD(S.fx, r);
         Rr = (psv_t * tot_out + (L.sorb_any ? Sr * vol : 0.0)) / dt - fixed / dt;
@@ -1315,12 +1448,12 @@ __device__ __forceinline__ void react_body(uint64_t praw) {
         scale = psv * (m + absum) / dt + fabs(Sr) * vol / dt + fabs(fixed) / dt;
       }
       // kinetic minerals (group-uniform rates, row-local residual/Jacobian)
-      const bool fd_jac = MODE == PFX_MODE_EVAL && L.num_jac;
+      const bool fd_jac = kEval && L.num_jac;
       // the capped-Q/K derivative for the attempt's first iterations only
       // (the attempt started at it_cap less its budget)
       const int att_it = it - (it_cap - ((MODE == PFX_MODE_REACT && P.guess_mode == PFX_GUESS_ARRAY_FALLBACK &&
                                           !fell_back) ? P.fallback_after : P.max_iterations));
-      const bool capped_jac = (P.jac_flags & PFX_JAC_CAPPED_QK) && (MODE == PFX_MODE_EVAL || att_it < PFX_JAC_CAPPED_ITERS);
+      const bool capped_jac = (P.jac_flags & PFX_JAC_CAPPED_QK) && (kEval || att_it < PFX_JAC_CAPPED_ITERS);
       for (int k = 0; k < K; k++) {
         double lnQK = SD(S.mlnK, k);
         for (int s = 0; s < L.S; s++) {
@@ -1371,9 +1504,9 @@ __device__ __forceinline__ void react_body(uint64_t praw) {
           SD(S.mrate, k) = 0.0;
         }
       }
-      if (MODE == PFX_MODE_EVAL && fd_jac && K > 0) mineral_fd_jacobian<G, XM>(Pp, S, r, live, m, lng, vol, row);
+      if (kEval && fd_jac && K > 0) mineral_fd_jacobian<G, XM>(Pp, S, r, live, m, lng, vol, row);
       rr = gmax<G>(live ? fabs(Rr) / fmax(scale, 1e-300) : 0.0, lane);
-      if (MODE == PFX_MODE_EVAL) {
+      if (kEval) {
         finish = true;
       } else if (cell_flag != PFX_CELL_CONVERGED) {
         finish = true;
@@ -1699,18 +1832,26 @@ __device__ __forceinline__ void react_body(uint64_t praw) {
       if (fell_back) P.num_iterations[cell] = it_cap - P.max_iterations;  // the warm attempt's iterations
     }
 
+    if constexpr (MODE == PFX_MODE_GI) {
+      // the cell's own block: the evaluated Jacobian, its faces' share in it
+#pragma unroll
+      for (int k = 0; k < G; k++) col[k] = P.col_scale ? row[k] * SD(S.mv, k) : row[k];
+      gi_store_blocks<G, XM>(Pp, col, r, active, gi_stage, 6, 7);
+    }
+
     // ---------------------------------------------------------------
     // retire the cell: write the state at this iterate
     if (active && finish) {
       const long long c = cell;
       if (deferred) {
         // nothing written: the inputs stay for the pivoting launch
-      } else if (MODE == PFX_MODE_EVAL) {
+      } else if (kEval) {
         if (live) {
           P.res_out[c * N + r] = Rr;
+          if (MODE == PFX_MODE_EVAL)
 #pragma unroll
-          for (int k = 0; k < G; k++)
-            if (k < N) P.jac_out[c * N * N + (long long)k * N + r] = P.col_scale ? row[k] * SD(S.mv, k) : row[k];
+            for (int k = 0; k < G; k++)
+              if (k < N) P.jac_out[c * N * N + (long long)k * N + r] = row[k];
         }
         // the mineral rates at this iterate (the last evaluation of a
         // global-implicit solve leaves those of its solution)
@@ -1827,12 +1968,18 @@ template __global__ void pfx_react_zones_kernel<1, true>(const pfx_kernel_params
   PFX_INST_LU(G, PFX_MODE_REACT, 1, PFX_LU_DEFER, true)     \
   PFX_INST_LU(G, PFX_MODE_REACT, 1, PFX_LU_ONDEMAND, true)  \
   PFX_INST_LU(G, PFX_MODE_REACT, 1, PFX_LU_PIVOT, true)     \
-  PFX_INST_LU(G, PFX_MODE_EVAL, 1, PFX_LU_PIVOT, true)
+  PFX_INST_LU(G, PFX_MODE_EVAL, 1, PFX_LU_PIVOT, true)      \
+  PFX_INST_LU(G, PFX_MODE_GI, 1, PFX_LU_PIVOT, false)       \
+  PFX_INST_LU(G, PFX_MODE_GI, 1, PFX_LU_PIVOT, true)
 // The instantiations are compiled in parts (PFX_REACT_PART 0..3), each its
 // own object, so that they build in parallel; without it one object has all.
 #if !defined(PFX_REACT_PART) || PFX_REACT_PART == 0
 PFX_INST(8)
-extern "C" int pfx_scr_doubles(int M, int G, int K, int xm) { return scr_doubles(M, G, K, xm != 0); }
+// LDS of a workgroup of `threads` threads beside the tables, bytes
+extern "C" int pfx_scr_bytes(int threads, int N, int M, int G, int K, int xm, int mode) {
+  const bool gi = mode == PFX_MODE_GI;
+  return 8 * ((threads / G) * scr_doubles(M, G, K, xm != 0, gi) + (gi ? (threads / 64) * gi_stage_doubles(N, G) : 0));
+}
 #endif
 #if !defined(PFX_REACT_PART) || PFX_REACT_PART == 1
 PFX_INST(16)
