@@ -387,6 +387,7 @@ void fill_params(pfx_tables *t, pfx_cells *cells, const pfx_react_opts *o, pfx_k
   P.status = cells->status;
   P.rel_res = cells->rel_res;
   P.dt = o->dt;
+  P.inv_dt = 1.0 / o->dt;
   P.rel_tol = o->rel_tol;
   P.default_guess = o->default_guess;
   P.def_porosity = o->porosity;
@@ -747,7 +748,9 @@ extern "C" int pfx_tables_create(const pfx_reaction_desc *d, pfx_tables **out) {
   }
   pfx_dev_layout L;
   memset(&L, 0, sizeof(L));
-  L.N = N; L.M = M; L.K = K; L.R = R; L.G = G; L.S = S0;
+  L.N = N; L.M = M; L.K = K; L.R = R; L.G = G;
+  L.packs = (S0 + 3) / 4;
+  const int SP = 4 * L.packs;
   L.Q = (M + G - 1) / G;
 
   auto cid = [&](int i, int s) { return d->eqcplxspecid[(size_t)i * (S0 + 1) + 1 + s]; };
@@ -764,17 +767,17 @@ extern "C" int pfx_tables_create(const pfx_reaction_desc *d, pfx_tables **out) {
   for (int j = 0; j < N; j++) { Z[j] = d->primary_spec_Z[j]; a0[j] = d->primary_spec_a0[j]; }
   L.o_Z = B.add(Z);
   L.o_a0 = B.add(a0);
-  std::vector<int32_t> cspec((size_t)M * S0, -1);
-  std::vector<double> cnuv((size_t)M * S0, 0.0), cZ(M), ca0(M), clogK(M), ccoef((size_t)M * 5, 0.0);
+  std::vector<uint16_t> cpk((size_t)std::max(M, 1) * SP, (uint16_t)(8 * G));
+  std::vector<double> cnuv((size_t)std::max(M, 1) * SP, 0.0), cZ(M), ca0(M), clogK(M), ccoef((size_t)M * 5, 0.0);
   for (int i = 0; i < M; i++) {
-    for (int s = 0; s < cnt(i); s++) { cspec[i * S0 + s] = cid(i, s); cnuv[i * S0 + s] = cnu(i, s); }
+    for (int s = 0; s < cnt(i); s++) { cpk[i * SP + s] = (uint16_t)(8 * cid(i, s)); cnuv[i * SP + s] = cnu(i, s); }
     cZ[i] = d->eqcplx_Z[i];
     ca0[i] = d->eqcplx_a0[i];
     clogK[i] = d->eqcplx_logK[i];
     if (d->eqcplx_logKcoef) for (int q = 0; q < 5; q++) ccoef[i * 5 + q] = d->eqcplx_logKcoef[i * 5 + q];
   }
   L.has_logk_coef = d->eqcplx_logKcoef != nullptr;
-  L.o_cspec = B.add(cspec);
+  L.o_cpk = B.add(cpk);
   L.o_cnu = B.add(cnuv);
   L.o_cZ = B.add(cZ);
   L.o_ca0 = B.add(ca0);
@@ -799,11 +802,11 @@ extern "C" int pfx_tables_create(const pfx_reaction_desc *d, pfx_tables **out) {
   int maxdeg = 0;
   for (int r = 0; r < G; r++) maxdeg = std::max<int>(maxdeg, (int)adj[r].size());
   L.maxdeg = maxdeg;
-  std::vector<int32_t> adj_c((size_t)std::max(maxdeg, 1) * G, M);
+  std::vector<int32_t> adj_c((size_t)std::max(maxdeg, 1) * G, 8 * M);
   std::vector<double> adj_nu((size_t)std::max(maxdeg, 1) * G, 0.0);
   for (int r = 0; r < G; r++)
     for (size_t e = 0; e < adj[r].size(); e++) {
-      adj_c[e * G + r] = adj[r][e].first;
+      adj_c[e * G + r] = 8 * adj[r][e].first;
       adj_nu[e * G + r] = adj[r][e].second;
     }
   L.o_adj_c = B.add(adj_c);
@@ -822,14 +825,14 @@ extern "C" int pfx_tables_create(const pfx_reaction_desc *d, pfx_tables **out) {
   }
   L.offq_start[nq] = rows;
   for (int q = nq + 1; q <= PFX_MAX_PRIMARY / 4; q++) L.offq_start[q] = rows;
-  std::vector<uint16_t> offq_c((size_t)std::max(rows, 1) * G * 4, (uint16_t)M);
+  std::vector<uint16_t> offq_c((size_t)std::max(rows, 1) * G * 4, (uint16_t)(8 * M));
   std::vector<double> offq_coef((size_t)std::max(rows, 1) * G * 4, 0.0);
   for (int q = 0; q < nq; q++)
     for (int j = 0; j < 4; j++)
       for (int r = 0; r < G; r++)
         for (size_t e = 0; e < off[4 * q + j][r].size(); e++) {
           const size_t row = (size_t)L.offq_start[q] + e;
-          offq_c[(row * G + r) * 4 + j] = (uint16_t)off[4 * q + j][r][e].first;
+          offq_c[(row * G + r) * 4 + j] = (uint16_t)(8 * off[4 * q + j][r][e].first);
           offq_coef[((row * 2 + j / 2) * G + r) * 2 + (j % 2)] = off[4 * q + j][r][e].second;
         }
   L.o_offq_c = B.add(offq_c);
@@ -838,8 +841,8 @@ extern "C" int pfx_tables_create(const pfx_reaction_desc *d, pfx_tables **out) {
   // minerals
   auto mid = [&](int k, int s) { return d->kinmnrlspecid[(size_t)k * (S0 + 1) + 1 + s]; };
   auto mcnt = [&](int k) { return d->kinmnrlspecid[(size_t)k * (S0 + 1)]; };
-  std::vector<int32_t> mspec((size_t)std::max(K, 1) * S0, -1);
-  std::vector<double> mnu((size_t)std::max(K, 1) * S0, 0.0), mnuG((size_t)std::max(K, 1) * G, 0.0);
+  std::vector<uint16_t> mpk((size_t)std::max(K, 1) * SP, (uint16_t)(8 * G));
+  std::vector<double> mnu((size_t)std::max(K, 1) * SP, 0.0), mnuG((size_t)std::max(K, 1) * G, 0.0);
   std::vector<double> mlogK(std::max(K, 1)), mcoef((size_t)std::max(K, 1) * 5, 0.0), mk(std::max(K, 1)),
       mmv(std::max(K, 1)), mEa(std::max(K, 1), 0.0), mthr(std::max(K, 1), 0.0), mlim(std::max(K, 1), 0.0),
       mpow(std::max(K, 1), 1.0), mtk(std::max(K, 1), 1.0);
@@ -848,8 +851,8 @@ extern "C" int pfx_tables_create(const pfx_reaction_desc *d, pfx_tables **out) {
     for (int s = 0; s < mcnt(k); s++) {
       const int sp = mid(k, s);
       if (sp < 0 || sp >= N) return PFX_E_ARG;
-      mspec[k * S0 + s] = sp;
-      mnu[k * S0 + s] = d->kinmnrlstoich[(size_t)k * S0 + s];
+      mpk[k * SP + s] = (uint16_t)(8 * sp);
+      mnu[k * SP + s] = d->kinmnrlstoich[(size_t)k * S0 + s];
       mnuG[k * G + sp] += d->kinmnrlstoich[(size_t)k * S0 + s];
     }
     mlogK[k] = d->kinmnrl_logK[k];
@@ -905,7 +908,7 @@ extern "C" int pfx_tables_create(const pfx_reaction_desc *d, pfx_tables **out) {
   L.mnrl_flags = (d->kinmnrl_affinity_threshold ? 1 : 0) | (d->kinmnrl_rate_limiter ? 2 : 0) |
                  (d->kinmnrl_affinity_power ? 4 : 0) | (d->kinmnrl_Temkin_const ? 8 : 0) |
                  (any_pref ? 16 : 0) | (d->kinmnrl_min_scale_factor ? 32 : 0);
-  L.o_mspec = B.add(mspec);
+  L.o_mpk = B.add(mpk);
   L.o_mnu = B.add(mnu);
   L.o_mnuG = B.add(mnuG);
   L.o_mlogK = B.add(mlogK);

@@ -15,7 +15,8 @@
 // primary species r (row r of the local Jacobian).  Per-lane tables are
 // stored [entry][G] so the G lanes of a group read consecutive words.
 struct pfx_dev_layout {
-  int32_t N, M, K, R, G, S;     // sizes; S = species slots per complex/mineral
+  int32_t N, M, K, R, G;        // sizes
+  int32_t packs;                // groups of 4 species slots per complex/mineral
   int32_t Q;                    // complex rounds per lane = ceil(M/G)
   int32_t maxdeg;               // max complexes touching one primary
   // off-diagonal co-occurrence lists of dT_r/dm_k in chunks of 4 columns:
@@ -41,17 +42,18 @@ struct pfx_dev_layout {
 
   // byte offsets into the table blob (doubles unless noted)
   int64_t o_Z, o_a0;                 // [G]
-  int64_t o_cspec;                   // int32 [M][S]  (-1 = empty slot)
-  int64_t o_cnu;                     // [M][S]
+  int64_t o_cpk;                     // uint16 [M][packs][4] byte offset of a slot's species in a
+                                     // cell's ln activities (8 G, where a zero is, if empty)
+  int64_t o_cnu;                     // [M][packs][4]
   int64_t o_cZ, o_ca0;               // [M]
   int64_t o_clogK;                   // [M] log10 K at the reference temperature
   int64_t o_clogKcoef;               // [M][5]
-  int64_t o_adj_c;                   // int32 [maxdeg][G], -> M = zero slot
+  int64_t o_adj_c;                   // int32 [maxdeg][G] byte offset in C (8 M = zero slot)
   int64_t o_adj_nu;                  // [maxdeg][G]
-  int64_t o_offq_c;                  // uint16 [rows][G][4] complex (M = zero slot)
+  int64_t o_offq_c;                  // uint16 [rows][G][4] byte offset in C (8 M = zero slot)
   int64_t o_offq_coef;               // [rows][2][G][2] nu_r * nu_k
-  int64_t o_mspec;                   // int32 [K][S]
-  int64_t o_mnu;                     // [K][S]
+  int64_t o_mpk;                     // uint16 [K][packs][4], as o_cpk
+  int64_t o_mnu;                     // [K][packs][4]
   int64_t o_mnuG;                    // [K][G] dense stoichiometry per lane
   int64_t o_mlogK, o_mlogKcoef;
   int64_t o_mk, o_mmolvol, o_mEa, o_mthr, o_mlim, o_mpow, o_mtemkin;  // [K]
@@ -101,7 +103,7 @@ struct pfx_kernel_params {
   int32_t *num_iterations, *status;
   double *rel_res;
   // options
-  double dt, rel_tol, default_guess;
+  double dt, inv_dt, rel_tol, default_guess;
   double def_porosity, def_saturation, def_volume, def_den;
   int32_t max_iterations, extra_iterations, guess_mode, reference_stop;
   int32_t fallback_after;       // warm-attempt iteration cap (PFX_GUESS_ARRAY_FALLBACK)

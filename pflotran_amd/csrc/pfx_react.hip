@@ -379,6 +379,31 @@ extern __shared__ __align__(16) unsigned char smem[];
 #define LI(off, i) (((const int32_t *)(smem + (off)))[(i)])
 #define SD(off, i) (((double *)(smem + (off)))[(i)])
 
+// lnq + sum_s nu_s ln a_s of reaction i, slots in order: 4 species at a time,
+// their byte offsets from la in one 8-byte word and their coefficients in two
+// 16-byte words (an empty slot reads la[G] = 0 with coefficient 0).
+// Bound by instruction issue (two wavefronts per SIMD hold the registers): four
+// LDS reads in flight and four multiply-adds, where a slot at a time took an
+// index load, an address, a compare and a branch each.
+__device__ __forceinline__ double ln_iap(double lnq, int o_pk, int o_nu, int i, int packs, int la) {
+  for (int b = 0; b < packs; b++) {
+    const int w = i * packs + b;
+    const uint2 k = *(const uint2 *)(smem + o_pk + w * 8);
+    const double2 n0 = *(const double2 *)(smem + o_nu + w * 32);
+    const double2 n1 = *(const double2 *)(smem + o_nu + w * 32 + 16);
+    lnq += n0.x * LD(la + (int)(k.x & 0xffffu), 0);
+    lnq += n0.y * LD(la + (int)(k.x >> 16), 0);
+    lnq += n1.x * LD(la + (int)(k.y & 0xffffu), 0);
+    lnq += n1.y * LD(la + (int)(k.y >> 16), 0);
+  }
+  return lnq;
+}
+// species of slot s of reaction i (G or above: empty) and its coefficient
+__device__ __forceinline__ int rxn_species(int o_pk, int i, int packs, int s) {
+  return (int)(((const uint16_t *)(smem + o_pk))[i * packs * 4 + s] >> 3);
+}
+__device__ __forceinline__ double rxn_nu(int o_nu, int i, int packs, int s) { return LD(o_nu, i * packs * 4 + s); }
+
 // 5-term log K(T) (reaction_aux.F90:1461-1488) evaluated without fused
 // multiply-add, in the reference's order: the fitted coefficients cancel to
 // ~1e-3 of their terms, so contraction alone would move K by ~1e-12.
@@ -404,9 +429,10 @@ __device__ __forceinline__ double logk_5term_ptr(const double *cf, double tk, do
 }
 
 // per-group scratch slice (doubles), as byte offsets from the slice base:
-//   C[M+1] complex molalities (C[M] = 0, padding slot), gsec[M] complex
-//   activity coefficients, lnK[M] = -log10 K * LOG_TO_LN of this cell,
-//   la[G] ln activities, mv[G] free ions, im[G] inverse free ions,
+//   C[M+1] complex molalities (C[M] = 0, padding slot), gsec[M] ln activity
+//   coefficients of the complexes, lnK[M] = -log10 K * LOG_TO_LN of this cell,
+//   la[G+1] ln activities (la[G] = 0, the empty stoichiometry slots' species),
+//   mv[G] free ions, im[G] inverse free ions,
 //   xb[G] ion-exchange fractions, mlnK/mkeff/marea/mvf/mrate[K] per mineral,
 //   cs[4] the cell's porosity, saturation, volume and water density (cs[6]
 //   in the prefactor kernels: then also its temperature (C) and a spare),
@@ -420,7 +446,7 @@ struct Scr {
 };
 
 __host__ __device__ inline int scr_doubles(int M, int G, int K, bool xm, bool gi) {
-  int n = (M + 1) + 2 * M + 5 * G + 5 * K + (xm ? 6 : 4) + PFX_MAX_IONX_RXN + (gi ? 12 : 0);
+  int n = (M + 1) + 2 * M + 5 * G + 2 + 5 * K + (xm ? 6 : 4) + PFX_MAX_IONX_RXN + (gi ? 12 : 0);
   return (n + 1) & ~1;
 }
 
@@ -435,7 +461,8 @@ __host__ __device__ inline int gi_stage_doubles(int N, int G) { return G <= 16 ?
 template <bool XM>
 __device__ __forceinline__ Scr make_scr(int base, int M, int G, int K) {
   Scr s;
-  s.la = base;
+  s.la = base;                // la[G] = 0 and a spare
+  base += 16;
   s.mv = base + 8 * G;
   s.im = base + 16 * G;
   s.xb = base + 24 * G;
@@ -460,12 +487,18 @@ __device__ __forceinline__ Scr make_scr(int base, int M, int G, int K) {
 }  // namespace
 
 // ---------------------------------------------------------------------------
+// ln of exp(v) as a double holds it: the coefficient that overflows or
+// vanishes counts as infinite or zero, as where it is formed and its log taken
+__device__ __forceinline__ double ln_of_exp(double v) {
+  return v > 709.782712893384 ? INFINITY : (v < -745.1332191019412 ? -INFINITY : v);
+}
+
 // x^z for the valence ratios of ion exchange: the common ratios 1, 2, 1/2
 // and 3 without the log/exp of a general power (same value to the last bit
 // or within one rounding)
 __device__ __forceinline__ double pow_ratio(double x, double z) {
-  if (z == 1.0) return x;
-  if (z == 2.0) return x * x;
+  const double p = z == 2.0 ? x * x : x;
+  if (z == 1.0 || z == 2.0) return p;
   if (z == 0.5) return sqrt(x);
   if (z == 3.0) return x * x * x;
   return pow(x, z);
@@ -562,7 +595,7 @@ __device__ __forceinline__ double mineral_rate(KP Pp, const Scr &S, int k, doubl
 // d monod_s / d a_s * gamma_s * k_p * Arrhenius_p, added to column s of the
 // lane's row with the lane's stoichiometric coefficient nur.  dIm_dsum is
 // Im (mol/s) over the summed rate constant.
-template <int G>
+template <int G, bool LN>
 __device__ __forceinline__ void prefactor_jacobian(KP Pp, const Scr &S, int k, double dIm_dsum, double nur,
                                                    double *row) {
   const int np = LI(Pp->L.o_mpn, k);
@@ -592,8 +625,7 @@ __device__ __forceinline__ void prefactor_jacobian(KP Pp, const Scr &S, int k, d
       const double lgb = beta * la;
       const double denom = 1.0 + exp(log(atten) + lgb);
       const double dden = -1.0 * exp(lps) / denom * atten * beta * exp(lgb - la);
-      const double gam_s = exp(la) * SD(S.im, sp);  // activity over molality
-      const double dspec = (dnum + dden) * gam_s;
+      const double dspec = (dnum + dden) * exp(la) * (LN ? 1.0 : SD(S.im, sp));
       const double dIm = dIm_dsum * dpref * dspec * LD(Pp->L.o_mprate, k * PP + p) * arr;
 #pragma unroll
       for (int kk = 0; kk < G; kk++) row[kk] += (kk == sp) ? nur * dIm : 0.0;
@@ -605,11 +637,12 @@ __device__ __forceinline__ void prefactor_jacobian(KP Pp, const Scr &S, int k, d
 // RReactionDerivative reaction.F90:3625-3684): column j is
 // (Res(m + e_j m_j 1e-5) - Res(m)) / (m_j 1e-5), Res = sum_k nu_ik Im_k V in
 // mineral order from zero; entries below 1e-40 in magnitude become 0.  The
-// perturbed ln activities use the unperturbed coefficients.  Adds to row[].
+// perturbed ln activities use the unperturbed coefficients.  Adds to row[],
+// whose columns are d / d ln m.
 template <int G, bool XM>
 __device__ __forceinline__ void mineral_fd_jacobian(KP Pp, const Scr &S, int r, bool live, double m, double lng,
                                                     double vol, double *row) {
-  const int K = Pp->L.K, nS = Pp->L.S;
+  const int K = Pp->L.K, packs = Pp->L.packs;
   {
 #pragma clang fp contract(off)
     if (live) SD(S.xb, r) = log(m + m * 1.0e-5) + lng;  // perturbed ln a_r
@@ -617,11 +650,7 @@ __device__ __forceinline__ void mineral_fd_jacobian(KP Pp, const Scr &S, int r, 
   wave_sync();
   double ro = 0.0;
   for (int k = 0; k < K; k++) {
-    double lnQK = SD(S.mlnK, k);
-    for (int s = 0; s < nS; s++) {
-      const int sp = LI(Pp->L.o_mspec, k * nS + s);
-      if (sp >= 0) lnQK += LD(Pp->L.o_mnu, k * nS + s) * SD(S.la, sp);
-    }
+    const double lnQK = ln_iap(SD(S.mlnK, k), (int)Pp->L.o_mpk, (int)Pp->L.o_mnu, k, packs, S.la);
     const double nur = live ? LD(Pp->L.o_mnuG, k * G + r) : 0.0;
     ro += nur * (mineral_rate<XM>(Pp, S, k, lnQK, -1) * vol);
   }
@@ -631,9 +660,9 @@ __device__ __forceinline__ void mineral_fd_jacobian(KP Pp, const Scr &S, int r, 
       double rp = 0.0;
       for (int k = 0; k < K; k++) {
         double lnQK = SD(S.mlnK, k);
-        for (int s = 0; s < nS; s++) {
-          const int sp = LI(Pp->L.o_mspec, k * nS + s);
-          if (sp >= 0) lnQK += LD(Pp->L.o_mnu, k * nS + s) * (sp == j ? SD(S.xb, j) : SD(S.la, sp));
+        for (int s = 0; s < 4 * packs; s++) {
+          const int sp = rxn_species((int)Pp->L.o_mpk, k, packs, s);
+          lnQK += rxn_nu((int)Pp->L.o_mnu, k, packs, s) * (sp == j ? SD(S.xb, j) : SD(S.la, sp));
         }
         const double nur = live ? LD(Pp->L.o_mnuG, k * G + r) : 0.0;
         rp += nur * (mineral_rate<XM>(Pp, S, k, lnQK, j) * vol);
@@ -645,7 +674,7 @@ __device__ __forceinline__ void mineral_fd_jacobian(KP Pp, const Scr &S, int r, 
       }
       double d = (rp - ro) / pert;
       if (fabs(d) < 1.0e-40) d = 0.0;
-      if (live) row[j] += d;
+      if (live) row[j] += d * SD(S.mv, j);
     }
   }
   wave_sync();
@@ -771,6 +800,17 @@ __device__ __forceinline__ void react_body(uint64_t praw) {
   const KP P0 = (KP)praw;
   const int N = P0->L.N, M = P0->L.M, K = P0->L.K, R = P0->L.R;
   constexpr bool kEval = MODE == PFX_MODE_EVAL || MODE == PFX_MODE_GI;
+  // A Newton pass is bound by FP64 issue, where a log costs about 40
+  // multiply-adds and a division 12: with ln m carried and ln coefficients kept
+  // in place of the coefficients, a pass of these forms holds one log and a few
+  // reciprocals, and the elimination's columns need no scaling.  1M cells of 15
+  // primaries 18.6 -> 14.9 ms, 50021 cells 2.07 -> 1.51 ms, 800k cells of three
+  // networks (15/20/30 primaries) 31.0 -> 23.9 ms.
+  // the unpivoted step and the evaluations carry ln m and the Jacobian's
+  // columns as d / d ln m; constraint rows replace m, and the pivoting step
+  // keeps the reference's columns (d / d m, equilibrated, then scaled by m), so
+  // that far from a solution it also fails as the reference does
+  constexpr bool kLn = (MODE == PFX_MODE_REACT && LUP == PFX_LU_DEFER) || kEval;
   // a pivoting reaction launch given the deferred list works through it
   constexpr bool kCanDefer = MODE == PFX_MODE_REACT && LUP == PFX_LU_DEFER;
   const bool from_list = MODE == PFX_MODE_REACT && LUP == PFX_LU_PIVOT && P0->defer != nullptr;
@@ -800,7 +840,11 @@ __device__ __forceinline__ void react_body(uint64_t praw) {
   int r_opq = r;
   // the wavefront's staging block (GI, groups of up to 16 lanes)
   const int gi_stage = lds_tab + (int)(blockDim.x / G) * sdoubles * 8 + (int)(threadIdx.x >> 6) * gi_stage_doubles(N, G) * 8;
-  if (r == 0) SD(make_scr<XM>(sbase, M, G, K).C, M) = 0.0;
+  if (r == 0) {
+    const Scr S0 = make_scr<XM>(sbase, M, G, K);
+    SD(S0.C, M) = 0.0;
+    SD(S0.la, G) = 0.0;
+  }
 
   // wave-level work queue state (identical in all lanes of the wave): each
   // wavefront owns a first share of the cells and fetches the rest.  q_seen
@@ -831,10 +875,10 @@ __device__ __forceinline__ void react_body(uint64_t praw) {
   // resolution of the free ions at the candidate iterate, whose step
   // (m_cand, its size rel_cand) waits
   bool floor_pass = false;
-  double rel_cand = 0.0, m_cand = 0.0;
+  double rel_cand = 0.0, m_cand = 0.0, l_cand = 0.0;
   double last_change = INFINITY;  // max|dm/m| of the attempt's last Newton update
   int cell_flag = PFX_CELL_CONVERGED;
-  double m = 1.0, gam = 1.0, lng = 0.0;
+  double m = 1.0, lnm = 0.0, gam = 1.0, lng = 0.0;
   // constraint speciation state
   int ctype = PFX_CONSTRAINT_FREE, nit_on = 0;
   bool compute_act = false;
@@ -994,7 +1038,7 @@ __device__ __forceinline__ void react_body(uint64_t praw) {
           const double ln_tk = log(tk);
           if (MODE == PFX_MODE_EQUIL) {
             gam = 1.0;
-            for (int cc = r; cc < M; cc += G) SD(S.gsec, cc) = 1.0;
+            for (int cc = r; cc < M; cc += G) SD(S.gsec, cc) = 0.0;
             const double molal_to_molar = P.molal ? den / 1000.0 : 1.0;
             const double molar_to_molal = P.molal ? 1.0 : 1000.0 / den;
             ctype = live ? P.ctype[r] : PFX_CONSTRAINT_FREE;
@@ -1028,7 +1072,7 @@ __device__ __forceinline__ void react_body(uint64_t praw) {
 #pragma unroll 4
             for (int cc = r; cc < M; cc += G) {
               const double g = ld_or(P.sec_act_coef, c * M + cc, dmy);
-              SD(S.gsec, cc) = P.sec_act_coef ? g : 1.0;
+              SD(S.gsec, cc) = P.sec_act_coef ? log(g) : 0.0;
             }
           }
           for (int cc = r; cc < M; cc += G) {
@@ -1068,6 +1112,7 @@ __device__ __forceinline__ void react_body(uint64_t praw) {
               else if (P.guess_mode == PFX_GUESS_DEFAULT) m = P.default_guess;
             }
           }
+          lnm = log(m);
         }
       }
     }
@@ -1099,6 +1144,7 @@ __device__ __forceinline__ void react_body(uint64_t praw) {
             if (P.guess_mode == PFX_GUESS_ARRAY || P.guess_mode == PFX_GUESS_ARRAY_FALLBACK)
               m = SD(S.xb, r);
             else if (P.guess_mode == PFX_GUESS_DEFAULT) m = P.default_guess;
+            lnm = log(m);
           }
         }
         const double A = L.debyeA, B = L.debyeB, Bd = L.debyeBdot;
@@ -1134,10 +1180,9 @@ __device__ __forceinline__ void react_body(uint64_t praw) {
                 if (fabs(z) > 0.0) {
                   const double t = 1.0 + B * LD(L.o_ca0, cc) * sqI;
                   double sum = 0.5 * A * z * z / (sqI * t * t) - Bd;
-                  const int nS = L.S;
-                  for (int s = 0; s < nS; s++) {
-                    const int sp = LI(L.o_cspec, cc * nS + s);
-                    if (sp >= 0 && fabs(LD(L.o_Z, sp)) > 0.0) sum += LD(L.o_cnu, cc * nS + s) * SD(S.im, sp);
+                  for (int s = 0; s < 4 * L.packs; s++) {
+                    const int sp = rxn_species((int)L.o_cpk, cc, L.packs, s);
+                    if (sp < G && fabs(LD(L.o_Z, sp)) > 0.0) sum += rxn_nu((int)L.o_cnu, cc, L.packs, s) * SD(S.im, sp);
                   }
                   const double dcdi = SD(S.C, cc) * PFX_LOG_TO_LN * sum;
                   dpart += 0.5 * z * z * dcdi;
@@ -1152,23 +1197,17 @@ __device__ __forceinline__ void react_body(uint64_t praw) {
             I = II;
             const double sqI = sqrt(I);
             if (live) {
-              gam = fabs(Zr) > 0.0 ? exp((-Zr * Zr * sqI * A / (1.0 + a0r * B * sqI) + Bd * I) * PFX_LOG_TO_LN)
-                                   : 1.0;
-              lng = log(gam);
+              lng = fabs(Zr) > 0.0 ? ln_of_exp((-Zr * Zr * sqI * A / (1.0 + a0r * B * sqI) + Bd * I) * PFX_LOG_TO_LN) : 0.0;
+              gam = exp(lng);
             }
             for (int cc = r; cc < M; cc += G) {
               const double z = LD(L.o_cZ, cc);
-              const double gs =
-                  fabs(z) > 0.0 ? exp((-z * z * sqI * A / (1.0 + LD(L.o_ca0, cc) * B * sqI) + Bd * I) * PFX_LOG_TO_LN)
-                                : 1.0;
-              SD(S.gsec, cc) = gs;
-              double lnQK = SD(S.lnK, cc);
-              const int nS = L.S;
-              for (int s = 0; s < nS; s++) {
-                const int sp = LI(L.o_cspec, cc * nS + s);
-                if (sp >= 0) lnQK += LD(L.o_cnu, cc * nS + s) * SD(S.la, sp);
-              }
-              SD(S.C, cc) = exp(lnQK) / gs;
+              const double lgs =
+                  fabs(z) > 0.0
+                      ? ln_of_exp((-z * z * sqI * A / (1.0 + LD(L.o_ca0, cc) * B * sqI) + Bd * I) * PFX_LOG_TO_LN)
+                      : 0.0;
+              SD(S.gsec, cc) = lgs;
+              SD(S.C, cc) = exp(ln_iap(SD(S.lnK, cc), (int)L.o_cpk, (int)L.o_cnu, cc, L.packs, S.la) - lgs);
             }
             wave_sync();
           }
@@ -1179,15 +1218,15 @@ __device__ __forceinline__ void react_body(uint64_t praw) {
           const double I = 0.5 * gsum<G>(part, lane);
           const double sqI = sqrt(I);
           if (live) {
-            gam = fabs(Zr) > 1e-10 ? exp((-Zr * Zr * sqI * A / (1.0 + a0r * B * sqI) + Bd * I) * PFX_LOG_TO_LN)
-                                   : 1.0;
-            lng = log(gam);
+            lng = fabs(Zr) > 1e-10 ? ln_of_exp((-Zr * Zr * sqI * A / (1.0 + a0r * B * sqI) + Bd * I) * PFX_LOG_TO_LN) : 0.0;
+            gam = exp(lng);
           }
           for (int cc = r; cc < M; cc += G) {
             const double z = LD(L.o_cZ, cc);
             SD(S.gsec, cc) = fabs(z) > 1e-10
-                                 ? exp((-z * z * sqI * A / (1.0 + LD(L.o_ca0, cc) * B * sqI) + Bd * I) * PFX_LOG_TO_LN)
-                                 : 1.0;
+                                 ? ln_of_exp((-z * z * sqI * A / (1.0 + LD(L.o_ca0, cc) * B * sqI) + Bd * I) *
+                                             PFX_LOG_TO_LN)
+                                 : 0.0;
           }
         }
       }
@@ -1197,6 +1236,7 @@ __device__ __forceinline__ void react_body(uint64_t praw) {
           if (P.guess_mode == PFX_GUESS_ARRAY || P.guess_mode == PFX_GUESS_ARRAY_FALLBACK)
             m = SD(S.xb, r);
           else if (P.guess_mode == PFX_GUESS_DEFAULT) m = P.default_guess;
+          lnm = log(m);
         }
       }
     }
@@ -1208,23 +1248,15 @@ __device__ __forceinline__ void react_body(uint64_t praw) {
     // ---------------------------------------------------------------
     // RTotal, phase A: complex molalities, complex c computed by lane c % G
     if (active) {
-      SD(S.la, r) = live ? log(m) + lng : 0.0;
+      SD(S.la, r) = live ? (kLn ? lnm : log(m)) + lng : 0.0;
       SD(S.mv, r) = m;
-      SD(S.im, r) = 1.0 / m;
+      if (!kLn) SD(S.im, r) = 1.0 / m;
     }
     wave_sync();
     if (active) {
       for (int cc = r; cc < M; cc += G) {
-        double lnQK = SD(S.lnK, cc);
-        const int nS = L.S;
-#pragma unroll
-        for (int s = 0; s < PFX_MAX_RXN_SPEC; s++) {
-          if (s < nS) {
-            const int sp = LI(L.o_cspec, cc * nS + s);
-            if (sp >= 0) lnQK += LD(L.o_cnu, cc * nS + s) * SD(S.la, sp);
-          }
-        }
-        SD(S.C, cc) = exp(lnQK) / SD(S.gsec, cc);
+        const double lnQK = ln_iap(SD(S.lnK, cc), (int)L.o_cpk, (int)L.o_cnu, cc, L.packs, S.la);
+        SD(S.C, cc) = exp((kLn ? lnQK : ln_of_exp(lnQK)) - SD(S.gsec, cc));
       }
     }
     wave_sync();
@@ -1234,17 +1266,17 @@ __device__ __forceinline__ void react_body(uint64_t praw) {
     // (not needed at the previous state, whose complexes only feed the
     // activity update)
     double row[G];
+    double own = 1.0;
     double col[MODE == PFX_MODE_GI ? G : 1];
     double Tsum = 0.0, absum = 0.0;
     const double den_kg_per_L = SD(S.cs, 3) * 1.0e-3;
     if (active && !(MODE == PFX_MODE_REACT && phase == 0)) {
       double diag = 0.0;
       const int maxdeg = L.maxdeg;
-#pragma unroll 2
+#pragma unroll 4
       for (int e = 0; e < maxdeg; e++) {
-        const int cc = LI(L.o_adj_c, e * G + r);
         const double nu = LD(L.o_adj_nu, e * G + r);
-        const double Cc = SD(S.C, cc);
+        const double Cc = LD(S.C + LI(L.o_adj_c, e * G + r), 0);
         Tsum += nu * Cc;
         absum += fabs(nu) * Cc;
         diag += nu * nu * Cc;
@@ -1261,21 +1293,25 @@ __device__ __forceinline__ void react_body(uint64_t praw) {
           const uint2 w = *(const uint2 *)(smem + L.o_offq_c + (s * G + r) * 8);
           const double2 fa = *(const double2 *)(smem + L.o_offq_coef + ((2 * s) * G + r) * 16);
           const double2 fb = *(const double2 *)(smem + L.o_offq_coef + ((2 * s + 1) * G + r) * 16);
-          a0 += fa.x * SD(S.C, (int)(w.x & 0xffffu));
-          a1 += fa.y * SD(S.C, (int)(w.x >> 16));
-          a2 += fb.x * SD(S.C, (int)(w.y & 0xffffu));
-          a3 += fb.y * SD(S.C, (int)(w.y >> 16));
+          a0 += fa.x * LD(S.C + (int)(w.x & 0xffffu), 0);
+          a1 += fa.y * LD(S.C + (int)(w.x >> 16), 0);
+          a2 += fb.x * LD(S.C + (int)(w.y & 0xffffu), 0);
+          a3 += fb.y * LD(S.C + (int)(w.y >> 16), 0);
         }
         row[4 * q] = a0;
         row[4 * q + 1] = a1;
         row[4 * q + 2] = a2;
         row[4 * q + 3] = a3;
       }
+      // dT/d ln m (kLn) or dT/dm, weighted by the accumulation in a step's or
+      // an evaluation's rows (on a grid later).  The lane's own entry stays
+      // apart, in `own`, until sorption has added to it: one select per column.
+      const double w = (MODE == PFX_MODE_REACT || MODE == PFX_MODE_EVAL)
+                           ? den_kg_per_L * (SD(S.cs, 0) * SD(S.cs, 1) * 1000.0 * SD(S.cs, 2) * P.inv_dt)
+                           : den_kg_per_L;
+      own = live ? (kLn ? m + diag : 1.0 + diag * SD(S.im, r)) * w : 1.0;
 #pragma unroll
-      for (int k = 0; k < G; k++)
-        row[k] = (k == r) ? (live ? 1.0 + diag * SD(S.im, k) : 1.0) : row[k] * SD(S.im, k);
-#pragma unroll
-      for (int k = 0; k < G; k++) row[k] = live ? row[k] * den_kg_per_L : row[k];
+      for (int k = 0; k < G; k++) row[k] = kLn ? row[k] * w : row[k] * SD(S.im, k) * w;
       tot_out = (m + Tsum) * den_kg_per_L;
     }
     PFX_PT(3);
@@ -1284,7 +1320,10 @@ __device__ __forceinline__ void react_body(uint64_t praw) {
       // neighbours' rows in this cell's column: each a scalar times dT/dm
       if (active && live) P.tot_eval_out[cell * N + r] = tot_out;
 #pragma unroll
-      for (int k = 0; k < G; k++) col[k] = P.col_scale ? row[k] * SD(S.mv, k) : row[k];
+      for (int k = 0; k < G; k++) {
+        const double d = k == r ? own : row[k];
+        col[k] = P.col_scale ? d : d / SD(S.mv, k);
+      }
       gi_store_blocks<G, XM>(Pp, col, r, active, gi_stage, 0, 6);
     }
     if (MODE == PFX_MODE_REACT && active && phase == 0) {
@@ -1315,12 +1354,13 @@ __device__ __forceinline__ void react_body(uint64_t praw) {
     // On a grid the rows take the accumulation's weight, with the cell's own
     // share of its faces' fluxes, before sorption and minerals add to them.
     if (MODE == PFX_MODE_GI && active) {
-      const double w = psv_t / dt + SD(S.gc, 6);
+      const double w = psv_t * P.inv_dt + SD(S.gc, 6);
 #pragma unroll
-      for (int k = 0; k < G; k++) row[k] = live ? row[k] * w : row[k];
+      for (int k = 0; k < G; k++) row[k] = row[k] * w;
+      own = live ? own * w : own;
     }
     if (active && R > 0 && (need_ionx || ionx_final)) {
-      const double ionx_w = need_ionx ? vol / dt : 0.0;
+      const double ionx_w = need_ionx ? vol * P.inv_dt : 0.0;
       for (int q = 0; q < R; q++) {
         const int role = live ? LI(L.o_ionx_role, q * G + r) : -1;
         const double kq = live ? LD(L.o_ionx_k, q * G + r) : 0.0;
@@ -1333,27 +1373,28 @@ __device__ __forceinline__ void react_body(uint64_t praw) {
           const double ref_Z = LD(L.o_Z, rl);
           const double ref_k = L.ionx_ref_k[q];
           double ref_X = ref_Z * SD(S.ionx, q) / omega;
-          double KDj = ref_X / (ref_k * ref_conc);
+          const double rk = ref_k * ref_conc;
+          double KDj = ref_X / rk;
           bool one_more = false;
           const double zratio = Zr / ref_Z;
+          const double ka = kq * m * gam;
           int iit = 0;
           for (;;) {
             if (++iit > 20000) {  // reference: error stop (reaction.F90:4382-4385)
               cell_flag = PFX_CELL_MAX_ITERATIONS;
               break;
             }
-            ref_X = KDj * (ref_k * ref_conc);
-            if (role > 0) X = kq * m * gam * pow_ratio(KDj, zratio);
-            else X = role == 0 ? ref_X : 0.0;
+            ref_X = KDj * rk;
+            X = role > 0 ? ka * pow_ratio(KDj, zratio) : (role == 0 ? ref_X : 0.0);
             const double total = gsum<G>(X, lane);
-            double dres = gsum<G>(role > 0 ? X / KDj * Zr : 0.0, lane);
-            dres = dres / ref_Z + (ref_k * ref_conc);
-            const double res = 1.0 - total;
             if (one_more) break;
-            const double delta = res / dres;
+            // KD is held at 1e-40 or more, so its reciprocal needs no scaling;
+            // the derivative may be as small as a vanishing reference cation
+            const double dsum = gsum<G>(role > 0 ? X * Zr : 0.0, lane);
+            const double delta = (1.0 - total) / (dsum * fast_rcp(KDj * ref_Z) + rk);
             KDj = KDj + delta;
             KDj = fmax(KDj, 1e-40);
-            if (fabs(delta / KDj) < 1e-12) one_more = true;
+            if (fabs(delta) < 1e-12 * KDj) one_more = true;
           }
           SD(S.ionx, q) = ref_X * omega / ref_Z;
         } else {
@@ -1366,16 +1407,14 @@ __device__ __forceinline__ void react_body(uint64_t praw) {
         const double t2 = Zr / sumZX;
         Sr += t1;
         if (need_ionx) {
-          // row[] is scaled by psv_t/dt later, but on a grid
-          const double wscale = MODE == PFX_MODE_GI ? ionx_w : ionx_w / (live ? psv_t / dt : 1.0);
           SD(S.xb, r) = X;
           wave_sync();
+          // the lane's own entry as w1 (1 - t2 X): where one cation fills the
+          // exchanger the difference is all that keeps the matrix regular
+          const double w1 = t1 * ionx_w, w2 = -w1 * t2;
+          own += w1 * (1.0 - t2 * X) * (kLn ? 1.0 : SD(S.im, r));
 #pragma unroll
-          for (int k = 0; k < G; k++) {
-            const double Xk = SD(S.xb, k);
-            const double d = (k == r) ? t1 * (1.0 - (t2 * Xk)) : (-t1) * t2 * Xk;
-            row[k] += d * SD(S.im, k) * wscale;
-          }
+          for (int k = 0; k < G; k++) row[k] += w2 * SD(S.xb, k) * (kLn ? 1.0 : SD(S.im, k));
           wave_sync();
         } else if (MODE == PFX_MODE_EQUIL && P.has_sorb) {
           SD(S.xb, r) = X;
@@ -1413,17 +1452,16 @@ __device__ __forceinline__ void react_body(uint64_t praw) {
           dres = res / m * inv_n;
         }
         Sr += res;
-        // row[] is scaled by psv_t/dt later, but on a grid
-        const double jw = !need_ionx ? 1.0 : (MODE == PFX_MODE_GI ? vol / dt : vol / psv_t);
+        if (need_ionx) own += dres * (kLn ? m : 1.0) * vol * P.inv_dt;
+        else if (MODE == PFX_MODE_EQUIL && P.has_sorb) {
 #pragma unroll
-        for (int k = 0; k < G; k++) {
-          if (k == r) {
-            if (need_ionx) row[k] += dres * jw;
-            else if (MODE == PFX_MODE_EQUIL && P.has_sorb) srow[k] += dres;
-          }
+          for (int k = 0; k < G; k++)
+            if (k == r) srow[k] += dres;
         }
       }
     }
+#pragma unroll
+    for (int k = 0; k < G; k++) row[k] = k == r ? own : row[k];
     sorb_out = Sr;
     PFX_PT(4);
 
@@ -1437,15 +1475,12 @@ __device__ __forceinline__ void react_body(uint64_t praw) {
     int use_log = L.use_log;
     if (MODE == PFX_MODE_AUX && active) finish = true;
     if ((MODE == PFX_MODE_REACT || kEval) && active) {
-      // accumulation (mol/s) and its derivative: the dt-consistent form
-      if (MODE != PFX_MODE_GI)
-#pragma unroll
-        for (int k = 0; k < G; k++) row[k] = live ? row[k] * (psv_t / dt) : row[k];
+      // accumulation (mol/s): the dt-consistent form
       if (live) {
         const double fixed = SD(S.fx, r);
-        Rr = (psv_t * tot_out + (L.sorb_any ? Sr * vol : 0.0)) / dt - fixed / dt;
+        Rr = (psv_t * tot_out + (L.sorb_any ? Sr * vol : 0.0) - fixed) * P.inv_dt;
         const double psv = SD(S.cs, 0) * SD(S.cs, 1) * SD(S.cs, 3) * vol;
-        scale = psv * (m + absum) / dt + fabs(Sr) * vol / dt + fabs(fixed) / dt;
+        scale = (psv * (m + absum) + fabs(Sr) * vol + fabs(fixed)) * P.inv_dt;
       }
       // kinetic minerals (group-uniform rates, row-local residual/Jacobian)
       const bool fd_jac = kEval && L.num_jac;
@@ -1455,11 +1490,7 @@ __device__ __forceinline__ void react_body(uint64_t praw) {
                                           !fell_back) ? P.fallback_after : P.max_iterations));
       const bool capped_jac = (P.jac_flags & PFX_JAC_CAPPED_QK) && (kEval || att_it < PFX_JAC_CAPPED_ITERS);
       for (int k = 0; k < K; k++) {
-        double lnQK = SD(S.mlnK, k);
-        for (int s = 0; s < L.S; s++) {
-          const int sp = LI(L.o_mspec, k * L.S + s);
-          if (sp >= 0) lnQK += LD(L.o_mnu, k * L.S + s) * SD(S.la, sp);
-        }
+        const double lnQK = ln_iap(SD(S.mlnK, k), (int)L.o_mpk, (int)L.o_mnu, k, L.packs, S.la);
         const double QK = lnQK <= 6.90776 ? exp(lnQK) : 1.0e3;
         const bool temkin = L.mnrl_flags & 8, msf_on = XM && (L.mnrl_flags & 32);
         const double msf = msf_on ? LD(L.o_mmsf, k) : 1.0;
@@ -1491,11 +1522,11 @@ __device__ __forceinline__ void react_body(uint64_t praw) {
             }
             if (!fd_jac && !(capped_jac && lnQK > 6.90776)) {
 #pragma unroll
-              for (int kk = 0; kk < G; kk++) row[kk] += f * LD(L.o_mnuG, k * G + kk) * SD(S.im, kk);
+              for (int kk = 0; kk < G; kk++) row[kk] += f * LD(L.o_mnuG, k * G + kk) * (kLn ? 1.0 : SD(S.im, kk));
             }
             if constexpr (XM) {
               if (!fd_jac && (L.mnrl_flags & 16) && LI(L.o_mpn, k) > 0)
-                prefactor_jacobian<G>(Pp, S, k, ImV / rate, nur, row);
+                prefactor_jacobian<G, kLn>(Pp, S, k, ImV / rate, nur, row);
             }
           } else if (r == 0) {
             SD(S.mrate, k) = 0.0;
@@ -1505,7 +1536,7 @@ __device__ __forceinline__ void react_body(uint64_t praw) {
         }
       }
       if (kEval && fd_jac && K > 0) mineral_fd_jacobian<G, XM>(Pp, S, r, live, m, lng, vol, row);
-      rr = gmax<G>(live ? fabs(Rr) / fmax(scale, 1e-300) : 0.0, lane);
+      rr = kEval ? 0.0 : gmax<G>(live ? fabs(Rr) / fmax(scale, 1e-300) : 0.0, lane);
       if (kEval) {
         finish = true;
       } else if (cell_flag != PFX_CELL_CONVERGED) {
@@ -1618,26 +1649,31 @@ __device__ __forceinline__ void react_body(uint64_t praw) {
       // side; they are no pivot candidates before step N and pivot on
       // themselves after it, where every multiplier is zero, so the live
       // rows see exactly the N-step elimination.
-      double b = 0.0;
-      {
+      double b = live ? (floor_pass ? 2.220446049250313e-16 * scale : Rr) : 0.0;
+      double vv = 0.0;
+      if (kLn) {
+        // the unpivoted elimination is indifferent to the rows' scale; the
+        // columns are d / d ln m, divided by m for linear unknowns
+        if (!use_log) {
+#pragma unroll
+          for (int k = 0; k < G; k++) row[k] = live ? row[k] / SD(S.mv, k) : row[k];
+        }
+      } else {
+        // the reference's row equilibration (RSolve, reaction.F90:4851-4862),
+        // on the entries with respect to m
         double mx = 0.0;
 #pragma unroll
         for (int k = 0; k < G; k++) mx = fmax(mx, fabs(row[k]));
         const double norm = live ? 1.0 / fmax(1.0, mx) : 1.0;
-        b = live ? (floor_pass ? 2.220446049250313e-16 * scale : Rr) * norm : 0.0;
+        b *= norm;
         const bool lg = live && use_log;
 #pragma unroll
         for (int k = 0; k < G; k++) {
-          // a multiply by 1 when the columns are not scaled (exact): a
-          // select of the product made the compiler branch around the load
           const double sk = SD(S.mv, k);
           row[k] = row[k] * norm;
           row[k] = row[k] * (lg ? sk : 1.0);
         }
-      }
-      double vv = 0.0;
-      {
-        double mx = 0.0;
+        mx = 0.0;
 #pragma unroll
         for (int k = 0; k < G; k++) mx = fmax(mx, fabs(row[k]));
         vv = mx > 0.0 ? 1.0 / mx : 0.0;
@@ -1729,7 +1765,7 @@ __device__ __forceinline__ void react_body(uint64_t praw) {
     // ---------------------------------------------------------------
     PFX_PT(7);
     // Newton update (reaction.F90:3454-3470; constraint form :1806-1826)
-    double mnew = m, rel = 0.0;
+    double mnew = m, lnew = lnm, rel = 0.0;
     if (MODE == PFX_MODE_REACT && active && !finish && !redo && floor_pass) {
       // the solve gave the resolution of the free ions at the candidate: a
       // waiting step within twice it is rounding noise, and the iterate is
@@ -1743,11 +1779,18 @@ __device__ __forceinline__ void react_body(uint64_t praw) {
         status = PFX_CELL_MAX_ITERATIONS;
       } else {
         mnew = m_cand;
+        if (kLn) lnew = l_cand;
         rel = rel_cand;
       }
     } else if ((MODE == PFX_MODE_REACT || MODE == PFX_MODE_EQUIL) && active && !finish && !redo) {
       const double mprev = m;
-      if (use_log) {
+      if (kLn && use_log) {
+        const double u = copysign(1.0, upd) * fmin(fabs(upd), L.max_dlnC);
+        if (live) {
+          mnew = m * exp(-u);
+          lnew = lnm - u;
+        }
+      } else if (use_log) {
         const double u = copysign(1.0, upd) * fmin(fabs(upd), L.max_dlnC);
         if (live) mnew = m * exp(-u);
       } else {
@@ -1756,6 +1799,7 @@ __device__ __forceinline__ void react_body(uint64_t praw) {
         if (MODE == PFX_MODE_EQUIL ? (min_ratio <= 1.0) : (min_ratio < 1.0)) upd = upd * min_ratio * 0.99;
         if (live) mnew = m - upd;
       }
+      if (kLn && !use_log) lnew = live ? log(mnew) : 0.0;
       rel = gmax<G>(live ? fabs((mnew - mprev) / mprev) : 0.0, lane);
       if (MODE == PFX_MODE_REACT && candidate) {
         // step test: the change this step would make, enlarged by
@@ -1773,6 +1817,7 @@ __device__ __forceinline__ void react_body(uint64_t praw) {
           floor_pass = true;
           rel_cand = rel;
           m_cand = mnew;
+          l_cand = lnew;
         } else if (it >= it_cap) {
           finish = true;
           status = PFX_CELL_MAX_ITERATIONS;
@@ -1781,6 +1826,7 @@ __device__ __forceinline__ void react_body(uint64_t praw) {
     }
     if ((MODE == PFX_MODE_REACT || MODE == PFX_MODE_EQUIL) && active && !finish && !redo && !floor_pass) {
       m = mnew;
+      lnm = lnew;
       it++;
       if (MODE == PFX_MODE_REACT) {
         last_change = rel;
@@ -1835,7 +1881,7 @@ __device__ __forceinline__ void react_body(uint64_t praw) {
     if constexpr (MODE == PFX_MODE_GI) {
       // the cell's own block: the evaluated Jacobian, its faces' share in it
 #pragma unroll
-      for (int k = 0; k < G; k++) col[k] = P.col_scale ? row[k] * SD(S.mv, k) : row[k];
+      for (int k = 0; k < G; k++) col[k] = P.col_scale ? row[k] : row[k] / SD(S.mv, k);
       gi_store_blocks<G, XM>(Pp, col, r, active, gi_stage, 6, 7);
     }
 
@@ -1851,7 +1897,7 @@ __device__ __forceinline__ void react_body(uint64_t praw) {
           if (MODE == PFX_MODE_EVAL)
 #pragma unroll
             for (int k = 0; k < G; k++)
-              if (k < N) P.jac_out[c * N * N + (long long)k * N + r] = row[k];
+              if (k < N) P.jac_out[c * N * N + (long long)k * N + r] = row[k] / SD(S.mv, k);
         }
         // the mineral rates at this iterate (the last evaluation of a
         // global-implicit solve leaves those of its solution)
@@ -1869,7 +1915,8 @@ __device__ __forceinline__ void react_body(uint64_t praw) {
           if (L.sorb_any && P.total_sorb) P.total_sorb[c * N + r] = sorb_out;
         }
         for (int cc = r; cc < M; cc += G) {
-          if (P.sec_act_coef) P.sec_act_coef[c * M + cc] = SD(S.gsec, cc);
+          if (P.sec_act_coef && !(MODE == PFX_MODE_REACT && L.act_freq == PFX_ACT_OFF))
+            P.sec_act_coef[c * M + cc] = exp(SD(S.gsec, cc));
           if (P.sec_molal) P.sec_molal[c * M + cc] = SD(S.C, cc);
         }
         if (MODE == PFX_MODE_REACT && P.mnrl_rate)
