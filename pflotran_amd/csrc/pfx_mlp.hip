@@ -2,11 +2,15 @@
 // a multilayer perceptron whose matrix products run on the gfx950 matrix
 // cores (v_mfma_f32_16x16x32_bf16: BF16 operands, FP32 accumulation).
 //
-//  * training: a tiled BF16 GEMM (64x64 block tile, 2x2 MFMA tiles per
-//    wavefront) with fused bias/GELU epilogue for the forward pass, the same
-//    GEMM on transposed operands (split-K, atomic FP32 accumulation) for the
-//    weight gradients, elementwise GELU backward, and Adam on FP32 master
-//    weights;
+//  * training, layers up to CHAIN_WIDTH wide: three launches a step.  One
+//    kernel takes 16 rows through every layer forward and back with the
+//    activations in LDS, one forms all layers' weight and bias gradients over
+//    slices of the batch, one adds the slices, applies Adam to the FP32 master
+//    weights and rewrites their BF16 fragments;
+//  * training, wider layers: a tiled BF16 GEMM (64x64 block tile, 2x2 MFMA
+//    tiles per wavefront) with fused bias/GELU epilogue for the forward pass,
+//    the same GEMM on transposed operands (split-K, atomic FP32 accumulation)
+//    for the weight gradients, elementwise GELU backward, then the same Adam;
 //  * inference: one fused kernel per 64 cells that computes the features,
 //    keeps every activation in LDS (BF16, two ping-pong buffers), streams
 //    the weights from L2 in the exact MFMA fragment order (pre-swizzled,
@@ -42,13 +46,19 @@ struct pfx_mlp {
   float *W[MLP_MAX_LAYERS], *b[MLP_MAX_LAYERS];  // FP32 master, W[l]: [dims[l+1]][dims[l]]
   float *gW[MLP_MAX_LAYERS], *gb[MLP_MAX_LAYERS];
   float *mW[MLP_MAX_LAYERS], *vW[MLP_MAX_LAYERS], *mb[MLP_MAX_LAYERS], *vb[MLP_MAX_LAYERS];
-  uint4 *Wsw[MLP_MAX_LAYERS];  // BF16 weights in MFMA fragment order (inference)
-  bool sw_dirty;
+  uint4 *Wsw[MLP_MAX_LAYERS];   // BF16 weights in MFMA fragment order
+  uint4 *Wtsw[MLP_MAX_LAYERS];  // the same of W transposed (backward chain)
+  bool sw_dirty;                // W set by the caller since the fragments were written
   float *in_shift, *in_scale, *out_shift, *out_scale;
   int bmax;
-  float *Z[MLP_MAX_LAYERS];      // pre-activations [bmax][dims[l+1]]
+  float *Z[MLP_MAX_LAYERS];      // pre-activations (or gelu' there) [bmax][dims[l+1]]
   float *A[MLP_MAX_LAYERS + 1];  // activations; A[0] is the caller's input
-  float *dA, *dZ;                // [bmax][max width]
+  // layers up to CHAIN_WIDTH wide (Z, A and dZl rows padded to 4 floats)
+  float *dZl[MLP_MAX_LAYERS];  // [bmax][dims[l+1]]
+  float *part;                 // gradient slices [gsplit(bmax)][params]
+  float *lpart;                // loss of each 16 rows
+  // wider layers
+  float *dA, *dZ;  // [bmax][max width]
   float *loss;
   int adam_step;
 };
@@ -77,6 +87,13 @@ __device__ __forceinline__ unsigned short f2bf(float f) {
 __device__ __forceinline__ float gelu(float z) { return 0.5f * z * (1.0f + erff(z * 0.70710678118654752f)); }
 __device__ __forceinline__ float gelu_grad(float z) {
   return 0.5f * (1.0f + erff(z * 0.70710678118654752f)) + z * 0.39894228040143268f * expf(-0.5f * z * z);
+}
+
+// gelu and its derivative from one erf
+__device__ __forceinline__ float gelu_both(float z, float &slope) {
+  const float e = 1.0f + erff(z * 0.70710678118654752f);
+  slope = 0.5f * e + z * 0.39894228040143268f * expf(-0.5f * z * z);
+  return 0.5f * z * e;
 }
 
 __device__ __forceinline__ bf16x8 as_frag(uint4 u) { return __builtin_bit_cast(bf16x8, u); }
@@ -240,7 +257,9 @@ struct mt_tensors {
 };
 struct mt_adam {
   float *w[MT_MAX], *g[MT_MAX], *m[MT_MAX], *v[MT_MAX];
-  long n[MT_MAX];
+  unsigned short *sw[MT_MAX], *swt[MT_MAX];  // BF16 fragments of a weight and of its transpose (or null)
+  int K[MT_MAX];                             // row length of a weight
+  long n[MT_MAX], off[MT_MAX];               // elements, first element in a gradient slice
   int count;
 };
 
@@ -252,20 +271,60 @@ __global__ void k_fill_multi(const mt_tensors T, float v) {
   for (long i = blockIdx.x * (long)blockDim.x + threadIdx.x; i < n; i += (long)gridDim.x * blockDim.x) p[i] = v;
 }
 
-// Adam with bias correction over every weight and bias tensor
-__global__ void k_adam_multi(const mt_adam T, float lr, float b1, float b2, float c1, float c2, float eps) {
+// element (r, c) of a matrix in MFMA fragment order (k_swizzle), kts
+// fragments of 32 columns to a row tile
+__device__ __forceinline__ long frag_at(int r, int c, int kts) {
+  return (((long)(r >> 4) * kts + (c >> 5)) * 64 + (r & 15) + 2 * (c & 24)) * 8 + (c & 7);
+}
+
+// Gradients from their nsplit slices (0: they are there already), then Adam
+// with bias correction over every weight and bias tensor (adam), which also
+// rewrites the BF16 fragments that the products read.  blockIdx.y == count
+// adds the rows' losses in a fixed order.  Bound by the slices' reads (9 MB at
+// 145k parameters in 16 slices).  A fill, the atomics, Adam and the fragments'
+// rewrite were four passes over the parameters.
+__global__ __launch_bounds__(256) void k_update(const mt_adam T, int nsplit, const float *part, long stride,
+                                                const float *lpart, int nlpart, float *loss, int adam, float lr,
+                                                float b1, float b2, float c1, float c2, float eps) {
   const int t = blockIdx.y;
-  if (t >= T.count) return;
-  float *w = T.w[t], *m = T.m[t], *v = T.v[t];
-  const float *g = T.g[t];
+  if (t >= T.count) {
+    if (blockIdx.x > 0) return;
+    __shared__ float red[4];
+    float l = 0.f;
+    for (int i = threadIdx.x; i < nlpart; i += 256) l += lpart[i];
+    for (int o = 32; o > 0; o >>= 1) l += __shfl_xor(l, o);
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = l;
+    __syncthreads();
+    if (threadIdx.x == 0) *loss = (red[0] + red[1]) + (red[2] + red[3]);
+    return;
+  }
+  float *w = T.w[t], *g = T.g[t], *m = T.m[t], *v = T.v[t];
   const long n = T.n[t];
+  const int K = T.K[t], N = (int)(n / K);
   for (long i = blockIdx.x * (long)blockDim.x + threadIdx.x; i < n; i += (long)gridDim.x * blockDim.x) {
-    const float gi = g[i];
+    float gi;
+    if (nsplit > 0) {
+      const float *q = part + T.off[t] + i;
+      gi = 0.f;
+#pragma unroll 8
+      for (int k = 0; k < nsplit; k++) gi += q[k * stride];
+      g[i] = gi;
+    } else {
+      gi = g[i];
+    }
+    if (!adam) continue;
     const float mi = b1 * m[i] + (1.f - b1) * gi;
     const float vi = b2 * v[i] + (1.f - b2) * gi * gi;
     m[i] = mi;
     v[i] = vi;
-    w[i] -= lr * (mi / c1) / (sqrtf(vi / c2) + eps);
+    const float wi = w[i] - lr * (mi / c1) / (sqrtf(vi / c2) + eps);
+    w[i] = wi;
+    if (T.sw[t]) {
+      const int r = (int)i / K, c = (int)i - r * K;
+      const unsigned short h = f2bf(wi);
+      T.sw[t][frag_at(r, c, (K + 31) / 32)] = h;
+      if (T.swt[t]) T.swt[t][frag_at(c, r, (N + 31) / 32)] = h;
+    }
   }
 }
 
@@ -277,9 +336,10 @@ inline unsigned mt_blocks(const long *n, int count) {
   return (unsigned)std::min<long>(1024, (mx + 255) / 256);
 }
 
-// W[N][K] FP32 -> BF16 fragments: uint4 index ((nt * Kp/32 + kt) * 64 + lane)
-// holds W[nt*16 + lane%16][kt*32 + 8*(lane/16) + 0..7] (zero outside)
-__global__ void k_swizzle(const float *W, int N, int K, int Np, int Kp, uint4 *out) {
+// W(n, k) = W[n*sn + k*sk] FP32 -> BF16 fragments: uint4 index
+// ((nt * Kp/32 + kt) * 64 + lane) holds W(nt*16 + lane%16,
+// kt*32 + 8*(lane/16) + 0..7) (zero outside)
+__global__ void k_swizzle(const float *W, int N, int K, long sn, long sk, int Np, int Kp, uint4 *out) {
   const long i = blockIdx.x * (long)blockDim.x + threadIdx.x;
   const int kts = Kp / 32;
   const long total = (long)(Np / 16) * kts * 64;
@@ -291,7 +351,7 @@ __global__ void k_swizzle(const float *W, int N, int K, int Np, int Kp, uint4 *o
   const int k0 = kt * 32 + 8 * (lane >> 4);
   unsigned short v[8];
 #pragma unroll
-  for (int q = 0; q < 8; q++) v[q] = f2bf((n < N && k0 + q < K) ? W[(long)n * K + k0 + q] : 0.0f);
+  for (int q = 0; q < 8; q++) v[q] = f2bf((n < N && k0 + q < K) ? W[n * sn + (k0 + q) * sk] : 0.0f);
   uint4 u;
   u.x = v[0] | ((unsigned)v[1] << 16);
   u.y = v[2] | ((unsigned)v[3] << 16);
@@ -448,6 +508,327 @@ __global__ __launch_bounds__(256) void k_surrogate_guess(const mlp_dev D, int64_
 }
 
 // ---------------------------------------------------------------------------
+// training and plain inference of layers up to CHAIN_WIDTH wide
+//
+// With 16 rows to a workgroup, batches of some thousand rows fill the chip
+// and one launch carries them through all layers: the weight fragments come
+// from L2 (each workgroup reads all of them, 290 KB at 40-256-256-256-15), the
+// activations stay in LDS as the BF16 operands they are rounded to anyway.
+// One training step of 4096 rows at that shape took 23 launches and 231 us with
+// the tiled products, whose scalar loads of transposed operands and passes
+// between layers bound them; now 27 us (this kernel) + 19 (weight gradients) + 7
+// (update).  What is left here is latency: 20 us remain with a single
+// fragment a product, 25 without the GELUs.
+// Widths (three equal hidden layers, 4096 rows, step / plain inference), tiled
+// products -> this: 256: 231 -> 53 / 70 -> 12 us, 512: 399 -> 114 / 168 -> 24,
+// 768: 720 -> 199 / 334 -> 39.  CHAIN_WIDTH is where the two buffers of 16 rows
+// reach 64 KB of LDS.
+constexpr int CHAIN_WIDTH = 960;
+constexpr int CHAIN_ROWS = 16;
+constexpr int CHAIN_THREADS = 512;
+
+struct mlp_chain {
+  int nlayers, B, astr;  // astr: LDS row stride (BF16 elements)
+  int dims[MLP_MAX_LAYERS + 1];
+  const uint4 *Wsw[MLP_MAX_LAYERS], *Wtsw[MLP_MAX_LAYERS];
+  const float *b[MLP_MAX_LAYERS];
+  float *S[MLP_MAX_LAYERS], *A[MLP_MAX_LAYERS + 1], *dZ[MLP_MAX_LAYERS];  // gelu', activations
+  const float *X, *T;
+  float *Y, *lpart;
+  float inv;
+};
+
+__host__ __device__ inline int ld4(int n) { return (n + 3) & ~3; }
+
+// D = W x in^T for 16 rows: W in fragments (rt row tiles of kts fragments), in
+// [16][astr] BF16 in LDS.  Each wavefront takes two row tiles at a time, the
+// fragments of 8 steps of k in flight together (the loop waits on L2, not on the
+// matrix cores).  Rows of D are walked up to the next multiple of 32, so that
+// the next product's operand is padded with what epi writes there.
+// pre(n0) loads four values ahead of the product, epi(n0, acc, those) takes
+// rows n0..n0+3 of this lane's column (row lane % 16 of the batch tile).
+template <class PRE, class EPI>
+__device__ __forceinline__ void chain_product(const uint4 *__restrict__ W, int nrows, int kts,
+                                              const unsigned short *in, int astr, PRE pre, EPI epi) {
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const int rt = (nrows + 15) / 16, ft = (nrows + 31) / 32 * 2;
+  const unsigned short *ap = in + (lane & 15) * astr + 8 * (lane >> 4);
+  for (int nt = 2 * w; nt < ft; nt += 2 * (CHAIN_THREADS / 64)) {
+    const uint4 *p0 = W + (long)min(nt, rt - 1) * kts * 64 + lane;
+    const uint4 *p1 = W + (long)min(nt + 1, rt - 1) * kts * 64 + lane;
+    const int n0 = nt * 16 + 4 * (lane >> 4);
+    f32x4 a0 = {0.f, 0.f, 0.f, 0.f}, a1 = {0.f, 0.f, 0.f, 0.f};
+    const f32x4 x0 = pre(n0), x1 = pre(n0 + 16);
+    for (int k0 = 0; k0 < kts; k0 += 8) {
+      uint4 f0[8], f1[8];
+#pragma unroll
+      for (int q = 0; q < 8; q++) {
+        const int kt = min(k0 + q, kts - 1);
+        f0[q] = p0[kt * 64];
+        f1[q] = p1[kt * 64];
+      }
+#pragma unroll
+      for (int q = 0; q < 8; q++)
+        if (k0 + q < kts) {
+          const bf16x8 b = as_frag(*(const uint4 *)&ap[(k0 + q) * 32]);
+          a0 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_frag(f0[q]), b, a0, 0, 0, 0);
+          a1 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_frag(f1[q]), b, a1, 0, 0, 0);
+        }
+    }
+    epi(n0, a0, x0);
+    epi(n0 + 16, a1, x1);
+  }
+}
+
+// Forward pass of 16 rows; TRAIN: also the loss and dZ of every layer,
+// with the activations and gelu' kept for it and for the weight gradients.
+template <bool TRAIN>
+__global__ __launch_bounds__(CHAIN_THREADS) void k_chain(const mlp_chain D) {
+  extern __shared__ __attribute__((aligned(16))) unsigned short chain_lds[];
+  __shared__ float lred[CHAIN_THREADS / 64];
+  const int t = threadIdx.x, lane = t & 63;
+  const int r0 = blockIdx.x * CHAIN_ROWS;
+  const long row = r0 + (lane & 15);
+  const bool live = row < D.B;
+  const int L = D.nlayers, astr = D.astr;
+  unsigned short *in = chain_lds, *out = chain_lds + CHAIN_ROWS * astr;
+  {
+    const int K = D.dims[0], Kp = roundup(K, 32);
+    for (int i = t; i < CHAIN_ROWS * Kp; i += CHAIN_THREADS) {
+      const int r = i / Kp, k = i - r * Kp;
+      in[r * astr + k] = f2bf((r0 + r < D.B && k < K) ? D.X[(long)(r0 + r) * K + k] : 0.0f);
+    }
+  }
+  __syncthreads();
+  auto put = [&](int n0, const f32x4 v) {
+    uint2 u;
+    u.x = f2bf(v[0]) | ((unsigned)f2bf(v[1]) << 16);
+    u.y = f2bf(v[2]) | ((unsigned)f2bf(v[3]) << 16);
+    *(uint2 *)&out[(lane & 15) * astr + n0] = u;
+  };
+  float loss = 0.f;
+  for (int l = 0; l < L; l++) {
+    const int K = D.dims[l], N = D.dims[l + 1], ld = ld4(N);
+    const float *bl = D.b[l];
+    const bool last = l == L - 1;
+    auto bias = [&](int n0) {
+      f32x4 v;
+#pragma unroll
+      for (int q = 0; q < 4; q++) v[q] = bl[min(n0 + q, N - 1)];
+      return v;
+    };
+    if (!last) {
+      float *Sl = D.S[l], *Al = D.A[l + 1];
+      chain_product(D.Wsw[l], N, roundup(K, 32) / 32, in, astr, bias, [&](int n0, f32x4 acc, f32x4 bv) {
+        f32x4 s, a;
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+          const float z = n0 + q < N ? acc[q] + bv[q] : 0.0f;
+          float slope = 0.f;
+          a[q] = TRAIN ? gelu_both(z, slope) : gelu(z);
+          s[q] = slope;
+        }
+        if (TRAIN && live && n0 < ld) {
+          *(f32x4 *)&Sl[row * ld + n0] = s;
+          *(f32x4 *)&Al[row * ld + n0] = a;
+        }
+        put(n0, a);
+      });
+    } else {
+      chain_product(D.Wsw[l], N, roundup(K, 32) / 32, in, astr, bias, [&](int n0, f32x4 acc, f32x4 bv) {
+        f32x4 dz = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int q = 0; q < 4; q++)
+          if (live && n0 + q < N) {
+            const float y = acc[q] + bv[q];
+            if (TRAIN) {
+              const float d = y - D.T[row * N + n0 + q];
+              dz[q] = 2.0f * d * D.inv;
+              loss += d * d * D.inv;
+            } else {
+              D.Y[row * N + n0 + q] = y;
+            }
+          }
+        if (TRAIN) {
+          if (live && n0 < ld) *(f32x4 *)&D.dZ[l][row * ld + n0] = dz;
+          put(n0, dz);
+        }
+      });
+    }
+    __syncthreads();
+    unsigned short *x = in;
+    in = out;
+    out = x;
+  }
+  if (!TRAIN) return;
+  for (int l = L - 1; l > 0; l--) {
+    // dA = dZ W; dZ of layer l-1 = dA * gelu'(Z), the slopes as this thread wrote them
+    const int K = D.dims[l], N = D.dims[l + 1], ld = ld4(K);
+    const float *Sl = D.S[l - 1];
+    float *dZl = D.dZ[l - 1];
+    chain_product(
+        D.Wtsw[l], K, roundup(N, 32) / 32, in, astr,
+        [&](int n0) {
+          return live && n0 < ld ? *(const f32x4 *)&Sl[row * ld + n0] : (f32x4){0.f, 0.f, 0.f, 0.f};
+        },
+        [&](int n0, f32x4 acc, f32x4 s) {
+          f32x4 dz;
+#pragma unroll
+          for (int q = 0; q < 4; q++) dz[q] = live && n0 + q < K ? acc[q] * s[q] : 0.0f;
+          if (live && n0 < ld) *(f32x4 *)&dZl[row * ld + n0] = dz;
+          put(n0, dz);
+        });
+    __syncthreads();
+    unsigned short *x = in;
+    in = out;
+    out = x;
+  }
+  for (int o = 32; o > 0; o >>= 1) loss += __shfl_xor(loss, o);
+  if (lane == 0) lred[t >> 6] = loss;
+  __syncthreads();
+  if (t == 0) {
+    float l = 0.f;
+    for (int i = 0; i < CHAIN_THREADS / 64; i++) l += lred[i];
+    D.lpart[blockIdx.x] = l;
+  }
+}
+
+// dW[n][k] = sum_b dZ[b][n] A[b][k] and db[n] = sum_b dZ[b][n] of every layer
+// in one launch: blockIdx.y is a 64x64 tile of some layer's dW, blockIdx.x a
+// slice of the batch (so that the tiles that read the same rows share an
+// XCD's L2 cache), whose sums go to a slice of their own.  Atomics into one
+// copy took longer than the products (a step of 12.9 us a layer, most of it
+// 16 additions to each address).
+// The operands' contiguous side is n (k) and their product's is b, so a thread
+// turns an 8 x 4 block in registers on its way to LDS; the loads of the next 128
+// rows are in flight while the matrix cores work.
+// Bound by the operands' reads (every row once for each of the other operand's
+// tiles, 84 MB of which L2 keeps most): 32.5 us at 4096 rows of 40-256-256-256-15
+// with the tile fastest over the grid, 30 with the slice fastest, 19 with
+// four workgroups on a CU (128 registers) instead of two, whose 640 did not fit
+// the chip at once.  Layer by layer with atomics: 99 us.
+constexpr int GT = 64;            // tile of dW
+constexpr int GB = 128;           // rows of the batch to a stage
+constexpr int GSTR = GB + 8;      // LDS row stride (BF16 elements)
+
+struct grad_layer {
+  const float *dZ, *A;
+  int N, K, ldz, lda, tk, tile0;
+  long off;  // of dW in a slice, db behind it
+  int avec;  // rows of A are 16-byte aligned
+};
+struct grad_args {
+  grad_layer l[MLP_MAX_LAYERS];
+  int nlayers, B, chunk;
+  long params;
+  float *part;
+};
+
+__device__ __forceinline__ void grad_load(f32x4 (&v)[8], const float *p, int ld, int n0, int n, bool vec, int b0,
+                                          int b1) {
+#pragma unroll
+  for (int q = 0; q < 8; q++) {
+    const int b = b0 + q;
+    v[q] = (f32x4){0.f, 0.f, 0.f, 0.f};
+    if (b >= b1) continue;
+    const float *r = p + (long)b * ld;
+    if (vec) {
+      if (n0 < ld) v[q] = *(const f32x4 *)&r[n0];
+    } else {
+#pragma unroll
+      for (int j = 0; j < 4; j++)
+        if (n0 + j < n) v[q][j] = r[n0 + j];
+    }
+  }
+}
+
+__device__ __forceinline__ void grad_stage(const f32x4 (&v)[8], unsigned short *s, int mg, int kg) {
+#pragma unroll
+  for (int j = 0; j < 4; j++) {
+    uint4 u;
+    u.x = f2bf(v[0][j]) | ((unsigned)f2bf(v[1][j]) << 16);
+    u.y = f2bf(v[2][j]) | ((unsigned)f2bf(v[3][j]) << 16);
+    u.z = f2bf(v[4][j]) | ((unsigned)f2bf(v[5][j]) << 16);
+    u.w = f2bf(v[6][j]) | ((unsigned)f2bf(v[7][j]) << 16);
+    *(uint4 *)&s[(4 * mg + j) * GSTR + 8 * kg] = u;
+  }
+}
+
+__global__ __launch_bounds__(256, 4) void k_weight_grad(const grad_args G) {
+  __shared__ __attribute__((aligned(16))) unsigned short Zs[GT * GSTR], As[GT * GSTR];
+  __shared__ float red[16][GT];
+  int li = 0;
+  for (int l = 1; l < G.nlayers; l++)
+    if ((int)blockIdx.y >= G.l[l].tile0) li = l;
+  const grad_layer &P = G.l[li];
+  const int tile = blockIdx.y - P.tile0;
+  const int n0 = tile / P.tk * GT, k0 = tile % P.tk * GT;
+  const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+  const int mg = t & 15, kg = t >> 4;
+  const int wm = (wave >> 1) * 32, wn = (wave & 1) * 32;
+  const int beg = blockIdx.x * G.chunk, end = min(G.B, beg + G.chunk);
+  const bool avec = P.avec != 0, want_db = k0 == 0;
+  f32x4 acc[2][2], db = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int i = 0; i < 2; i++)
+#pragma unroll
+    for (int j = 0; j < 2; j++) acc[i][j] = (f32x4){0.f, 0.f, 0.f, 0.f};
+  f32x4 vz[8], va[8];
+  grad_load(vz, P.dZ, P.ldz, n0 + 4 * mg, P.N, true, beg + 8 * kg, end);
+  grad_load(va, P.A, P.lda, k0 + 4 * mg, P.K, avec, beg + 8 * kg, end);
+  for (int b = beg; b < end; b += GB) {
+    if (b > beg) __syncthreads();
+    grad_stage(vz, Zs, mg, kg);
+    grad_stage(va, As, mg, kg);
+    if (want_db) {
+#pragma unroll
+      for (int q = 0; q < 8; q++) db += vz[q];
+    }
+    __syncthreads();
+    if (b + GB < end) {
+      grad_load(vz, P.dZ, P.ldz, n0 + 4 * mg, P.N, true, b + GB + 8 * kg, end);
+      grad_load(va, P.A, P.lda, k0 + 4 * mg, P.K, avec, b + GB + 8 * kg, end);
+    }
+    const int fr = lane & 15, fk = (lane >> 4) * 8;
+#pragma unroll
+    for (int kk = 0; kk < GB; kk += 32) {
+      bf16x8 af[2], bfr[2];
+#pragma unroll
+      for (int i = 0; i < 2; i++) {
+        af[i] = as_frag(*(const uint4 *)&Zs[(wm + 16 * i + fr) * GSTR + kk + fk]);
+        bfr[i] = as_frag(*(const uint4 *)&As[(wn + 16 * i + fr) * GSTR + kk + fk]);
+      }
+#pragma unroll
+      for (int i = 0; i < 2; i++)
+#pragma unroll
+        for (int j = 0; j < 2; j++)
+          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af[i], bfr[j], acc[i][j], 0, 0, 0);
+    }
+  }
+  float *out = G.part + blockIdx.x * G.params + P.off;
+#pragma unroll
+  for (int i = 0; i < 2; i++)
+#pragma unroll
+    for (int j = 0; j < 2; j++)
+#pragma unroll
+      for (int q = 0; q < 4; q++) {
+        const int n = n0 + wm + 16 * i + 4 * (lane >> 4) + q;
+        const int k = k0 + wn + 16 * j + (lane & 15);
+        if (n < P.N && k < P.K) out[(long)n * P.K + k] = acc[i][j][q];
+      }
+  if (want_db) {
+    *(f32x4 *)&red[kg][4 * mg] = db;
+    __syncthreads();
+    if (t < GT && n0 + t < P.N) {
+      float s = 0.f;
+#pragma unroll
+      for (int i = 0; i < 16; i++) s += red[i][t];
+      out[(long)P.N * P.K + n0 + t] = s;
+    }
+  }
+}
+
+// ---------------------------------------------------------------------------
 int launch_gemm(int epi, int M, int N, int K, const float *A, long sam, long sak, const float *B, long sbn,
                 long sbk, float *C, long ldc, const float *bias, float *Zout, int ksplit, hipStream_t s) {
   if (M <= 0 || N <= 0) return 0;
@@ -509,164 +890,121 @@ int refresh_swizzled(pfx_mlp *m, hipStream_t s) {
     const int N = m->dims[l + 1], K = m->dims[l];
     const int Np = roundup(N, 16), Kp = roundup(K, 32);
     const long total = (long)(Np / 16) * (Kp / 32) * 64;
-    hipLaunchKernelGGL(k_swizzle, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, s, m->W[l], N, K, Np, Kp,
-                       m->Wsw[l]);
+    hipLaunchKernelGGL(k_swizzle, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, s, m->W[l], N, K, (long)K, 1L,
+                       Np, Kp, m->Wsw[l]);
+    if (m->Wtsw[l]) {
+      const int Nq = roundup(N, 32), Kq = roundup(K, 16);
+      const long tt = (long)(Kq / 16) * (Nq / 32) * 64;
+      hipLaunchKernelGGL(k_swizzle, dim3((unsigned)((tt + 255) / 256)), dim3(256), 0, s, m->W[l], K, N, 1L, (long)K,
+                         Kq, Nq, m->Wtsw[l]);
+    }
   }
   MCHK(hipGetLastError());
   m->sw_dirty = false;
   return 0;
 }
 
-bool fused_shape_ok(const pfx_mlp *m, int N) {
-  if (m->nlayers < 2 || m->dims[0] > 256) return false;
-  for (int l = 1; l < m->nlayers; l++)
-    if (m->dims[l] % 64 != 0 || m->dims[l] > 256) return false;
-  const int nout = m->dims[m->nlayers];
-  return nout >= 1 && nout <= 16 && N <= nout;
-}
+bool chain_ok(const pfx_mlp *m) { return max_width(m) <= CHAIN_WIDTH; }
 
-}  // namespace
-
-// ---------------------------------------------------------------------------
-extern "C" int pfx_mlp_create(int32_t nlayers, const int32_t *dims, int32_t batch_max, uint64_t seed,
-                              pfx_mlp **out) {
-  if (!out) return PFX_E_ARG;
-  *out = nullptr;
-  if (!dims || nlayers < 1 || nlayers > MLP_MAX_LAYERS || batch_max < 1) return PFX_E_ARG;
-  for (int l = 0; l <= nlayers; l++)
-    if (dims[l] < 1 || dims[l] > 4096) return PFX_E_ARG;
-  pfx_mlp *m = new pfx_mlp();
-  memset(m, 0, sizeof(*m));
-  m->nlayers = nlayers;
-  for (int l = 0; l <= nlayers; l++) m->dims[l] = dims[l];
-  m->bmax = batch_max;
-  // uniform(-a, a) initial weights, a = sqrt(3 / fan_in), from a seeded
-  // splitmix64 stream on the host; zero biases
-  uint64_t st = seed;
-  auto next = [&]() {
-    st += 0x9E3779B97F4A7C15ull;
-    uint64_t z = st;
-    z = (z ^ (z >> 30)) * 0xBF58476D1CE4E5B9ull;
-    z = (z ^ (z >> 27)) * 0x94D049BB133111EBull;
-    return z ^ (z >> 31);
-  };
-  int rc = 0;
-  for (int l = 0; l < nlayers && !rc; l++) {
-    const long nw = (long)dims[l + 1] * dims[l];
-    const int nb = dims[l + 1];
-    std::vector<float> w(nw), bz(nb, 0.0f);
-    const double a = std::sqrt(3.0 / dims[l]);
-    for (long i = 0; i < nw; i++) w[i] = (float)(((double)(next() >> 11) * 0x1.0p-53 * 2.0 - 1.0) * a);
-    const long nsw = (long)(roundup(dims[l + 1], 16) / 16) * (roundup(dims[l], 32) / 32) * 64;
-    if (hipMalloc(&m->W[l], nw * 4) != hipSuccess || hipMalloc(&m->b[l], nb * 4) != hipSuccess ||
-        hipMalloc(&m->gW[l], nw * 4) != hipSuccess || hipMalloc(&m->gb[l], nb * 4) != hipSuccess ||
-        hipMalloc(&m->mW[l], nw * 4) != hipSuccess || hipMalloc(&m->vW[l], nw * 4) != hipSuccess ||
-        hipMalloc(&m->mb[l], nb * 4) != hipSuccess || hipMalloc(&m->vb[l], nb * 4) != hipSuccess ||
-        hipMalloc(&m->Wsw[l], nsw * sizeof(uint4)) != hipSuccess ||
-        hipMalloc(&m->Z[l], (long)batch_max * nb * 4) != hipSuccess ||
-        hipMalloc(&m->A[l + 1], (long)batch_max * nb * 4) != hipSuccess) {
-      rc = PFX_E_NOMEM;
-      break;
-    }
-    if (hipMemcpy(m->W[l], w.data(), nw * 4, hipMemcpyHostToDevice) != hipSuccess ||
-        hipMemcpy(m->b[l], bz.data(), nb * 4, hipMemcpyHostToDevice) != hipSuccess)
-      rc = PFX_E_DEVICE;
-    if (!rc) rc = fill(m->mW[l], nw, 0.f, 0);
-    if (!rc) rc = fill(m->vW[l], nw, 0.f, 0);
-    if (!rc) rc = fill(m->mb[l], nb, 0.f, 0);
-    if (!rc) rc = fill(m->vb[l], nb, 0.f, 0);
-    if (!rc) rc = fill(m->gW[l], nw, 0.f, 0);
-    if (!rc) rc = fill(m->gb[l], nb, 0.f, 0);
-  }
-  const int md = max_width(m);
-  if (!rc && (hipMalloc(&m->dA, (long)batch_max * md * 4) != hipSuccess ||
-              hipMalloc(&m->dZ, (long)batch_max * md * 4) != hipSuccess || hipMalloc(&m->loss, 4) != hipSuccess ||
-              hipMalloc(&m->in_shift, dims[0] * 4) != hipSuccess ||
-              hipMalloc(&m->in_scale, dims[0] * 4) != hipSuccess ||
-              hipMalloc(&m->out_shift, dims[nlayers] * 4) != hipSuccess ||
-              hipMalloc(&m->out_scale, dims[nlayers] * 4) != hipSuccess))
-    rc = PFX_E_NOMEM;
-  if (!rc) rc = fill(m->in_shift, dims[0], 0.f, 0);
-  if (!rc) rc = fill(m->in_scale, dims[0], 1.f, 0);
-  if (!rc) rc = fill(m->out_shift, dims[nlayers], 0.f, 0);
-  if (!rc) rc = fill(m->out_scale, dims[nlayers], 1.f, 0);
-  if (!rc && hipDeviceSynchronize() != hipSuccess) rc = PFX_E_DEVICE;
-  m->sw_dirty = true;
-  if (rc) {
-    pfx_mlp_destroy(m);
-    return rc;
-  }
-  *out = m;
-  return 0;
-}
-
-extern "C" int pfx_mlp_destroy(pfx_mlp *m) {
-  if (!m) return PFX_E_ARG;
+// batch rows B through all layers: Y (T null) or gradients' operands
+int launch_chain(pfx_mlp *m, const float *X, const float *T, float *Y, int B, hipStream_t s) {
+  int rc = refresh_swizzled(m, s);
+  if (rc) return rc;
+  mlp_chain D;
+  memset(&D, 0, sizeof(D));
+  D.nlayers = m->nlayers;
+  D.B = B;
+  D.astr = roundup(max_width(m), 32) + 8;
+  for (int l = 0; l <= m->nlayers; l++) D.dims[l] = m->dims[l];
   for (int l = 0; l < m->nlayers; l++) {
-    (void)hipFree(m->W[l]);
-    (void)hipFree(m->b[l]);
-    (void)hipFree(m->gW[l]);
-    (void)hipFree(m->gb[l]);
-    (void)hipFree(m->mW[l]);
-    (void)hipFree(m->vW[l]);
-    (void)hipFree(m->mb[l]);
-    (void)hipFree(m->vb[l]);
-    (void)hipFree(m->Wsw[l]);
-    (void)hipFree(m->Z[l]);
-    (void)hipFree(m->A[l + 1]);
+    D.Wsw[l] = m->Wsw[l], D.Wtsw[l] = m->Wtsw[l], D.b[l] = m->b[l];
+    D.S[l] = m->Z[l], D.A[l + 1] = m->A[l + 1], D.dZ[l] = m->dZl[l];
   }
-  (void)hipFree(m->dA);
-  (void)hipFree(m->dZ);
-  (void)hipFree(m->loss);
-  (void)hipFree(m->in_shift);
-  (void)hipFree(m->in_scale);
-  (void)hipFree(m->out_shift);
-  (void)hipFree(m->out_scale);
-  delete m;
+  D.X = X, D.T = T, D.Y = Y, D.lpart = m->lpart;
+  D.inv = 1.0f / (float)((long)B * m->dims[m->nlayers]);
+  const unsigned grid = (unsigned)((B + CHAIN_ROWS - 1) / CHAIN_ROWS);
+  const size_t lds = (size_t)2 * CHAIN_ROWS * D.astr * sizeof(unsigned short);
+  if (T) hipLaunchKernelGGL(k_chain<true>, dim3(grid), dim3(CHAIN_THREADS), lds, s, D);
+  else hipLaunchKernelGGL(k_chain<false>, dim3(grid), dim3(CHAIN_THREADS), lds, s, D);
+  MCHK(hipGetLastError());
   return 0;
 }
 
-extern "C" int pfx_mlp_params(pfx_mlp *m, int32_t which, int32_t layer, float *host, int32_t to_device) {
-  if (!m || !host) return PFX_E_ARG;
-  if (which == 4) {
-    const int ni = m->dims[0], no = m->dims[m->nlayers];
-    float *dst[4] = {m->in_shift, m->in_scale, m->out_shift, m->out_scale};
-    const int len[4] = {ni, ni, no, no};
-    long off = 0;
-    for (int q = 0; q < 4; q++) {
-      if (to_device) MCHK(hipMemcpy(dst[q], host + off, len[q] * 4, hipMemcpyHostToDevice));
-      else MCHK(hipMemcpy(host + off, dst[q], len[q] * 4, hipMemcpyDeviceToHost));
-      off += len[q];
-    }
-    return 0;
+long param_count(const pfx_mlp *m) {
+  long n = 0;
+  for (int l = 0; l < m->nlayers; l++) n += (long)m->dims[l + 1] * (m->dims[l] + 1);
+  return n;
+}
+
+// Slices of the batch in the weight gradients: about 1024 workgroups (4 on a
+// CU, as many as LDS and registers admit), of at least one stage of rows each
+// and at most 16, beyond which the slices' traffic outweighs.
+int grad_split(const pfx_mlp *m, int B) {
+  int tiles = 0;
+  for (int l = 0; l < m->nlayers; l++) tiles += ((m->dims[l + 1] + GT - 1) / GT) * ((m->dims[l] + GT - 1) / GT);
+  return std::max(1, std::min({1024 / tiles, 16, (B + GB - 1) / GB}));
+}
+
+int launch_weight_grad(pfx_mlp *m, const float *X, int B, int nsplit, hipStream_t s) {
+  grad_args G;
+  memset(&G, 0, sizeof(G));
+  G.nlayers = m->nlayers;
+  G.B = B;
+  G.chunk = roundup((B + nsplit - 1) / nsplit, 32);
+  G.params = param_count(m);
+  G.part = m->part;
+  int tiles = 0;
+  long off = 0;
+  for (int l = 0; l < m->nlayers; l++) {
+    grad_layer &P = G.l[l];
+    P.N = m->dims[l + 1], P.K = m->dims[l];
+    P.dZ = m->dZl[l], P.ldz = ld4(P.N);
+    P.A = l ? m->A[l] : X, P.lda = l ? ld4(P.K) : P.K;
+    P.avec = l > 0 || (P.K % 4 == 0 && (uintptr_t)X % 16 == 0);
+    P.tk = (P.K + GT - 1) / GT;
+    P.tile0 = tiles, P.off = off;
+    tiles += P.tk * ((P.N + GT - 1) / GT);
+    off += (long)P.N * (P.K + 1);
   }
-  if (layer < 0 || layer >= m->nlayers || which < 0 || which > 3) return PFX_E_ARG;
-  float *p = which == 0 ? m->W[layer] : which == 1 ? m->b[layer] : which == 2 ? m->gW[layer] : m->gb[layer];
-  const long n = (which == 0 || which == 2) ? (long)m->dims[layer + 1] * m->dims[layer] : m->dims[layer + 1];
-  if (to_device) {
-    MCHK(hipMemcpy(p, host, n * 4, hipMemcpyHostToDevice));
-    if (which <= 1) m->sw_dirty = true;
-  } else {
-    MCHK(hipMemcpy(host, p, n * 4, hipMemcpyDeviceToHost));
-  }
+  hipLaunchKernelGGL(k_weight_grad, dim3((unsigned)nsplit, (unsigned)tiles), dim3(256), 0, s, G);
+  MCHK(hipGetLastError());
   return 0;
 }
 
-extern "C" int pfx_mlp_forward(pfx_mlp *m, const float *X, int64_t B, float *Y, void *stream) {
-  if (!m || B < 0 || (B > 0 && (!X || !Y))) return PFX_E_ARG;
-  hipStream_t s = (hipStream_t)stream;
-  for (int64_t b0 = 0; b0 < B; b0 += m->bmax) {
-    const int nb = (int)((B - b0) < m->bmax ? (B - b0) : m->bmax);
-    int rc = forward(m, X + b0 * m->dims[0], nb, Y + b0 * m->dims[m->nlayers], false, s);
-    if (rc) return rc;
+struct adam_rates {
+  float lr, b1, b2, eps;
+};
+
+// gradients from nsplit slices (0: in place), loss from nlpart parts, and
+// the Adam update if rates are given
+int launch_update(pfx_mlp *m, int nsplit, int nlpart, const adam_rates *r, hipStream_t s) {
+  mt_adam T{};
+  long off = 0;
+  for (int l = 0; l < m->nlayers; l++) {
+    const int N = m->dims[l + 1], K = m->dims[l];
+    T.w[T.count] = m->W[l], T.g[T.count] = m->gW[l], T.m[T.count] = m->mW[l], T.v[T.count] = m->vW[l];
+    T.sw[T.count] = (unsigned short *)m->Wsw[l], T.swt[T.count] = (unsigned short *)m->Wtsw[l];
+    T.K[T.count] = K, T.off[T.count] = off;
+    T.n[T.count++] = (long)N * K;
+    T.w[T.count] = m->b[l], T.g[T.count] = m->gb[l], T.m[T.count] = m->mb[l], T.v[T.count] = m->vb[l];
+    T.K[T.count] = 1, T.off[T.count] = off + (long)N * K;
+    T.n[T.count++] = N;
+    off += (long)N * (K + 1);
   }
+  float c1 = 1.f, c2 = 1.f;
+  if (r) {
+    m->adam_step++;
+    c1 = 1.0f - powf(r->b1, (float)m->adam_step), c2 = 1.0f - powf(r->b2, (float)m->adam_step);
+  }
+  hipLaunchKernelGGL(k_update, dim3(mt_blocks(T.n, T.count), (unsigned)(T.count + (nlpart > 0))), dim3(256), 0, s, T,
+                     nsplit, m->part, off, m->lpart, nlpart, m->loss, r ? 1 : 0, r ? r->lr : 0.f, r ? r->b1 : 0.f,
+                     r ? r->b2 : 0.f, c1, c2, r ? r->eps : 0.f);
+  MCHK(hipGetLastError());
   return 0;
 }
 
-extern "C" int pfx_mlp_gradients(pfx_mlp *m, const float *X, const float *T, int32_t B, float *loss_out,
-                                 void *stream) {
-  if (!m || !X || !T || B < 1 || B > m->bmax) return PFX_E_ARG;
-  hipStream_t s = (hipStream_t)stream;
+// gradients by tiled products, layer by layer (layers wider than CHAIN_WIDTH)
+int wide_gradients(pfx_mlp *m, const float *X, const float *T, int B, hipStream_t s) {
   const int L = m->nlayers;
   m->A[0] = (float *)X;
   int rc = forward(m, X, B, m->A[L], true, s);
@@ -709,6 +1047,186 @@ extern "C" int pfx_mlp_gradients(pfx_mlp *m, const float *X, const float *T, int
       MCHK(hipGetLastError());
     }
   }
+  return 0;
+}
+
+bool fused_shape_ok(const pfx_mlp *m, int N) {
+  if (m->nlayers < 2 || m->dims[0] > 256) return false;
+  for (int l = 1; l < m->nlayers; l++)
+    if (m->dims[l] % 64 != 0 || m->dims[l] > 256) return false;
+  const int nout = m->dims[m->nlayers];
+  return nout >= 1 && nout <= 16 && N <= nout;
+}
+
+}  // namespace
+
+// ---------------------------------------------------------------------------
+extern "C" int pfx_mlp_create(int32_t nlayers, const int32_t *dims, int32_t batch_max, uint64_t seed,
+                              pfx_mlp **out) {
+  if (!out) return PFX_E_ARG;
+  *out = nullptr;
+  if (!dims || nlayers < 1 || nlayers > MLP_MAX_LAYERS || batch_max < 1) return PFX_E_ARG;
+  for (int l = 0; l <= nlayers; l++)
+    if (dims[l] < 1 || dims[l] > 4096) return PFX_E_ARG;
+  pfx_mlp *m = new pfx_mlp();
+  memset(m, 0, sizeof(*m));
+  m->nlayers = nlayers;
+  for (int l = 0; l <= nlayers; l++) m->dims[l] = dims[l];
+  m->bmax = batch_max;
+  // uniform(-a, a) initial weights, a = sqrt(3 / fan_in), from a seeded
+  // splitmix64 stream on the host; zero biases
+  uint64_t st = seed;
+  auto next = [&]() {
+    st += 0x9E3779B97F4A7C15ull;
+    uint64_t z = st;
+    z = (z ^ (z >> 30)) * 0xBF58476D1CE4E5B9ull;
+    z = (z ^ (z >> 27)) * 0x94D049BB133111EBull;
+    return z ^ (z >> 31);
+  };
+  int rc = 0;
+  const bool chain = chain_ok(m);
+  for (int l = 0; l < nlayers && !rc; l++) {
+    const long nw = (long)dims[l + 1] * dims[l];
+    const int nb = dims[l + 1];
+    std::vector<float> w(nw), bz(nb, 0.0f);
+    const double a = std::sqrt(3.0 / dims[l]);
+    for (long i = 0; i < nw; i++) w[i] = (float)(((double)(next() >> 11) * 0x1.0p-53 * 2.0 - 1.0) * a);
+    const long nsw = (long)(roundup(dims[l + 1], 16) / 16) * (roundup(dims[l], 32) / 32) * 64;
+    const long nswt = (long)(roundup(dims[l], 16) / 16) * (roundup(dims[l + 1], 32) / 32) * 64;
+    if (hipMalloc(&m->W[l], nw * 4) != hipSuccess || hipMalloc(&m->b[l], nb * 4) != hipSuccess ||
+        hipMalloc(&m->gW[l], nw * 4) != hipSuccess || hipMalloc(&m->gb[l], nb * 4) != hipSuccess ||
+        hipMalloc(&m->mW[l], nw * 4) != hipSuccess || hipMalloc(&m->vW[l], nw * 4) != hipSuccess ||
+        hipMalloc(&m->mb[l], nb * 4) != hipSuccess || hipMalloc(&m->vb[l], nb * 4) != hipSuccess ||
+        hipMalloc(&m->Wsw[l], nsw * sizeof(uint4)) != hipSuccess ||
+        hipMalloc(&m->Z[l], (long)batch_max * ld4(nb) * 4) != hipSuccess ||
+        hipMalloc(&m->A[l + 1], (long)batch_max * ld4(nb) * 4) != hipSuccess ||
+        (chain && (hipMalloc(&m->dZl[l], (long)batch_max * ld4(nb) * 4) != hipSuccess ||
+                   hipMalloc(&m->Wtsw[l], nswt * sizeof(uint4)) != hipSuccess))) {
+      rc = PFX_E_NOMEM;
+      break;
+    }
+    if (hipMemcpy(m->W[l], w.data(), nw * 4, hipMemcpyHostToDevice) != hipSuccess ||
+        hipMemcpy(m->b[l], bz.data(), nb * 4, hipMemcpyHostToDevice) != hipSuccess)
+      rc = PFX_E_DEVICE;
+    if (!rc) rc = fill(m->mW[l], nw, 0.f, 0);
+    if (!rc) rc = fill(m->vW[l], nw, 0.f, 0);
+    if (!rc) rc = fill(m->mb[l], nb, 0.f, 0);
+    if (!rc) rc = fill(m->vb[l], nb, 0.f, 0);
+    if (!rc) rc = fill(m->gW[l], nw, 0.f, 0);
+    if (!rc) rc = fill(m->gb[l], nb, 0.f, 0);
+  }
+  const int md = max_width(m);
+  if (!rc && chain &&
+      (hipMalloc(&m->part, grad_split(m, batch_max) * param_count(m) * 4) != hipSuccess ||
+       hipMalloc(&m->lpart, ((long)batch_max + CHAIN_ROWS - 1) / CHAIN_ROWS * 4) != hipSuccess))
+    rc = PFX_E_NOMEM;
+  if (!rc && !chain &&
+      (hipMalloc(&m->dA, (long)batch_max * md * 4) != hipSuccess ||
+       hipMalloc(&m->dZ, (long)batch_max * md * 4) != hipSuccess))
+    rc = PFX_E_NOMEM;
+  if (!rc && (hipMalloc(&m->loss, 4) != hipSuccess ||
+              hipMalloc(&m->in_shift, dims[0] * 4) != hipSuccess ||
+              hipMalloc(&m->in_scale, dims[0] * 4) != hipSuccess ||
+              hipMalloc(&m->out_shift, dims[nlayers] * 4) != hipSuccess ||
+              hipMalloc(&m->out_scale, dims[nlayers] * 4) != hipSuccess))
+    rc = PFX_E_NOMEM;
+  if (!rc) rc = fill(m->in_shift, dims[0], 0.f, 0);
+  if (!rc) rc = fill(m->in_scale, dims[0], 1.f, 0);
+  if (!rc) rc = fill(m->out_shift, dims[nlayers], 0.f, 0);
+  if (!rc) rc = fill(m->out_scale, dims[nlayers], 1.f, 0);
+  if (!rc && hipDeviceSynchronize() != hipSuccess) rc = PFX_E_DEVICE;
+  m->sw_dirty = true;
+  if (rc) {
+    pfx_mlp_destroy(m);
+    return rc;
+  }
+  *out = m;
+  return 0;
+}
+
+extern "C" int pfx_mlp_destroy(pfx_mlp *m) {
+  if (!m) return PFX_E_ARG;
+  for (int l = 0; l < m->nlayers; l++) {
+    (void)hipFree(m->W[l]);
+    (void)hipFree(m->b[l]);
+    (void)hipFree(m->gW[l]);
+    (void)hipFree(m->gb[l]);
+    (void)hipFree(m->mW[l]);
+    (void)hipFree(m->vW[l]);
+    (void)hipFree(m->mb[l]);
+    (void)hipFree(m->vb[l]);
+    (void)hipFree(m->Wsw[l]);
+    (void)hipFree(m->Wtsw[l]);
+    (void)hipFree(m->dZl[l]);
+    (void)hipFree(m->Z[l]);
+    (void)hipFree(m->A[l + 1]);
+  }
+  (void)hipFree(m->part);
+  (void)hipFree(m->lpart);
+  (void)hipFree(m->dA);
+  (void)hipFree(m->dZ);
+  (void)hipFree(m->loss);
+  (void)hipFree(m->in_shift);
+  (void)hipFree(m->in_scale);
+  (void)hipFree(m->out_shift);
+  (void)hipFree(m->out_scale);
+  delete m;
+  return 0;
+}
+
+extern "C" int pfx_mlp_params(pfx_mlp *m, int32_t which, int32_t layer, float *host, int32_t to_device) {
+  if (!m || !host) return PFX_E_ARG;
+  if (which == 4) {
+    const int ni = m->dims[0], no = m->dims[m->nlayers];
+    float *dst[4] = {m->in_shift, m->in_scale, m->out_shift, m->out_scale};
+    const int len[4] = {ni, ni, no, no};
+    long off = 0;
+    for (int q = 0; q < 4; q++) {
+      if (to_device) MCHK(hipMemcpy(dst[q], host + off, len[q] * 4, hipMemcpyHostToDevice));
+      else MCHK(hipMemcpy(host + off, dst[q], len[q] * 4, hipMemcpyDeviceToHost));
+      off += len[q];
+    }
+    return 0;
+  }
+  if (layer < 0 || layer >= m->nlayers || which < 0 || which > 3) return PFX_E_ARG;
+  float *p = which == 0 ? m->W[layer] : which == 1 ? m->b[layer] : which == 2 ? m->gW[layer] : m->gb[layer];
+  const long n = (which == 0 || which == 2) ? (long)m->dims[layer + 1] * m->dims[layer] : m->dims[layer + 1];
+  if (to_device) {
+    MCHK(hipMemcpy(p, host, n * 4, hipMemcpyHostToDevice));
+    if (which <= 1) m->sw_dirty = true;
+  } else {
+    MCHK(hipMemcpy(host, p, n * 4, hipMemcpyDeviceToHost));
+  }
+  return 0;
+}
+
+extern "C" int pfx_mlp_forward(pfx_mlp *m, const float *X, int64_t B, float *Y, void *stream) {
+  if (!m || B < 0 || (B > 0 && (!X || !Y))) return PFX_E_ARG;
+  hipStream_t s = (hipStream_t)stream;
+  for (int64_t b0 = 0; b0 < B; b0 += m->bmax) {
+    const int nb = (int)((B - b0) < m->bmax ? (B - b0) : m->bmax);
+    const float *x = X + b0 * m->dims[0];
+    float *y = Y + b0 * m->dims[m->nlayers];
+    int rc = chain_ok(m) ? launch_chain(m, x, nullptr, y, nb, s) : forward(m, x, nb, y, false, s);
+    if (rc) return rc;
+  }
+  return 0;
+}
+
+// gradients of a batch, and the Adam update if rates are given
+static int gradients(pfx_mlp *m, const float *X, const float *T, int32_t B, float *loss_out, const adam_rates *r,
+                     hipStream_t s) {
+  if (!m || !X || !T || B < 1 || B > m->bmax) return PFX_E_ARG;
+  int rc;
+  if (chain_ok(m)) {
+    const int nsplit = grad_split(m, B);
+    if ((rc = launch_chain(m, X, T, nullptr, B, s))) return rc;
+    if ((rc = launch_weight_grad(m, X, B, nsplit, s))) return rc;
+    if ((rc = launch_update(m, nsplit, (B + CHAIN_ROWS - 1) / CHAIN_ROWS, r, s))) return rc;
+  } else {
+    if ((rc = wide_gradients(m, X, T, B, s))) return rc;
+    if (r && (rc = launch_update(m, 0, 0, r, s))) return rc;
+  }
   if (loss_out) {
     MCHK(hipMemcpyAsync(loss_out, m->loss, 4, hipMemcpyDeviceToHost, s));
     MCHK(hipStreamSynchronize(s));
@@ -716,30 +1234,21 @@ extern "C" int pfx_mlp_gradients(pfx_mlp *m, const float *X, const float *T, int
   return 0;
 }
 
+extern "C" int pfx_mlp_gradients(pfx_mlp *m, const float *X, const float *T, int32_t B, float *loss_out,
+                                 void *stream) {
+  return gradients(m, X, T, B, loss_out, nullptr, (hipStream_t)stream);
+}
+
 extern "C" int pfx_mlp_adam(pfx_mlp *m, float lr, float beta1, float beta2, float eps, void *stream) {
   if (!m) return PFX_E_ARG;
-  hipStream_t s = (hipStream_t)stream;
-  m->adam_step++;
-  const float c1 = 1.0f - powf(beta1, (float)m->adam_step), c2 = 1.0f - powf(beta2, (float)m->adam_step);
-  mt_adam T{};
-  for (int l = 0; l < m->nlayers; l++) {
-    T.w[T.count] = m->W[l], T.g[T.count] = m->gW[l], T.m[T.count] = m->mW[l], T.v[T.count] = m->vW[l];
-    T.n[T.count++] = (long)m->dims[l + 1] * m->dims[l];
-    T.w[T.count] = m->b[l], T.g[T.count] = m->gb[l], T.m[T.count] = m->mb[l], T.v[T.count] = m->vb[l];
-    T.n[T.count++] = m->dims[l + 1];
-  }
-  hipLaunchKernelGGL(k_adam_multi, dim3(mt_blocks(T.n, T.count), (unsigned)T.count), dim3(256), 0, s, T, lr, beta1,
-                     beta2, c1, c2, eps);
-  MCHK(hipGetLastError());
-  m->sw_dirty = true;
-  return 0;
+  const adam_rates r = {lr, beta1, beta2, eps};
+  return launch_update(m, 0, 0, &r, (hipStream_t)stream);
 }
 
 extern "C" int pfx_mlp_train_step(pfx_mlp *m, const float *X, const float *T, int32_t B, float lr, float *loss_out,
                                   void *stream) {
-  int rc = pfx_mlp_gradients(m, X, T, B, loss_out, stream);
-  if (rc) return rc;
-  return pfx_mlp_adam(m, lr, 0.9f, 0.999f, 1e-8f, stream);
+  const adam_rates r = {lr, 0.9f, 0.999f, 1e-8f};
+  return gradients(m, X, T, B, loss_out, &r, (hipStream_t)stream);
 }
 
 extern "C" int pfx_surrogate_features(pfx_tables *tables, pfx_mlp *m, const pfx_cells *cells, float *X,
