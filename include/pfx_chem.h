@@ -347,8 +347,9 @@ int pfx_tables_destroy(pfx_tables *tables);
 int pfx_tables_tune(pfx_tables *tables, int32_t kernel, int32_t variant);
 
 /* Device time (ms, HIP events) of the launches of the last call made with
-   these tables: ms[0] the per-cell kernel, ms[1] the global-implicit
-   assembly kernel (0 if the call had none).  Profiling aid; no counterpart
+   these tables: ms[0] the per-cell kernel (it writes the blocks of a
+   global-implicit evaluation), ms[1] the global-implicit flux-residual
+   kernel (0 if the call had none).  Profiling aid; no counterpart
    in the reference (its PetscLogEvent timers play this role). */
 int pfx_tables_timing(pfx_tables *tables, double *ms);
 

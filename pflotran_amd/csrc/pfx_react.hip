@@ -3,10 +3,11 @@
 // One cell per group of G lanes (G = 8, 16 or 32 >= N primaries); lane r
 // owns primary species r: its free ion, its total, row r of the local
 // Jacobian and row r of the LU factors.  Reaction tables are staged in LDS
-// once per workgroup; per-cell complex data (concentrations, activity
-// coefficients, log K) live in a per-group LDS slice.  A persistent grid
-// pulls cells from a device work queue in chunks, and a group whose cell
-// converged refills from the queue while the other groups of its wavefront
+// once per workgroup; per-cell complex data (concentrations, ln activity
+// coefficients, log K) live in a per-group LDS slice.  Each wavefront of a
+// persistent grid owns a share of the cells and
+// pulls the rest from a device work queue in chunks, and a group whose cell
+// converged refills while the other groups of its wavefront
 // keep iterating, so cells with 2 or 25 Newton iterations share one launch.
 //
 // Reference path (src/pflotran/):
