@@ -287,9 +287,9 @@ def main():
     try:
         with open(os.path.join(ROOT, "profiles", "pmc_traffic_pfx_react_kernel_1M.json")) as f:
             prof = json.load(f)["pfx_react_kernel<16,0>"]
-        # the counters were read on the uncapped variant: they stand for
-        # the timed kernel only when the autotuner picked that one too
-        if n == 1_000_000 and warm is not None and tab.tune(abi.PFX_KERNEL_REACT) == 0:
+        # the counters were read on one variant: they stand for the timed
+        # kernel only when the autotuner picked that one too
+        if n == 1_000_000 and warm is not None and tab.tune(abi.PFX_KERNEL_REACT) == prof["variant"]:
             traffic = prof["traffic_bytes"]
     except (OSError, KeyError, ValueError):
         traffic = None
