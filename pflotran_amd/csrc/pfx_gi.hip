@@ -8,7 +8,7 @@
 //     species-independent dispersion a scalar times dT/dm each, the blocks of
 //     its column in its neighbours' rows.  No block is written to memory only
 //     to be read again: 128^3 x 15 wrote 7.5 GB of them and read 8.4 GB back
-//     in a second kernel over the block rows, 15.1 ms an evaluation, 10.5 now
+//     in a second kernel over the block rows, 15.1 ms an evaluation, 10.1 now
 //     (26.2 GB of matrix);
 //  2. k_gi_flux_residual adds the upwind fluxes of the totals (TFluxCoef,
 //     TFlux) to the residual.
