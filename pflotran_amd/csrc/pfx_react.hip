@@ -1915,9 +1915,13 @@ __device__ __forceinline__ void react_body(uint64_t praw) {
           if (P.pri_act_coef) P.pri_act_coef[c * N + r] = gam;
           if (L.sorb_any && P.total_sorb) P.total_sorb[c * N + r] = sorb_out;
         }
+        // the complexes' coefficients are kept as logarithms, and the exp of a
+        // given one's log is not it to the last bit: they are written only
+        // where this call formed them
+        const bool formed = MODE == PFX_MODE_REACT ? L.act_freq != PFX_ACT_OFF
+                                                   : (MODE == PFX_MODE_AUX ? P.aux_passes > 0 : true);
         for (int cc = r; cc < M; cc += G) {
-          if (P.sec_act_coef && !(MODE == PFX_MODE_REACT && L.act_freq == PFX_ACT_OFF))
-            P.sec_act_coef[c * M + cc] = exp(SD(S.gsec, cc));
+          if (P.sec_act_coef && formed) P.sec_act_coef[c * M + cc] = exp(SD(S.gsec, cc));
           if (P.sec_molal) P.sec_molal[c * M + cc] = SD(S.C, cc);
         }
         if (MODE == PFX_MODE_REACT && P.mnrl_rate)
