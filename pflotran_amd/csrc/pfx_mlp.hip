@@ -48,7 +48,6 @@ struct pfx_mlp {
   float *mW[MLP_MAX_LAYERS], *vW[MLP_MAX_LAYERS], *mb[MLP_MAX_LAYERS], *vb[MLP_MAX_LAYERS];
   uint4 *Wsw[MLP_MAX_LAYERS];   // BF16 weights in MFMA fragment order
   uint4 *Wtsw[MLP_MAX_LAYERS];  // the same of W transposed (backward chain)
-  bool sw_dirty;                // W set by the caller since the fragments were written
   float *in_shift, *in_scale, *out_shift, *out_scale;
   int bmax;
   float *Z[MLP_MAX_LAYERS];      // pre-activations (or gelu' there) [bmax][dims[l+1]]
@@ -940,23 +939,24 @@ int forward(pfx_mlp *m, const float *X, int B, float *Y, bool keep, hipStream_t 
   return 0;
 }
 
-int refresh_swizzled(pfx_mlp *m, hipStream_t s) {
-  if (!m->sw_dirty) return 0;
-  for (int l = 0; l < m->nlayers; l++) {
-    const int N = m->dims[l + 1], K = m->dims[l];
-    const int Np = roundup(N, 16), Kp = roundup(K, 32);
-    const long total = (long)(Np / 16) * (Kp / 32) * 64;
-    hipLaunchKernelGGL(k_swizzle, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, s, m->W[l], N, K, (long)K, 1L,
-                       Np, Kp, m->Wsw[l]);
-    if (m->Wtsw[l]) {
-      const int Nq = roundup(N, 32), Kq = roundup(K, 16);
-      const long tt = (long)(Kq / 16) * (Nq / 32) * 64;
-      hipLaunchKernelGGL(k_swizzle, dim3((unsigned)((tt + 255) / 256)), dim3(256), 0, s, m->W[l], K, N, 1L, (long)K,
-                         Kq, Nq, m->Wtsw[l]);
-    }
+// The fragments of layer l from W[l].  They follow W wherever it changes: here
+// once the caller has set it, in k_update with the step that moves it.  So every
+// pass may read them as it reads W, on any stream and in a captured graph (a
+// refresh ahead of the next pass would be enqueued on that pass's stream only,
+// and not at all while one is captured or replayed).
+int write_fragments(pfx_mlp *m, int l, hipStream_t s) {
+  const int N = m->dims[l + 1], K = m->dims[l];
+  const int Np = roundup(N, 16), Kp = roundup(K, 32);
+  const long total = (long)(Np / 16) * (Kp / 32) * 64;
+  hipLaunchKernelGGL(k_swizzle, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, s, m->W[l], N, K, (long)K, 1L,
+                     Np, Kp, m->Wsw[l]);
+  if (m->Wtsw[l]) {
+    const int Nq = roundup(N, 32), Kq = roundup(K, 16);
+    const long tt = (long)(Kq / 16) * (Nq / 32) * 64;
+    hipLaunchKernelGGL(k_swizzle, dim3((unsigned)((tt + 255) / 256)), dim3(256), 0, s, m->W[l], K, N, 1L, (long)K,
+                       Kq, Nq, m->Wtsw[l]);
   }
   MCHK(hipGetLastError());
-  m->sw_dirty = false;
   return 0;
 }
 
@@ -964,8 +964,6 @@ bool chain_ok(const pfx_mlp *m) { return max_width(m) <= CHAIN_WIDTH; }
 
 // batch rows B through all layers: Y (T null) or gradients' operands
 int launch_chain(pfx_mlp *m, const float *X, const float *T, float *Y, int B, hipStream_t s) {
-  int rc = refresh_swizzled(m, s);
-  if (rc) return rc;
   mlp_chain D;
   memset(&D, 0, sizeof(D));
   D.nlayers = m->nlayers;
@@ -1170,6 +1168,7 @@ extern "C" int pfx_mlp_create(int32_t nlayers, const int32_t *dims, int32_t batc
     if (!rc) rc = fill(m->vb[l], nb, 0.f, 0);
     if (!rc) rc = fill(m->gW[l], nw, 0.f, 0);
     if (!rc) rc = fill(m->gb[l], nb, 0.f, 0);
+    if (!rc) rc = write_fragments(m, l, 0);
   }
   const int md = max_width(m);
   if (!rc && chain &&
@@ -1191,7 +1190,6 @@ extern "C" int pfx_mlp_create(int32_t nlayers, const int32_t *dims, int32_t batc
   if (!rc) rc = fill(m->out_shift, dims[nlayers], 0.f, 0);
   if (!rc) rc = fill(m->out_scale, dims[nlayers], 1.f, 0);
   if (!rc && hipDeviceSynchronize() != hipSuccess) rc = PFX_E_DEVICE;
-  m->sw_dirty = true;
   if (rc) {
     pfx_mlp_destroy(m);
     return rc;
@@ -1249,7 +1247,11 @@ extern "C" int pfx_mlp_params(pfx_mlp *m, int32_t which, int32_t layer, float *h
   const long n = (which == 0 || which == 2) ? (long)m->dims[layer + 1] * m->dims[layer] : m->dims[layer + 1];
   if (to_device) {
     MCHK(hipMemcpy(p, host, n * 4, hipMemcpyHostToDevice));
-    if (which <= 1) m->sw_dirty = true;
+    if (which == 0) {
+      int rc = write_fragments(m, layer, 0);
+      if (rc) return rc;
+      MCHK(hipStreamSynchronize(0));  // in place when the call returns, as W is
+    }
   } else {
     MCHK(hipMemcpy(host, p, n * 4, hipMemcpyDeviceToHost));
   }
@@ -1332,8 +1334,6 @@ extern "C" int pfx_surrogate_guess(pfx_tables *tables, pfx_mlp *m, pfx_cells *ce
   if (cells->ncells == 0) return 0;
   if (!cells->guess || !cells->total || !cells->pri_molal) return PFX_E_ARG;
   hipStream_t s = (hipStream_t)stream;
-  int rc = refresh_swizzled(m, s);
-  if (rc) return rc;
   mlp_dev D;
   memset(&D, 0, sizeof(D));
   D.nlayers = m->nlayers;
