@@ -506,9 +506,12 @@ int ensure_side(pfx_tables *t) {
   return 0;
 }
 
-int zone_lds(const pfx_tables *t) {
+// LDS of a zone's workgroup in a kernel with (xm) or without the prefactors'
+// cell scalars: in a zoned launch the kernel's, whatever the zone's own network
+// needs, since one prefactor network puts every zone into that instantiation
+int zone_lds(const pfx_tables *t, bool xm) {
   const int G = t->L.G;
-  return (int)(t->L.lds_table_bytes + pfx_scr_bytes(BLOCK, t->L.N, t->L.M, G, t->L.K, tables_xm(t), PFX_MODE_REACT));
+  return (int)(t->L.lds_table_bytes + pfx_scr_bytes(BLOCK, t->L.N, t->L.M, G, t->L.K, xm, PFX_MODE_REACT));
 }
 
 int zones_prepare(int32_t nzones, pfx_tables *const *tables, pfx_cells *cells, const pfx_react_opts *o,
@@ -532,6 +535,8 @@ int zones_prepare(int32_t nzones, pfx_tables *const *tables, pfx_cells *cells, c
   memset(&zs.Z, 0, sizeof(zs.Z));
   zs.Z.nzones = nzones;
   zs.lds = 0;
+  bool xm = false;
+  for (int z = 0; z < nzones; z++) xm = xm || tables_xm(tables[z]);
   double w[PFX_MAX_ZONES], wsum = 0.0;
   for (int z = 0; z < nzones; z++) {
     pfx_tables *t = tables[z];
@@ -544,14 +549,12 @@ int zones_prepare(int32_t nzones, pfx_tables *const *tables, pfx_cells *cells, c
     zs.P[z].fallback_count = t->d_queue + 1;
     zs.n[z] = cells[z].ncells;
     zs.Z.G[z] = t->L.G;
-    zs.lds = std::max<int64_t>(zs.lds, zone_lds(t));
+    zs.lds = std::max<int64_t>(zs.lds, zone_lds(t, xm));
     w[z] = (double)cells[z].ncells * t->L.N * t->L.N;
     wsum += w[z];
   }
   if (zs.lds > kMaxLds) return PFX_E_UNSUP;
   zs.variant = plan && plan->variant >= 0 && plan->variant <= 2 ? plan->variant : 0;
-  bool xm = false;
-  for (int z = 0; z < nzones; z++) xm = xm || tables_xm(tables[z]);
   zs.fn = zones_kernel_ptr(zs.variant, xm);
   if (zs.lds > 64 * 1024) HIPCHK(hipFuncSetAttribute(zs.fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)zs.lds));
   int occ = 0;
@@ -604,7 +607,7 @@ int zones_enqueue(pfx_tables *const *tables, zone_setup &zs, const pfx_kernel_pa
     P2.waves = 0;
     P2.share = 0;
     P2.block0 = 0;
-    const int64_t lds = zone_lds(t);
+    const int64_t lds = zone_lds(t, tables_xm(t));
     const void *fn_piv = kernel_ptr(t->L.G, PFX_MODE_REACT, 0, PFX_LU_PIVOT, tables_xm(t));
     if (lds > 64 * 1024) HIPCHK(hipFuncSetAttribute(fn_piv, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
     const int64_t need = (zs.n[z] + (BLOCK / t->L.G) - 1) / (BLOCK / t->L.G);
