@@ -286,8 +286,10 @@ int resident(int occ, int64_t lds) {
 // 0.84 ms of an evaluation that takes 0.2.  One evaluation per cell is even
 // work, owned whole; Newton cells differ, so half of them stays in the queue to
 // level the wavefronts, in guided sizes (a quarter left four zones of unequal
-// networks 3 % slower, three quarters are no faster).  Owned shares need every
-// workgroup resident from the start: the grid is never larger (resident()).
+// networks 3 % slower, three quarters are no faster).  The grids are no larger than
+// what is resident from the start (resident()), so that no share waits for a
+// workgroup to end; only a caller's own zone plan can be (four zones, twice the
+// resident workgroups: 42.8 ms with shares and with the queue alone).
 // Measured: 50k cells of N = 15 2.46 -> 2.09 ms, 63k-cell evaluation 0.84 ->
 // 0.24 ms, speciation of 200k cells 2.40 -> 2.06 ms.
 void distribute(pfx_kernel_params &P, int G, int mode, int64_t waves) {
@@ -571,6 +573,13 @@ int zones_prepare(int32_t nzones, pfx_tables *const *tables, pfx_cells *cells, c
     b = (int)std::max<int64_t>(1, std::min<int64_t>(b, std::max<int64_t>(need, 1)));
     blocks[z] = b;
     total += b;
+  }
+  // the default split's rounding may not exceed the resident workgroups
+  while (!given && total > full) {
+    const int zmax = (int)(std::max_element(blocks, blocks + nzones) - blocks);
+    if (blocks[zmax] == 1) break;
+    blocks[zmax]--;
+    total--;
   }
   int acc = 0;
   for (int z = 0; z < nzones; z++) {
