@@ -171,6 +171,8 @@ __device__ __forceinline__ double gbcast(double v, int gbase) {
 // and BM enable 16-lane rows and 4-lane banks; the other lanes keep acc.  A
 // DPP source may not be read within two wait states of its write, which the
 // compiler cannot see inside the statement: every statement waits them itself.
+// Statements of four mark their accumulators as written early: an operand of
+// the same value may not share the register of one that is already changed.
 template <int J, int RM, int BM>
 __device__ __forceinline__ void fmac_bcast(double &acc, double src, double f) {
   asm("s_nop 1\n\t"
@@ -192,7 +194,7 @@ __device__ __forceinline__ void fmac_bcast_self(double f, double &a, double &b, 
       "v_fmac_f64_dpp %1, %1, %4 row_newbcast:%5 row_mask:%6 bank_mask:%7\n\t"
       "v_fmac_f64_dpp %2, %2, %4 row_newbcast:%5 row_mask:%6 bank_mask:%7\n\t"
       "v_fmac_f64_dpp %3, %3, %4 row_newbcast:%5 row_mask:%6 bank_mask:%7"
-      : "+v"(a), "+v"(b), "+v"(c), "+v"(d)
+      : "+&v"(a), "+&v"(b), "+&v"(c), "+&v"(d)
       : "v"(f), "n"(J), "n"(RM), "n"(BM));
 }
 template <int J, int RM, int BM>
@@ -203,7 +205,7 @@ __device__ __forceinline__ void fmac_bcast4(double f, double &a, double pa, doub
       "v_fmac_f64_dpp %1, %5, %8 row_newbcast:%9 row_mask:%10 bank_mask:%11\n\t"
       "v_fmac_f64_dpp %2, %6, %8 row_newbcast:%9 row_mask:%10 bank_mask:%11\n\t"
       "v_fmac_f64_dpp %3, %7, %8 row_newbcast:%9 row_mask:%10 bank_mask:%11"
-      : "+v"(a), "+v"(b), "+v"(c), "+v"(d)
+      : "+&v"(a), "+&v"(b), "+&v"(c), "+&v"(d)
       : "v"(pa), "v"(pb), "v"(pc), "v"(pd), "v"(f), "n"(J), "n"(RM), "n"(BM));
 }
 
