@@ -31,13 +31,17 @@ namespace {
 
 constexpr int BLOCK = 256;
 
-// Profiling build (this file compiled with -DPFX_SECTION_TIMERS):
+// Profiling build (this file in one piece, with -DPFX_SECTION_TIMERS:
+// pflotran_amd.build.build(out=..., defines=("PFX_SECTION_TIMERS",))):
 // shader-clock cycles per section of the Newton pass, summed per wavefront
 // and added into a device array when the wavefront exits; the product build
 // compiles every marker to nothing.  Sections: 0 refill/load, 1 activity,
 // 2 complexes, 3 totals and dT/dm, 4 ion exchange, 5 residual, minerals and
 // convergence, 6 constraint rows, 7 LU solve, 8 update and retire.
 #ifdef PFX_SECTION_TIMERS
+#ifdef PFX_REACT_PART
+#error "the section timers have one set of counters: compile this file in one piece"
+#endif
 __device__ unsigned long long g_section_cycles[16];
 #define PFX_PT(i)                                  \
   {                                                \
