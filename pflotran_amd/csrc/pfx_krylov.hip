@@ -501,6 +501,24 @@ struct mrhs_sc {
 
 __device__ __forceinline__ int mrhs_comps(int C) { return (BLOCK / C) * C; }
 
+// sh[0] + sh[C] + ... over `rows` rows, in order.  One load at a time waits out
+// the LDS latency for each: 12 us for the 256 rows of a single component, twice
+// per reduction; eight in flight 2 us (4200 rows, 1 component: a solve of 5
+// iterations 824 -> 333 us).
+__device__ __forceinline__ double mrhs_column(const double *sh, int rows, int C) {
+  double s = 0.0;
+  int k = 0;
+  for (; k + 8 <= rows; k += 8) {
+    double a[8];
+#pragma unroll
+    for (int j = 0; j < 8; j++) a[j] = sh[(k + j) * C];
+#pragma unroll
+    for (int j = 0; j < 8; j++) s += a[j];
+  }
+  for (; k < rows; k++) s += sh[k * C];
+  return s;
+}
+
 // per-component sums of NS values over this workgroup's threads: thread c < C
 // of the workgroup writes partial[(blockIdx.x * C + c) * NS + {0..NS-1}]
 template <int NS>
@@ -509,15 +527,11 @@ __device__ __forceinline__ void mrhs_block_sum(const double (&v)[NS], int C, dou
 #pragma unroll
   for (int q = 0; q < NS; q++) sh[q][threadIdx.x] = v[q];
   __syncthreads();
-  const int used = mrhs_comps(C);
   if ((int)threadIdx.x < C) {
 #pragma unroll
-    for (int q = 0; q < NS; q++) {
-      double s = 0.0;
-      for (int t = threadIdx.x; t < used; t += C) s += sh[q][t];
-      __hip_atomic_store(&partial[((int64_t)blockIdx.x * C + threadIdx.x) * NS + q], s, __ATOMIC_RELAXED,
-                         __HIP_MEMORY_SCOPE_AGENT);
-    }
+    for (int q = 0; q < NS; q++)
+      __hip_atomic_store(&partial[((int64_t)blockIdx.x * C + threadIdx.x) * NS + q],
+                         mrhs_column(sh[q] + threadIdx.x, BLOCK / C, C), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
 }
 
@@ -560,12 +574,10 @@ __device__ __forceinline__ void mrhs_sums(int nb, int C, const double *partial, 
 #pragma unroll
   for (int q = 0; q < NS; q++) sh[q][threadIdx.x] = v[q];
   __syncthreads();
+  // rows beyond the workgroups hold zeros
 #pragma unroll
-  for (int q = 0; q < NS; q++) {
-    out[q] = 0.0;
-    if ((int)threadIdx.x < C)
-      for (int t = threadIdx.x; t < used; t += C) out[q] += sh[q][t];
-  }
+  for (int q = 0; q < NS; q++)
+    out[q] = (int)threadIdx.x < C ? mrhs_column(sh[q] + threadIdx.x, step < nb ? step : nb, C) : 0.0;
 }
 
 __device__ __forceinline__ void mrhs_set_done(int C, const mrhs_sc *sc, int *done) {
