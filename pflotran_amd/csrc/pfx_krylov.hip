@@ -925,10 +925,12 @@ __global__ __launch_bounds__(BLOCK) void k_m_xr(const mrhs_args A) {
 // 2-3 us each whatever the size, five an iteration; here an iteration is two
 // products and four workgroup sums.  100 cells x 5 components, 12 enqueued
 // iterations: the captured operator-split step 227 -> 80 us.  Used up to
-// MRHS_SMALL rows, where one compute unit's share of the products still costs
-// less than the launches: 16x16x15 cells x 5 components 121 us a step, 16x16x17 by
-// launches 247.
-constexpr int MRHS_SMALL = 4096;
+// MRHS_SMALL rows and MRHS_SMALL_ENTRIES matrix entries, where one compute unit's
+// share of the products (each thread walks its rows' entries) still costs less
+// than the launches.  A solve of 3 to 6 iterations, 5 components, in one launch /
+// by launches: 4000 rows of 7 entries 147 / 284 us, of 13 309 / 315, 1000 of 27
+// 249 / 284; 2000 of 27 406 / 235, 1000 of 60 471 / 336, 4000 of 200 6590 / 711.
+constexpr int MRHS_SMALL = 4096, MRHS_SMALL_ENTRIES = 13 * MRHS_SMALL;
 
 template <int NS>
 __device__ __forceinline__ void wg_sum(double (&v)[NS], double (*sh)[16]) {
@@ -1459,7 +1461,7 @@ extern "C" int pfx_bsr_solve_multi(pfx_bsr *h, const double *values, const doubl
     hipLaunchKernelGGL(k_copy, dim3(grid_for((int64_t)nv)), dim3(BLOCK), 0, s, (int64_t)nv, B, own);
     A.b = own;
   }
-  if (n <= MRHS_SMALL) {
+  if (n <= MRHS_SMALL && h->nnzb <= MRHS_SMALL_ENTRIES) {
     const int T = n <= 256 ? 256 : 1024;
     const size_t lds = (size_t)n * sizeof(double);
     if (n <= 1024) hipLaunchKernelGGL(k_m_small<1>, dim3(C), dim3(T), lds, s, A);
