@@ -580,7 +580,8 @@ __global__ __launch_bounds__(256, 3) void k_surrogate_guess(const mlp_dev D, int
 // reach 64 KB of LDS.
 constexpr int CHAIN_WIDTH = 960;
 constexpr int CHAIN_ROWS = 16;
-constexpr int CHAIN_THREADS = 512;
+constexpr int CHAIN_THREADS = 512;  // inference: fewer for narrow networks (launch_chain)
+constexpr int CHAIN_RESIDENT = 256 * 4 * CHAIN_ROWS;
 
 struct mlp_chain {
   int nlayers, B, astr;  // astr: LDS row stride (BF16 elements)
@@ -602,13 +603,13 @@ __host__ __device__ inline int ld4(int n) { return (n + 3) & ~3; }
 // the next product's operand is padded with what epi writes there.
 // pre(n0) loads four values ahead of the product, epi(n0, acc, those) takes
 // rows n0..n0+3 of this lane's column (row lane % 16 of the batch tile).
-template <class PRE, class EPI>
+template <int THREADS, class PRE, class EPI>
 __device__ __forceinline__ void chain_product(const uint4 *__restrict__ W, int nrows, int kts,
                                               const unsigned short *in, int astr, PRE pre, EPI epi) {
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
   const int rt = (nrows + 15) / 16, ft = (nrows + 31) / 32 * 2;
   const unsigned short *ap = in + (lane & 15) * astr + 8 * (lane >> 4);
-  for (int nt = 2 * w; nt < ft; nt += 2 * (CHAIN_THREADS / 64)) {
+  for (int nt = 2 * w; nt < ft; nt += 2 * (THREADS / 64)) {
     const uint4 *p0 = W + (long)min(nt, rt - 1) * kts * 64 + lane;
     const uint4 *p1 = W + (long)min(nt + 1, rt - 1) * kts * 64 + lane;
     const int n0 = nt * 16 + 4 * (lane >> 4);
@@ -637,10 +638,10 @@ __device__ __forceinline__ void chain_product(const uint4 *__restrict__ W, int n
 
 // Forward pass of 16 rows; TRAIN: also the loss and dZ of every layer,
 // with the activations and gelu' kept for it and for the weight gradients.
-template <bool TRAIN>
-__global__ __launch_bounds__(CHAIN_THREADS) void k_chain(const mlp_chain D) {
+template <bool TRAIN, int THREADS>
+__global__ __launch_bounds__(THREADS) void k_chain(const mlp_chain D) {
   extern __shared__ __attribute__((aligned(16))) unsigned short chain_lds[];
-  __shared__ float lred[CHAIN_THREADS / 64];
+  __shared__ float lred[THREADS / 64];
   const int t = threadIdx.x, lane = t & 63;
   const int r0 = blockIdx.x * CHAIN_ROWS;
   const long row = r0 + (lane & 15);
@@ -649,7 +650,7 @@ __global__ __launch_bounds__(CHAIN_THREADS) void k_chain(const mlp_chain D) {
   unsigned short *in = chain_lds, *out = chain_lds + CHAIN_ROWS * astr;
   {
     const int K = D.dims[0], Kp = roundup(K, 32);
-    for (int i = t; i < CHAIN_ROWS * Kp; i += CHAIN_THREADS) {
+    for (int i = t; i < CHAIN_ROWS * Kp; i += THREADS) {
       const int r = i / Kp, k = i - r * Kp;
       in[r * astr + k] = f2bf((r0 + r < D.B && k < K) ? D.X[(long)(r0 + r) * K + k] : 0.0f);
     }
@@ -674,7 +675,7 @@ __global__ __launch_bounds__(CHAIN_THREADS) void k_chain(const mlp_chain D) {
     };
     if (!last) {
       float *Sl = D.S[l], *Al = D.A[l + 1];
-      chain_product(D.Wsw[l], N, roundup(K, 32) / 32, in, astr, bias, [&](int n0, f32x4 acc, f32x4 bv) {
+      chain_product<THREADS>(D.Wsw[l], N, roundup(K, 32) / 32, in, astr, bias, [&](int n0, f32x4 acc, f32x4 bv) {
         f32x4 s, a;
 #pragma unroll
         for (int q = 0; q < 4; q++) {
@@ -690,7 +691,7 @@ __global__ __launch_bounds__(CHAIN_THREADS) void k_chain(const mlp_chain D) {
         put(n0, a);
       });
     } else {
-      chain_product(D.Wsw[l], N, roundup(K, 32) / 32, in, astr, bias, [&](int n0, f32x4 acc, f32x4 bv) {
+      chain_product<THREADS>(D.Wsw[l], N, roundup(K, 32) / 32, in, astr, bias, [&](int n0, f32x4 acc, f32x4 bv) {
         f32x4 dz = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int q = 0; q < 4; q++)
@@ -721,7 +722,7 @@ __global__ __launch_bounds__(CHAIN_THREADS) void k_chain(const mlp_chain D) {
     const int K = D.dims[l], N = D.dims[l + 1], ld = ld4(K);
     const float *Sl = D.S[l - 1];
     float *dZl = D.dZ[l - 1];
-    chain_product(
+    chain_product<THREADS>(
         D.Wtsw[l], K, roundup(N, 32) / 32, in, astr,
         [&](int n0) {
           return live && n0 < ld ? *(const f32x4 *)&Sl[row * ld + n0] : (f32x4){0.f, 0.f, 0.f, 0.f};
@@ -743,7 +744,7 @@ __global__ __launch_bounds__(CHAIN_THREADS) void k_chain(const mlp_chain D) {
   __syncthreads();
   if (t == 0) {
     float l = 0.f;
-    for (int i = 0; i < CHAIN_THREADS / 64; i++) l += lred[i];
+    for (int i = 0; i < THREADS / 64; i++) l += lred[i];
     D.lpart[blockIdx.x] = l;
   }
 }
@@ -978,8 +979,19 @@ int launch_chain(pfx_mlp *m, const float *X, const float *T, float *Y, int B, hi
   D.inv = 1.0f / (float)((long)B * m->dims[m->nlayers]);
   const unsigned grid = (unsigned)((B + CHAIN_ROWS - 1) / CHAIN_ROWS);
   const size_t lds = (size_t)2 * CHAIN_ROWS * D.astr * sizeof(unsigned short);
-  if (T) hipLaunchKernelGGL(k_chain<true>, dim3(grid), dim3(CHAIN_THREADS), lds, s, D);
-  else hipLaunchKernelGGL(k_chain<false>, dim3(grid), dim3(CHAIN_THREADS), lds, s, D);
+  // A wavefront takes 32 columns of a layer.  A batch too large to be resident at
+  // once (CHAIN_RESIDENT rows, in workgroups of 8 wavefronts) gets no more
+  // wavefronts in inference than the widest layer keeps busy: idle ones hold places
+  // that other rows could have (262144 rows: 16-32-16 123 -> 52 us, 40-64-64-15 217
+  // -> 113, 40-128-128-15 250 -> 180).  Below, 8 read the rows sooner (4096 rows of
+  // 40-64-64-15 23.3 us, with two wavefronts 24.2).  Any split gives the same bits.
+  // Training stays at 8: its weight gradients hide the difference.
+  const int wide = T || B <= CHAIN_RESIDENT ? CHAIN_WIDTH : max_width(m);
+  if (T) hipLaunchKernelGGL((k_chain<true, CHAIN_THREADS>), dim3(grid), dim3(CHAIN_THREADS), lds, s, D);
+  else if (wide > 128) hipLaunchKernelGGL((k_chain<false, 512>), dim3(grid), dim3(512), lds, s, D);
+  else if (wide > 64) hipLaunchKernelGGL((k_chain<false, 256>), dim3(grid), dim3(256), lds, s, D);
+  else if (wide > 32) hipLaunchKernelGGL((k_chain<false, 128>), dim3(grid), dim3(128), lds, s, D);
+  else hipLaunchKernelGGL((k_chain<false, 64>), dim3(grid), dim3(64), lds, s, D);
   MCHK(hipGetLastError());
   return 0;
 }
@@ -1265,7 +1277,13 @@ extern "C" int pfx_mlp_forward(pfx_mlp *m, const float *X, int64_t B, float *Y, 
     const int nb = (int)((B - b0) < m->bmax ? (B - b0) : m->bmax);
     const float *x = X + b0 * m->dims[0];
     float *y = Y + b0 * m->dims[m->nlayers];
-    int rc = chain_ok(m) ? launch_chain(m, x, nullptr, y, nb, s) : forward(m, x, nb, y, false, s);
+    // One narrow layer over many rows is a plain product, whose tiles are 64 rows:
+    // 262144 rows of 4-1 26 us (by rows of 16 70), of 256-16 169 (228).  The line
+    // moves out with the inputs: 20000 rows of 16-16 20.6 us (22.2), of 256-16 37.6
+    // (28.5), 65536 of 256-16 57.7 (60.5).
+    const bool plain =
+        m->nlayers == 1 && m->dims[1] <= 32 && nb > (long)CHAIN_RESIDENT * std::max(1, m->dims[0] / 64);
+    int rc = chain_ok(m) && !plain ? launch_chain(m, x, nullptr, y, nb, s) : forward(m, x, nb, y, false, s);
     if (rc) return rc;
   }
   return 0;
