@@ -42,7 +42,7 @@ struct pfx_tables {
   pfx_kernel_params *d_zone_params = nullptr;
   uint64_t *d_finish = nullptr;
   int finish_cap = 0;
-  hipEvent_t ev0 = nullptr, ev1 = nullptr;
+  hipEvent_t ev0 = nullptr, ev1 = nullptr, ev2 = nullptr;
   // side stream of a zoned launch's pivoting follow-up for these tables'
   // zone (default priority), with its fork and join events
   hipStream_t side = nullptr;
@@ -688,7 +688,8 @@ int use_scratch(pfx_tables *t, pfx_kernel_params &P, int64_t n) {
 }  // namespace
 
 // one evaluation of every cell of a grid, straight into the block matrix;
-// *tot: the totals (the tables' scratch, grown on demand)
+// *tot: the totals (the tables' scratch, grown on demand).  Enqueued between ev0
+// and ev1: gi_finish waits for it and for the caller's launches behind it.
 int pfx_internal::gi_evaluate_cells(pfx_tables *t, pfx_cells *cells, const pfx_react_opts *o, int col_scale,
                                     const pfx_gi_faces &gi, double *residual, double **tot) {
   int rc = check_cells(t, cells, o);
@@ -710,20 +711,19 @@ int pfx_internal::gi_evaluate_cells(pfx_tables *t, pfx_cells *cells, const pfx_r
   P.tot_eval_out = *tot;
   P.col_scale = col_scale ? 1 : 0;
   double ms = 0.0;
-  return launch(t, P, PFX_MODE_GI, (hipStream_t)o->stream, o->stream_ordered ? nullptr : &ms);
+  return launch(t, P, PFX_MODE_GI, (hipStream_t)o->stream, &ms, nullptr, nullptr, false);
 }
 
-int pfx_internal::timed_launch_begin(pfx_tables *t, hipStream_t s) {
-  HIPCHK(hipEventRecord(t->ev0, s));
-  return 0;
-}
-
-int pfx_internal::timed_launch_end(pfx_tables *t, hipStream_t s, int slot) {
-  HIPCHK(hipEventRecord(t->ev1, s));
-  HIPCHK(hipEventSynchronize(t->ev1));
-  float f = 0.f;
-  HIPCHK(hipEventElapsedTime(&f, t->ev0, t->ev1));
-  t->last_ms[slot] = f;
+// the end of a grid evaluation: one wait for its launches (a wait between them
+// cost more than the work on grids of up to some hundred cells), their times read
+int pfx_internal::gi_finish(pfx_tables *t, hipStream_t s) {
+  HIPCHK(hipEventRecord(t->ev2, s));
+  HIPCHK(hipEventSynchronize(t->ev2));
+  float cell = 0.f, flux = 0.f;
+  HIPCHK(hipEventElapsedTime(&cell, t->ev0, t->ev1));
+  HIPCHK(hipEventElapsedTime(&flux, t->ev1, t->ev2));
+  t->last_ms[0] = cell;
+  t->last_ms[1] = flux;
   return 0;
 }
 
@@ -1055,6 +1055,7 @@ extern "C" int pfx_tables_create(const pfx_reaction_desc *d, pfx_tables **out) {
   HIPCHK(hipHostMalloc(&t->h_stats, kStatsWords * sizeof(unsigned long long)));
   HIPCHK(hipEventCreate(&t->ev0));
   HIPCHK(hipEventCreate(&t->ev1));
+  HIPCHK(hipEventCreate(&t->ev2));
   {
     // the device address of this GPU's fixed scratch array, once per device
     // (the array's name is a host stand-in, not a device address)
@@ -1084,6 +1085,7 @@ extern "C" int pfx_tables_destroy(pfx_tables *t) {
   if (t->d_defer) (void)hipFree(t->d_defer);
   if (t->ev0) (void)hipEventDestroy(t->ev0);
   if (t->ev1) (void)hipEventDestroy(t->ev1);
+  if (t->ev2) (void)hipEventDestroy(t->ev2);
   if (t->fork_ev) (void)hipEventDestroy(t->fork_ev);
   if (t->join_ev) (void)hipEventDestroy(t->join_ev);
   if (t->side) (void)hipStreamDestroy(t->side);

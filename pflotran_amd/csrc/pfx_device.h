@@ -193,7 +193,6 @@ int bsr_multi_rhs(::pfx_bsr *h, int C, double **B);
 int tables_reserve(pfx_tables *t, const pfx_cells *cells);
 // arm pfx_tables_stats for a replayed stream-ordered reaction step of n cells
 void tables_rearm_stats(pfx_tables *t, int64_t n, hipStream_t stream, bool fallback);
-// event-timed launch bracket; the time goes to the tables' last_ms[slot]
-int timed_launch_begin(pfx_tables *t, hipStream_t s);
-int timed_launch_end(pfx_tables *t, hipStream_t s, int slot);
+// wait for a grid evaluation and what was enqueued behind it, and read their times
+int gi_finish(pfx_tables *t, hipStream_t s);
 }

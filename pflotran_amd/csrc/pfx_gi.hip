@@ -310,10 +310,9 @@ extern "C" int pfx_gi_residual_jacobian(pfx_tables *t, pfx_cells *cells, const p
   int rc = pfx_internal::gi_evaluate_cells(t, cells, o, g->log_formulation, P, residual, &tot);
   if (rc) return rc;
   hipStream_t s = (hipStream_t)o->stream;
-  if ((rc = pfx_internal::timed_launch_begin(t, s))) return rc;
   hipLaunchKernelGGL(k_gi_flux_residual, dim3((unsigned)((n * N + 255) / 256)), dim3(256), 0, s, P, N, tot, residual);
   GCHK(hipGetLastError());
-  return pfx_internal::timed_launch_end(t, s, 1);
+  return pfx_internal::gi_finish(t, s);
 }
 
 extern "C" int pfx_gi_dispersion(const pfx_grid *g, const double *porosity, const double *saturation,
