@@ -56,7 +56,9 @@ int pfx_mlp_destroy(pfx_mlp *mlp);
 /* HOST <-> device copy of one parameter array: which = 0 weights of
    `layer`, 1 biases, 2 weight gradients, 3 bias gradients, 4 normalisation
    (in_shift[dims0], in_scale[dims0], out_shift[out], out_scale[out]
-   concatenated, layer ignored).  to_device != 0 uploads. */
+   concatenated, layer ignored).  to_device != 0 uploads; the array is in
+   place when the call returns, for passes on any stream and for captured
+   passes replayed later. */
 int pfx_mlp_params(pfx_mlp *mlp, int32_t which, int32_t layer, float *host, int32_t to_device);
 
 /* Inference Y[B][out] = f(X[B][dims0]) with the BF16 product kernels. */

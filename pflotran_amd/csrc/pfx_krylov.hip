@@ -480,8 +480,9 @@ __global__ __launch_bounds__(BLOCK) void k_newton_update(int64_t n, double *__re
 // component and the per-component partial sums of a workgroup are fixed-order
 // sums.  The last workgroup of a reducing launch turns the partial sums into
 // each component's scalars and convergence status; the element kernels skip
-// components whose status is set.  No value goes to the host between
-// iterations: a solve is stream-ordered and can be captured in a graph.
+// components whose status is set.  No iteration needs a value on the host: an
+// enqueued solve can be captured in a graph (one that the caller waits for reads
+// a flag every four iterations, to stop).
 //
 // HBM-bound: 19 passes over an [n][C] vector per iteration (4 p, 3 v, 3 s, 2 t,
 // 7 xr).  The preconditioned vectors are not stored (1/diagonal times p or s

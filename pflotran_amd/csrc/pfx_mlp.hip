@@ -94,7 +94,9 @@ __device__ __forceinline__ float gelu_grad(float z) {
 // least squares (3e-9 in Phi).  Against 64 bits over normal and uniform z in
 // [-6, 6] the result is off by 3.8e-7 at most and 5.3e-8 rms, the form with erff by
 // 4.5e-7 and 5.8e-8; about 25 issue slots where erff's two ranges took 80, which
-// bounded the kernel (its 768 values a cell).
+// bounded the kernel (its 768 values a cell).  Training, and plain inference with
+// its kernel, keep erff: the slope from the shared exponential would be off by
+// 2.1e-7 (now 1.4e-7), and the GELUs are 2 of that kernel's 27 us.
 __device__ __forceinline__ float gelu_tail(float z) {
   const float t = fabsf(z);
   const float s = __builtin_amdgcn_rcpf(fmaf(0.32f, t, 1.0f));

@@ -1692,10 +1692,11 @@ __device__ __forceinline__ void react_body(uint64_t praw) {
       // exchange and mineral terms (nu^T diag(C) nu, diag(X) - X X^T,
       // nu nu^T dI/dlnQ) with rows scaled by positive factors, so it needs
       // no row exchanges, and the reaction kernels factor without a pivot
-      // search.  A zero pivot or a non-finite multiplier (far from the
-      // solution, or where a rate-law option makes a mineral term
-      // indefinite) breaks the unpivoted factorisation down: under
-      // PFX_LU_DEFER the cell is listed and left untouched for the pivoting
+      // search.  It breaks down far from the solution, or where a rate-law
+      // option makes a mineral term indefinite: a zero pivot or an overflow
+      // leaves an unknown that is not finite (lu_solve), and one beyond 1e300
+      // counts as such, the only test there is.  Then, under
+      // PFX_LU_DEFER, the cell is listed and left untouched for the pivoting
       // launch, which redoes its step from the start; under
       // PFX_LU_ONDEMAND its wave pivots from the cell's next pass on, at
       // the same iterate.  Pivoting (the constraint solve always, and
